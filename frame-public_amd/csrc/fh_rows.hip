@@ -1,8 +1,9 @@
 // Row reductions over the last axis of [rows, cols]: softmax and LayerNorm.
 //
-// One wavefront (64 lanes) owns a row when the row fits in registers (cols <= 64 * 32): the row is read
-// once, reduced with cross-lane shuffles, and written once. Longer rows fall back to one workgroup per row
-// that streams the row through global memory in three passes.
+// A row is owned by 8, 16, 32, 64 or 256 lanes, whichever hold it as at most four (fp32 up to eight) 16-byte vectors
+// each: it is read once, reduced with cross-lane shuffles (and LDS across four waves), and written once. Rows shorter
+// than one vector take one element per lane; rows too long for registers fall back to one workgroup per row that
+// streams the row through global memory in three passes.
 //
 // softmax (reference: src/backends/cpu/kernels/sequence.cpp:114-174): m = max, e = exp(x - m), s = sum(e),
 // y = round(e / s). LayerNorm (reference: src/backends/cpu/kernels/sequence.cpp:182-279): two-pass mean and
@@ -59,92 +60,147 @@ __device__ __forceinline__ float softmax_div(float e, float s, float r) {
   }
 }
 
-typedef unsigned int u4_t __attribute__((ext_vector_type(4)));
+// A row's 16-byte vectors over its L lanes (256 / L rows per workgroup): lane l holds the elements
+// [V * (l + L * t), + V) for t < NV. Rows start wherever row * cols puts them, so the accesses are 16 bytes at element
+// alignment (global memory takes them at any alignment). kRowFull: the row is exactly V * NV * L elements, no lane is
+// idle. kRowVectors: whole vectors, the last lanes idle. kRowRagged: cols is no multiple of V, and the row's last vector
+// is moved back to end at the row's end; the elements it then shares with the vector before it ("dup" of them) are
+// left out of the sums, and both lanes store them with the same value.
+// What bounds these kernels is HBM once the accesses are vectors (softmax bf16, us, one element per lane and access
+// before): [32768, 1000] 52.7 -> 25.5 (5.1 TB/s), [32768, 1001] 53.5 -> 26.5, [65536, 47] f32 12.7 -> 6.9; rows of
+// more than 2,048 elements, in three passes over memory before: [4096, 8192] f16 98 -> 30.
+enum RowMode { kRowFull, kRowVectors, kRowRagged };
 
-template <typename T, int PER>
-__global__ __launch_bounds__(256) void softmax_wave_kernel(const typename Io<T>::storage* __restrict__ x,
-                                                           typename Io<T>::storage* __restrict__ y, int64_t rows,
-                                                           int64_t cols) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * kRowsPerBlock + (threadIdx.x >> 6);
-  if (row >= rows) return;
+template <int V, int NV, int L, int MODE>
+struct RowVectors {
+  int64_t at[NV];  // first element of each vector; -1 where the row has none
+  int dup[NV];     // elements at its start that the vector before it holds as well
+  __device__ RowVectors(int l, int64_t cols) {
+#pragma unroll
+    for (int t = 0; t < NV; ++t) {
+      const int64_t j = static_cast<int64_t>(V) * (l + L * t);
+      at[t] = j;
+      dup[t] = 0;
+      if constexpr (MODE != kRowFull) at[t] = j >= cols ? -1 : at[t];
+      if constexpr (MODE == kRowRagged) {
+        if (j < cols && j + V > cols) at[t] = cols - V, dup[t] = static_cast<int>(j - at[t]);
+      }
+    }
+  }
+  __device__ bool has(int t) const { return MODE == kRowFull || at[t] >= 0; }
+  // whether element i of vector t is this lane's own
+  __device__ bool own(int t, int i) const { return has(t) && (MODE != kRowRagged || i >= dup[t]); }
+};
+
+// One 16-byte vector at element alignment. Each row is read and written once, so whole rows go past the caches
+// (non-temporal); a ragged row shares its first and last cache lines with its neighbours and does not.
+typedef unsigned int u4_t __attribute__((ext_vector_type(4)));
+typedef u4_t u4_any __attribute__((aligned(2)));
+template <typename T, int MODE, int V>
+__device__ __forceinline__ void row_load(const typename Io<T>::storage* p, float (&v)[V]) {
+  const u4_any* q = reinterpret_cast<const u4_any*>(p);
+  u4_t w;
+  if constexpr (MODE == kRowRagged) w = *q;
+  else w = __builtin_nontemporal_load(q);
+  unpack_vec<T>(make_uint4(w.x, w.y, w.z, w.w), v);
+}
+template <typename T, int MODE, int V>
+__device__ __forceinline__ void row_store(typename Io<T>::storage* p, const float (&v)[V]) {
+  const uint4 w = pack_vec<T>(v);
+  u4_any* q = reinterpret_cast<u4_any*>(p);
+  if constexpr (MODE == kRowRagged) *q = u4_t{w.x, w.y, w.z, w.w};
+  else __builtin_nontemporal_store(u4_t{w.x, w.y, w.z, w.w}, q);
+}
+
+// Reductions over the L lanes of a row (L = 256: all four waves of the workgroup, through `scratch`).
+template <int L>
+__device__ __forceinline__ float row_max(float v, float* scratch) {
+#pragma unroll
+  for (int o = (L < 64 ? L : 64) / 2; o > 0; o >>= 1) {
+    const float other = __shfl_xor(v, o, 64);
+    v = (other > v) ? other : v;
+  }
+  if constexpr (L == 256) {
+    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = scratch[0];
+#pragma unroll
+    for (int k = 1; k < 4; ++k) v = (scratch[k] > v) ? scratch[k] : v;
+  }
+  return v;
+}
+template <int L>
+__device__ __forceinline__ float row_sum(float v, float* scratch) {
+#pragma unroll
+  for (int o = (L < 64 ? L : 64) / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  if constexpr (L == 256) {
+    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = ((scratch[0] + scratch[1]) + scratch[2]) + scratch[3];
+  }
+  return v;
+}
+
+template <typename T, int NV, int L, int MODE>
+__global__ __launch_bounds__(256) void softmax_row_kernel(const typename Io<T>::storage* __restrict__ x,
+                                                          typename Io<T>::storage* __restrict__ y, int64_t rows,
+                                                          int64_t cols) {
+  constexpr int V = 16 / static_cast<int>(sizeof(typename Io<T>::storage));
+  __shared__ float scratch[2][4];
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * (256 / L) + threadIdx.x / L;
+  if (row >= rows) return;  // (whole row groups leave; with L = 256 every workgroup has its row)
+  const RowVectors<V, NV, L, MODE> rv(threadIdx.x % L, cols);
   const auto* xr = x + row * cols;
   auto* yr = y + row * cols;
-  float v[PER];
+  float v[NV][V];
+#pragma unroll
+  for (int t = 0; t < NV; ++t) {
+    if (rv.has(t)) {
+      row_load<T, MODE>(xr + rv.at[t], v[t]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < V; ++i) v[t][i] = -__builtin_inff();
+    }
+  }
   float m = -__builtin_inff();
 #pragma unroll
-  for (int t = 0; t < PER; ++t) {
-    const int64_t j = lane + 64 * t;
-    v[t] = (j < cols) ? Io<T>::load(xr[j]) : -__builtin_inff();
-    m = (v[t] > m) ? v[t] : m;
-  }
-  m = wave_max(m);
+  for (int t = 0; t < NV; ++t)
+#pragma unroll
+    for (int i = 0; i < V; ++i) m = (v[t][i] > m) ? v[t][i] : m;
+  m = row_max<L>(m, scratch[0]);
   float s = 0.0f;
 #pragma unroll
-  for (int t = 0; t < PER; ++t) {
-    const int64_t j = lane + 64 * t;
-    v[t] = (j < cols) ? softmax_exp<T>(v[t] - m) : 0.0f;
-    s += v[t];
-  }
-  s = wave_sum(s);
+  for (int t = 0; t < NV; ++t)
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      v[t][i] = softmax_exp<T>(v[t][i] - m);
+      s += rv.own(t, i) ? v[t][i] : 0.0f;
+    }
+  s = row_sum<L>(s, scratch[1]);
   const float r = 1.0f / s;
 #pragma unroll
-  for (int t = 0; t < PER; ++t) {
-    const int64_t j = lane + 64 * t;
-    if (j < cols) yr[j] = Io<T>::store(softmax_div<T>(v[t], s, r));
+  for (int t = 0; t < NV; ++t) {
+    if (!rv.has(t)) continue;
+    float o[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) o[i] = softmax_div<T>(v[t][i], s, r);
+    row_store<T, MODE>(yr + rv.at[t], o);
   }
 }
 
-// Rows of 64 * PER elements with 16-byte aligned rows, one wave per row: lane l owns the contiguous elements
-// [V*l + 64*V*t, +V) for t < PER / V, all loaded (16-byte accesses) before the max reduction. The arithmetic is
-// softmax_wave_kernel's (m = max, e = exp(x - m), s = sum e, y = round(e / s)); only the order of the terms of
-// the lane's partial sum differs.
-template <typename T, int PER>
-__global__ __launch_bounds__(256) void softmax_vec_kernel(const typename Io<T>::storage* __restrict__ x,
-                                                         typename Io<T>::storage* __restrict__ y, int64_t rows) {
-  using S = typename Io<T>::storage;
-  constexpr int V = 16 / static_cast<int>(sizeof(S));
-  constexpr int NV = PER / V;
-  constexpr int64_t COLS = 64 * PER;
-  static_assert(PER % V == 0, "whole vectors per lane");
+// Rows shorter than one vector: one element per lane, one wave per row.
+template <typename T>
+__global__ __launch_bounds__(256) void softmax_short_kernel(const typename Io<T>::storage* __restrict__ x,
+                                                            typename Io<T>::storage* __restrict__ y, int64_t rows,
+                                                            int64_t cols) {
   const int lane = threadIdx.x & 63;
   const int64_t row = static_cast<int64_t>(blockIdx.x) * kRowsPerBlock + (threadIdx.x >> 6);
   if (row >= rows) return;
-  const u4_t* xr = reinterpret_cast<const u4_t*>(x + row * COLS);
-  u4_t* yr = reinterpret_cast<u4_t*>(y + row * COLS);
-  u4_t xv[NV];
-#pragma unroll
-  for (int t = 0; t < NV; ++t) xv[t] = __builtin_nontemporal_load(xr + lane + 64 * t);
-  float v[PER];
-  float m = -__builtin_inff();
-#pragma unroll
-  for (int t = 0; t < NV; ++t) {
-    S e[V];
-    __builtin_memcpy(e, &xv[t], 16);
-#pragma unroll
-    for (int i = 0; i < V; ++i) {
-      v[t * V + i] = Io<T>::load(e[i]);
-      m = (v[t * V + i] > m) ? v[t * V + i] : m;
-    }
-  }
-  m = wave_max(m);
-  float s = 0.0f;
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    v[i] = softmax_exp<T>(v[i] - m);
-    s += v[i];
-  }
-  s = wave_sum(s);
-  const float r = 1.0f / s;
-#pragma unroll
-  for (int t = 0; t < NV; ++t) {
-    S o[V];
-#pragma unroll
-    for (int i = 0; i < V; ++i) o[i] = Io<T>::store(softmax_div<T>(v[t * V + i], s, r));
-    u4_t w;
-    __builtin_memcpy(&w, o, 16);
-    __builtin_nontemporal_store(w, yr + lane + 64 * t);
-  }
+  const float v = (lane < cols) ? Io<T>::load(x[row * cols + lane]) : -__builtin_inff();
+  const float m = wave_max((v > -__builtin_inff()) ? v : -__builtin_inff());
+  const float e = (lane < cols) ? softmax_exp<T>(v - m) : 0.0f;
+  const float s = wave_sum(e);
+  if (lane < cols) y[row * cols + lane] = Io<T>::store(softmax_div<T>(e, s, 1.0f / s));
 }
 
 __device__ float block_reduce(float v, bool is_max, float* scratch) {
@@ -177,108 +233,76 @@ __global__ __launch_bounds__(256) void softmax_block_kernel(const typename Io<T>
   for (int64_t j = threadIdx.x; j < cols; j += blockDim.x) yr[j] = Io<T>::store(expf(Io<T>::load(xr[j]) - m) / s);
 }
 
-template <typename T, int PER>
-__global__ __launch_bounds__(256) void layer_norm_wave_kernel(const typename Io<T>::storage* __restrict__ x,
-                                                              const typename Io<T>::storage* __restrict__ gamma,
-                                                              const typename Io<T>::storage* __restrict__ beta,
-                                                              typename Io<T>::storage* __restrict__ y,
-                                                              int64_t rows, int64_t cols, float eps) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * kRowsPerBlock + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const auto* xr = x + row * cols;
-  auto* yr = y + row * cols;
-  float v[PER];
-  float sum = 0.0f;
-#pragma unroll
-  for (int t = 0; t < PER; ++t) {
-    const int64_t j = lane + 64 * t;
-    v[t] = (j < cols) ? Io<T>::load(xr[j]) : 0.0f;
-    sum += v[t];
-  }
-  const float mean = wave_sum(sum) / static_cast<float>(cols);
-  float var_sum = 0.0f;
-#pragma unroll
-  for (int t = 0; t < PER; ++t) {
-    const int64_t j = lane + 64 * t;
-    const float c = v[t] - mean;
-    var_sum += (j < cols) ? c * c : 0.0f;
-  }
-  const float variance = wave_sum(var_sum) / static_cast<float>(cols);
-  const float r = 1.0f / sqrtf(variance + eps);
-#pragma unroll
-  for (int t = 0; t < PER; ++t) {
-    const int64_t j = lane + 64 * t;
-    if (j < cols) {
-      const float xhat = (v[t] - mean) * r;
-      const float g = Io<T>::load(gamma[j]);
-      const float b = Io<T>::load(beta[j]);
-      yr[j] = Io<T>::store(g * xhat + b);
-    }
-  }
-}
-
-// Same arithmetic with 16-byte accesses, for rows of exactly 64 * PER elements (PER a multiple of the vector
-// width): lane l owns the contiguous elements [V*l + 64*V*t, +V) for t < PER / V. Every load (x, gamma, beta)
-// is issued before the first reduction, so one memory latency covers the row.
-template <typename T, int PER>
-__global__ __launch_bounds__(256) void layer_norm_vec_kernel(const typename Io<T>::storage* __restrict__ x,
+template <typename T, int NV, int L, int MODE>
+__global__ __launch_bounds__(256) void layer_norm_row_kernel(const typename Io<T>::storage* __restrict__ x,
                                                              const typename Io<T>::storage* __restrict__ gamma,
                                                              const typename Io<T>::storage* __restrict__ beta,
                                                              typename Io<T>::storage* __restrict__ y, int64_t rows,
-                                                             float eps) {
-  using S = typename Io<T>::storage;
-  constexpr int V = 16 / static_cast<int>(sizeof(S));
-  constexpr int NV = PER / V;
-  constexpr int64_t COLS = 64 * PER;
-  static_assert(PER % V == 0, "whole vectors per lane");
-  const int lane = threadIdx.x & 63;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * kRowsPerBlock + (threadIdx.x >> 6);
+                                                             int64_t cols, float eps) {
+  constexpr int V = 16 / static_cast<int>(sizeof(typename Io<T>::storage));
+  __shared__ float scratch[2][4];
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * (256 / L) + threadIdx.x / L;
   if (row >= rows) return;
-  const u4_t* xr = reinterpret_cast<const u4_t*>(x + row * COLS);
-  const u4_t* gr = reinterpret_cast<const u4_t*>(gamma);
-  const u4_t* br = reinterpret_cast<const u4_t*>(beta);
-  u4_t* yr = reinterpret_cast<u4_t*>(y + row * COLS);
-  u4_t xv[NV], gv[NV], bv[NV];
-#pragma unroll
-  for (int t = 0; t < NV; ++t) xv[t] = __builtin_nontemporal_load(xr + lane + 64 * t);
-#pragma unroll
-  for (int t = 0; t < NV; ++t) {
-    gv[t] = gr[lane + 64 * t];
-    bv[t] = br[lane + 64 * t];
-  }
-  float v[PER];
-  float sum = 0.0f;
+  const RowVectors<V, NV, L, MODE> rv(threadIdx.x % L, cols);
+  const auto* xr = x + row * cols;
+  auto* yr = y + row * cols;
+  // every load (x, gamma, beta) is issued before the first reduction, so one memory latency covers the row
+  float v[NV][V];
+  uint4 gv[NV], bv[NV];
 #pragma unroll
   for (int t = 0; t < NV; ++t) {
-    S e[V];
-    __builtin_memcpy(e, &xv[t], 16);
+    if (rv.has(t)) {
+      row_load<T, MODE>(xr + rv.at[t], v[t]);
+      __builtin_memcpy(&gv[t], gamma + rv.at[t], 16);
+      __builtin_memcpy(&bv[t], beta + rv.at[t], 16);
+    } else {
 #pragma unroll
-    for (int i = 0; i < V; ++i) {
-      v[t * V + i] = Io<T>::load(e[i]);
-      sum += v[t * V + i];
+      for (int i = 0; i < V; ++i) v[t][i] = 0.0f;
+      gv[t] = bv[t] = make_uint4(0, 0, 0, 0);
     }
   }
-  const float mean = wave_sum(sum) / static_cast<float>(COLS);
+  float sum = 0.0f;
+#pragma unroll
+  for (int t = 0; t < NV; ++t)
+#pragma unroll
+    for (int i = 0; i < V; ++i) sum += rv.own(t, i) ? v[t][i] : 0.0f;
+  const float mean = row_sum<L>(sum, scratch[0]) / static_cast<float>(cols);
   float var_sum = 0.0f;
 #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    v[i] -= mean;  // x - mean, kept for the normalisation (the same fp32 value the reference computes twice)
-    var_sum += v[i] * v[i];
-  }
-  const float variance = wave_sum(var_sum) / static_cast<float>(COLS);
+  for (int t = 0; t < NV; ++t)
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      v[t][i] -= mean;  // kept for the normalisation (the same fp32 value the reference computes twice)
+      var_sum += rv.own(t, i) ? v[t][i] * v[t][i] : 0.0f;
+    }
+  const float variance = row_sum<L>(var_sum, scratch[1]) / static_cast<float>(cols);
   const float r = 1.0f / sqrtf(variance + eps);
 #pragma unroll
   for (int t = 0; t < NV; ++t) {
-    S g[V], b[V];
-    __builtin_memcpy(g, &gv[t], 16);
-    __builtin_memcpy(b, &bv[t], 16);
-    float o[V];
+    if (!rv.has(t)) continue;
+    float g[V], b[V], o[V];
+    unpack_vec<T>(gv[t], g);
+    unpack_vec<T>(bv[t], b);
 #pragma unroll
-    for (int i = 0; i < V; ++i) o[i] = Io<T>::load(g[i]) * (v[t * V + i] * r) + Io<T>::load(b[i]);
-    const uint4 pw = pack_vec<T>(o);
-    __builtin_nontemporal_store(u4_t{pw.x, pw.y, pw.z, pw.w}, yr + lane + 64 * t);
+    for (int i = 0; i < V; ++i) o[i] = g[i] * (v[t][i] * r) + b[i];
+    row_store<T, MODE>(yr + rv.at[t], o);
   }
+}
+
+// Rows shorter than one vector: one element per lane, one wave per row.
+template <typename T>
+__global__ __launch_bounds__(256) void layer_norm_short_kernel(const typename Io<T>::storage* __restrict__ x,
+                                                               const typename Io<T>::storage* __restrict__ gamma,
+                                                               const typename Io<T>::storage* __restrict__ beta,
+                                                               typename Io<T>::storage* __restrict__ y, int64_t rows,
+                                                               int64_t cols, float eps) {
+  const int lane = threadIdx.x & 63;
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * kRowsPerBlock + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const float v = (lane < cols) ? Io<T>::load(x[row * cols + lane]) : 0.0f;
+  const float c = v - wave_sum(v) / static_cast<float>(cols);
+  const float r = 1.0f / sqrtf(wave_sum((lane < cols) ? c * c : 0.0f) / static_cast<float>(cols) + eps);
+  if (lane < cols) y[row * cols + lane] = Io<T>::store(Io<T>::load(gamma[lane]) * (c * r) + Io<T>::load(beta[lane]));
 }
 
 template <typename T>
@@ -306,89 +330,72 @@ __global__ __launch_bounds__(256) void layer_norm_block_kernel(const typename Io
   }
 }
 
-template <typename T, template <typename, int> class Launcher, typename... Args>
-fh_status by_width(int64_t cols, Args... args) {
-  if (cols <= 64) return Launcher<T, 1>::go(args...);
-  if (cols <= 128) return Launcher<T, 2>::go(args...);
-  if (cols <= 256) return Launcher<T, 4>::go(args...);
-  if (cols <= 512) return Launcher<T, 8>::go(args...);
-  if (cols <= 1024) return Launcher<T, 16>::go(args...);
-  return Launcher<T, 32>::go(args...);
+// Lanes and vectors per row, for rows of at least one vector. The fewest of 8, 16, 32 or 64 lanes that hold the row as
+// one vector each, so that short rows share a wave; then 64 lanes of up to four vectors, then the whole workgroup of
+// 256, up to 64 values in a lane's registers. go<NV, L, MODE>() launches; false when the row does not fit.
+template <int V, typename Go>
+bool by_row_width(int64_t cols, Go&& go) {
+  const int64_t vecs = (cols + V - 1) / V;
+  const auto pick = [&]<int NV, int L>() {
+    if (cols == int64_t{V} * NV * L) go.template operator()<NV, L, kRowFull>();
+    else if (cols % V == 0) go.template operator()<NV, L, kRowVectors>();
+    else go.template operator()<NV, L, kRowRagged>();
+    return true;
+  };
+  if (cols < V) return false;
+  if (vecs <= 8) return pick.template operator()<1, 8>();
+  if (vecs <= 16) return pick.template operator()<1, 16>();
+  if (vecs <= 32) return pick.template operator()<1, 32>();
+  if (vecs <= 64) return pick.template operator()<1, 64>();
+  if (vecs <= 128) return pick.template operator()<2, 64>();
+  if (vecs <= 256) return pick.template operator()<4, 64>();
+  if (vecs <= 512) return pick.template operator()<2, 256>();
+  if (vecs <= 1024) return pick.template operator()<4, 256>();
+  if (vecs <= 2048) return pick.template operator()<8, 256>();
+  return false;
 }
-
-template <typename T, int PER>
-struct SoftmaxLaunch {
-  using S = typename Io<T>::storage;
-  static fh_status go(const void* x, void* y, int64_t rows, int64_t cols, hipStream_t s) {
-    const dim3 grid(static_cast<uint32_t>((rows + kRowsPerBlock - 1) / kRowsPerBlock));
-    hipLaunchKernelGGL((softmax_wave_kernel<T, PER>), grid, dim3(256), 0, s, static_cast<const S*>(x),
-                       static_cast<S*>(y), rows, cols);
-    return launch_status("softmax_wave_kernel launch");
-  }
-};
-
-template <typename T, int PER>
-struct LayerNormLaunch {
-  using S = typename Io<T>::storage;
-  static fh_status go(const void* x, const void* g, const void* b, void* y, int64_t rows, int64_t cols, float eps,
-                      hipStream_t s) {
-    const dim3 grid(static_cast<uint32_t>((rows + kRowsPerBlock - 1) / kRowsPerBlock));
-    hipLaunchKernelGGL((layer_norm_wave_kernel<T, PER>), grid, dim3(256), 0, s, static_cast<const S*>(x),
-                       static_cast<const S*>(g), static_cast<const S*>(b), static_cast<S*>(y), rows, cols, eps);
-    return launch_status("layer_norm_wave_kernel launch");
-  }
-};
-
-template <typename T, int PER>
-fh_status launch_softmax_vec(const void* x, void* y, int64_t rows, hipStream_t s) {
-  using S = typename Io<T>::storage;
-  const dim3 grid(static_cast<uint32_t>((rows + kRowsPerBlock - 1) / kRowsPerBlock));
-  hipLaunchKernelGGL((softmax_vec_kernel<T, PER>), grid, dim3(256), 0, s, static_cast<const S*>(x),
-                     static_cast<S*>(y), rows);
-  return launch_status("softmax_vec_kernel launch");
+uint32_t row_blocks(int64_t rows, int lanes) {
+  const int64_t per = 256 / lanes;
+  return static_cast<uint32_t>((rows + per - 1) / per);
 }
-
-bool aligned16(const void* p);
 
 template <typename T>
 fh_status softmax_typed(const void* x, void* y, int64_t rows, int64_t cols, hipStream_t s) {
   using S = typename Io<T>::storage;
   constexpr int V = 16 / static_cast<int>(sizeof(S));
-  if (aligned16(x) && aligned16(y)) {
-    if (cols == 64 * V) return launch_softmax_vec<T, V>(x, y, rows, s);
-    if (cols == 64 * 2 * V) return launch_softmax_vec<T, 2 * V>(x, y, rows, s);
-    if (cols == 64 * 4 * V) return launch_softmax_vec<T, 4 * V>(x, y, rows, s);
+  const S* xs = static_cast<const S*>(x);
+  S* ys = static_cast<S*>(y);
+  const auto row_kernel = [&]<int NV, int L, int MODE>() {
+    hipLaunchKernelGGL((softmax_row_kernel<T, NV, L, MODE>), dim3(row_blocks(rows, L)), dim3(256), 0, s, xs, ys, rows,
+                       cols);
+  };
+  if (by_row_width<V>(cols, row_kernel)) return launch_status("softmax_row_kernel launch");
+  if (cols < V) {
+    hipLaunchKernelGGL(softmax_short_kernel<T>, dim3(row_blocks(rows, 64)), dim3(256), 0, s, xs, ys, rows, cols);
+    return launch_status("softmax_short_kernel launch");
   }
-  if (cols <= 64 * 32) return by_width<T, SoftmaxLaunch>(cols, x, y, rows, cols, s);
   hipLaunchKernelGGL(softmax_block_kernel<T>, dim3(static_cast<uint32_t>(rows)), dim3(256), 0, s,
                      static_cast<const S*>(x), static_cast<S*>(y), cols);
   return launch_status("softmax_block_kernel launch");
 }
 
-template <typename T, int PER>
-fh_status launch_layer_norm_vec(const void* x, const void* g, const void* b, void* y, int64_t rows, float eps,
-                                hipStream_t s) {
-  using S = typename Io<T>::storage;
-  const dim3 grid(static_cast<uint32_t>((rows + kRowsPerBlock - 1) / kRowsPerBlock));
-  hipLaunchKernelGGL((layer_norm_vec_kernel<T, PER>), grid, dim3(256), 0, s, static_cast<const S*>(x),
-                     static_cast<const S*>(g), static_cast<const S*>(b), static_cast<S*>(y), rows, eps);
-  return launch_status("layer_norm_vec_kernel launch");
-}
-
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
-
 template <typename T>
 fh_status layer_norm_typed(const void* x, const void* g, const void* b, void* y, int64_t rows, int64_t cols,
                            float eps, hipStream_t s) {
   using S = typename Io<T>::storage;
-  if (aligned16(x) && aligned16(g) && aligned16(b) && aligned16(y)) {
-    constexpr int V = 16 / static_cast<int>(sizeof(S));
-    if (cols == 64 * V) return launch_layer_norm_vec<T, V>(x, g, b, y, rows, eps, s);
-    if (cols == 64 * 2 * V) return launch_layer_norm_vec<T, 2 * V>(x, g, b, y, rows, eps, s);
-    if (cols == 64 * 4 * V) return launch_layer_norm_vec<T, 4 * V>(x, g, b, y, rows, eps, s);
-    if (V == 4 && cols == 64 * 8 * V) return launch_layer_norm_vec<T, 8 * V>(x, g, b, y, rows, eps, s);
+  const S *xs = static_cast<const S*>(x), *gs = static_cast<const S*>(g), *bs = static_cast<const S*>(b);
+  S* ys = static_cast<S*>(y);
+  constexpr int V = 16 / static_cast<int>(sizeof(S));
+  const auto row_kernel = [&]<int NV, int L, int MODE>() {
+    hipLaunchKernelGGL((layer_norm_row_kernel<T, NV, L, MODE>), dim3(row_blocks(rows, L)), dim3(256), 0, s, xs, gs, bs,
+                       ys, rows, cols, eps);
+  };
+  if (by_row_width<V>(cols, row_kernel)) return launch_status("layer_norm_row_kernel launch");
+  if (cols < V) {
+    hipLaunchKernelGGL(layer_norm_short_kernel<T>, dim3(row_blocks(rows, 64)), dim3(256), 0, s, xs, gs, bs, ys, rows,
+                       cols, eps);
+    return launch_status("layer_norm_short_kernel launch");
   }
-  if (cols <= 64 * 32) return by_width<T, LayerNormLaunch>(cols, x, g, b, y, rows, cols, eps, s);
   hipLaunchKernelGGL(layer_norm_block_kernel<T>, dim3(static_cast<uint32_t>(rows)), dim3(256), 0, s,
                      static_cast<const S*>(x), static_cast<const S*>(g), static_cast<const S*>(b), static_cast<S*>(y),
                      cols, eps);

@@ -424,6 +424,43 @@ def test_softmax_known_answer(hip):
     np.testing.assert_allclose(got, [[0.26894142, 0.73105858]] * 2, rtol=1e-6)
 
 
+# Widths around every change of lanes per row and vectors per lane (vectors of 8 16-bit or 4 fp32 elements): shorter than
+# one vector, whole and ragged vectors at 8 / 16 / 32 / 64 / 128 / 256 / 512 / 1024 / 2048 vectors, and past them. Row
+# counts leave the last workgroup ragged; x and y start one element into their buffers, so no row is 16-byte aligned,
+# and the elements around y must stay as they were.
+ROW_VECS = [0, 1, 8, 16, 32, 64, 128, 256, 512, 1024, 2048]
+
+
+@pytest.mark.parametrize("op", ["softmax", "layer_norm"])
+@pytest.mark.parametrize("dtype", [F32, BF16, F16])
+def test_row_kernel_widths(hip, op, dtype):
+    v = 4 if dtype == F32 else 8
+    widths = sorted({w for k in ROW_VECS for w in (k * v - 1, k * v, k * v + 1) if w > 0})
+    for rows, cols in [(37 if w <= 64 * v else 3, w) for w in widths]:
+        say(f"{op} dtype={dtype} {rows}x{cols}")
+        x = synth.tensor(64, (rows, cols), dtype, "normal", 2.0)
+        x[0, -1] = x[0, 0]  # (ties at both ends of a row)
+        g, b = synth.tensor(65, (cols,), dtype, "normal"), synth.tensor(66, (cols,), dtype, "normal")
+        pad = np.full(1, 7, x.dtype)
+        dx = dev(hip, np.concatenate([pad, x.ravel(), pad]))
+        dy = dev(hip, np.full(rows * cols + 2, 7, x.dtype))
+        e = x.itemsize
+        if op == "softmax":
+            hip.check(hip.lib().fh_softmax_rows(dtype, dx.value + e, dy.value + e, rows, cols, None))
+            want = orc.softmax(dtype, x)
+        else:
+            dg, db = dev(hip, g), dev(hip, b)
+            hip.check(hip.lib().fh_layer_norm_rows(dtype, dx.value + e, dg.value, db.value, dy.value + e, rows, cols, 1e-5,
+                                                   None))
+            want = orc.layer_norm(dtype, x, g, b, 1e-5)
+        got = dy.download((rows * cols + 2,), x.dtype)
+        assert got[0] == 7 and got[-1] == 7, "an element outside the output was written"
+        # the file's rule; a LayerNorm row of one or two elements divides by a variance near zero, where the rule's
+        # absolute part (the output's rms times rtol) carries it
+        assert_close(got[1:-1].reshape(x.shape), want, dtype, atol=(1e-7 if dtype == F32 else 1e-4) if op == "softmax"
+                     else None, what=f"{op} {rows}x{cols}")
+
+
 # (BF16, 4096, 1024), (BF16, 5, 512), (F16, 9, 2048), (F32, 6, 256/1024/2048) take the 16-byte vector kernel
 @pytest.mark.parametrize("dtype,rows,cols", [(F32, 2, 5), (BF16, 4096, 1024), (F32, 3, 5000), (BF16, 7, 33),
                                              (BF16, 5, 512), (F16, 9, 2048), (F32, 6, 256), (F32, 6, 1024),

@@ -296,7 +296,7 @@ __device__ __forceinline__ float epilogue_one(const EP& ep, float v, int64_t idx
   return v;
 }
 
-// Same program on one 16-byte vector of consecutive outputs starting at index idx (16-byte aligned operands).
+// Same program on one 16-byte vector of consecutive outputs starting at index idx (operands at any alignment).
 template <typename T, typename EP>
 __device__ __forceinline__ uint4 epilogue_vec(const EP& ep, uint4 packed, int64_t idx) {
   using S = typename Io<T>::storage;
@@ -312,9 +312,8 @@ __device__ __forceinline__ uint4 epilogue_vec(const EP& ep, uint4 packed, int64_
     if (s >= ep.nseg) break;
     const uint8_t op = static_cast<uint8_t>(opw >> (8 * s));
     if (ew_is_binary(op)) {
-      const uint4 in = *reinterpret_cast<const uint4*>(static_cast<const S*>(ep.ins[s]) + idx);
       S iv[V];
-      __builtin_memcpy(iv, &in, 16);
+      __builtin_memcpy(iv, static_cast<const S*>(ep.ins[s]) + idx, 16);
 #pragma unroll
       for (int x = 0; x < V; ++x) v[x] = epi_binary(op, v[x], Io<T>::load(iv[x]));
     } else {
@@ -437,7 +436,7 @@ template <int E, typename T, typename EP>
 __device__ __forceinline__ void epi_load(const EP& ep, int64_t idx, uint4* in) {
   using S = typename Io<T>::storage;
 #pragma unroll
-  for (int s = 0; s < epi_operands<E>(); ++s) in[s] = *reinterpret_cast<const uint4*>(static_cast<const S*>(ep.ins[s]) + idx);
+  for (int s = 0; s < epi_operands<E>(); ++s) __builtin_memcpy(&in[s], static_cast<const S*>(ep.ins[s]) + idx, 16);
 }
 
 template <int E, typename T, typename EP>

@@ -26,8 +26,8 @@ struct GemmArgs {
   int64_t stride_a, stride_b, stride_c;  // batch strides in elements (blockIdx.y)
   int32_t tiles_m, tiles_n;
   EpilogueArgs ep;
-  // Transposed operand storage, honoured by the sequential kernel only: A(m, k) = A[k * lda + m],
-  // B(k, n) = B[n * ldb + k].
+  // Transposed operand storage, honoured by the sequential kernel and the kernel of any alignment:
+  // A(m, k) = A[k * lda + m], B(k, n) = B[n * ldb + k].
   int32_t trans_a, trans_b;
   // FH_GEMM_ANY_ORDER: the k-sum may be reassociated (small problems then take the split-k kernel).
   int32_t any_order;

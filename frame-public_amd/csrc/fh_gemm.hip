@@ -1,21 +1,10 @@
-// Dense GEMM for gfx950: C[M,N] = A[M,K] · B[K,N], row-major, fp32 accumulation on MFMA.
+// Dense GEMM for gfx950: C[M,N] = A[M,K] · B[K,N], row-major, fp32 accumulation: the dispatch between the MFMA kernels
+// (fh_gemm16.hip, fh_gemm_any.hip, fh_gemm_f32.hip) and the kernels of small problems here.
 //
 // Semantics follow Frame's matmul (reference: src/backends/cpu/kernels/matmul.cpp:92-185): dtype in = out,
 // products accumulated in fp32, one round-to-nearest-even store. The optional epilogue applies the
 // elementwise segments Frame's graph would run next (bias add, ReLU, ...) on the rounded product before
 // the single store, rounding between segments exactly like the unfused graph.
-//
-// Tile kernel layout (one workgroup = 4 waves = 256 threads):
-//   * Block tile BM x BN, K staged in slices of 128 bytes per row (64 bf16/f16 or 32 fp32 values).
-//   * A slice is stored in LDS row-major [BM][128 B]; B slice is stored transposed [BN][128 B] so both MFMA
-//     operands read 16-byte k-contiguous fragments. B is transposed in registers (E x E blocks) between
-//     the global load and the LDS store, so global reads stay fully coalesced.
-//   * Every 16-byte chunk is XOR-swizzled inside its row by ((row ^ row>>3) & 7): fragment reads, A stores
-//     and transposed B stores are all bank-conflict free.
-//   * Two LDS stages: the global loads of slice k+1 are in flight while the MFMAs consume slice k.
-//   * Waves are laid out 2 x 2; each owns a (BM/2) x (BN/2) sub-tile of 32x32 MFMA tiles.
-//   * Workgroup ids are remapped so that consecutive tiles land on the same XCD (blocks are dispatched
-//     round-robin over the 8 XCDs) and tiles are visited in groups of rows for L2 reuse.
 #include <hip/hip_runtime.h>
 
 #include <string>
@@ -23,265 +12,12 @@
 
 #include "fh_common.h"
 #include "fh_gemm.h"
+#include "fh_gemm_any.h"
 
 namespace fh {
 namespace {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-
-template <typename T>
-struct GemmTraits;
-template <>
-struct GemmTraits<bf16_t> {
-  static constexpr int E = 8;  // elements per 16-byte chunk
-};
-template <>
-struct GemmTraits<f16_t> {
-  static constexpr int E = 8;
-};
-template <>
-struct GemmTraits<float> {
-  static constexpr int E = 4;
-};
-
-__device__ __forceinline__ int swz(int row, int chunk) { return chunk ^ ((row ^ (row >> 3)) & 7); }
-
-// Transposes an E x E block of 16-bit values held as E rows of 16 bytes.
-__device__ __forceinline__ void transpose8x8_u16(const uint4 (&in)[8], uint4 (&out)[8]) {
-  const uint32_t* src = reinterpret_cast<const uint32_t*>(in);  // src[r*4 + d]
-  uint32_t* dst = reinterpret_cast<uint32_t*>(out);
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const uint32_t a = src[(2 * q) * 4 + (c >> 1)];
-      const uint32_t b = src[(2 * q + 1) * 4 + (c >> 1)];
-      dst[c * 4 + q] = (c & 1) ? ((a >> 16) | (b & 0xffff0000u)) : ((a & 0xffffu) | (b << 16));
-    }
-  }
-}
-
-__device__ __forceinline__ void transpose4x4_u32(const uint4 (&in)[4], uint4 (&out)[4]) {
-  const uint32_t* src = reinterpret_cast<const uint32_t*>(in);
-  uint32_t* dst = reinterpret_cast<uint32_t*>(out);
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) dst[c * 4 + r] = src[r * 4 + c];
-}
-
-template <typename T>
-__device__ __forceinline__ void mfma_step(const uint4& a, const uint4& b, f32x16_t& acc);
-
-template <>
-__device__ __forceinline__ void mfma_step<bf16_t>(const uint4& a, const uint4& b, f32x16_t& acc) {
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b),
-                                                acc, 0, 0, 0);
-}
-template <>
-__device__ __forceinline__ void mfma_step<f16_t>(const uint4& a, const uint4& b, f32x16_t& acc) {
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b),
-                                               acc, 0, 0, 0);
-}
-// fp32: one 16-byte chunk holds 4 k-values; lane halves read different chunks and both operands use the
-// same k assignment, so four 32x32x2 MFMAs consume the pair of chunks.
-template <>
-__device__ __forceinline__ void mfma_step<float>(const uint4& a, const uint4& b, f32x16_t& acc) {
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.x), __uint_as_float(b.x), acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.y), __uint_as_float(b.y), acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.z), __uint_as_float(b.z), acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.w), __uint_as_float(b.w), acc, 0, 0, 0);
-}
-
-template <typename T, int BM, int BN, bool kGuard>
-__global__ __launch_bounds__(256) void gemm_tile_kernel(GemmArgs args) {
-  using S = typename Io<T>::storage;
-  constexpr int E = GemmTraits<T>::E;
-  constexpr int BK = 8 * E;  // 128 bytes of K per row
-  constexpr int WM = BM / 2, WN = BN / 2;
-  constexpr int TM = WM / 32, TN = WN / 32;
-  constexpr int A_LOADS = BM * 8 / 256;
-  constexpr int B_BLOCKS = 8 * BN / E;  // E x E blocks in a K slice
-  constexpr int B_ITERS = (B_BLOCKS + 255) / 256;
-  constexpr int NB_PER_ROW = BN / E;
-  static_assert(A_LOADS >= 1, "BM too small");
-
-  __shared__ uint4 lds[2][(BM + BN) * 8];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-
-  // --- tile scheduling: XCD-aware remap, then grouped row-major order ---
-  const int tiles = args.tiles_m * args.tiles_n;
-  int bid = blockIdx.x;
-  if ((tiles & 7) == 0) bid = (bid & 7) * (tiles >> 3) + (bid >> 3);
-  constexpr int GROUP_M = 4;
-  const int group = bid / (GROUP_M * args.tiles_n);
-  const int first_m = group * GROUP_M;
-  const int gsize = min(args.tiles_m - first_m, GROUP_M);
-  const int tm = first_m + (bid % gsize);
-  const int tn = (bid % (GROUP_M * args.tiles_n)) / gsize;
-  const int64_t m0 = static_cast<int64_t>(tm) * BM;
-  const int64_t n0 = static_cast<int64_t>(tn) * BN;
-
-  const S* __restrict__ A = static_cast<const S*>(args.A) + blockIdx.y * args.stride_a;
-  const S* __restrict__ B = static_cast<const S*>(args.B) + blockIdx.y * args.stride_b;
-  S* __restrict__ C = static_cast<S*>(args.C) + blockIdx.y * args.stride_c;
-  const int64_t M = args.M, N = args.N, K = args.K;
-  const int64_t lda = args.lda, ldb = args.ldb, ldc = args.ldc;
-
-  uint4 ra[A_LOADS];
-  uint4 rb[B_ITERS][E];
-
-  auto load_slice = [&](int kt) {
-    const int64_t k0 = static_cast<int64_t>(kt) * BK;
-#pragma unroll
-    for (int i = 0; i < A_LOADS; ++i) {
-      const int id = tid + 256 * i;
-      const int row = id >> 3, c = id & 7;
-      const int64_t gr = m0 + row, gk = k0 + c * E;
-      if (!kGuard || (gr < M && gk < K)) {
-        ra[i] = *reinterpret_cast<const uint4*>(A + gr * lda + gk);
-      } else {
-        ra[i] = make_uint4(0, 0, 0, 0);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < B_ITERS; ++j) {
-      const int blk = tid + 256 * j;
-      const int kb = blk / NB_PER_ROW, nb = blk % NB_PER_ROW;
-      const int64_t gn = n0 + nb * E;
-#pragma unroll
-      for (int r = 0; r < E; ++r) {
-        const int64_t gk = k0 + kb * E + r;
-        if ((B_BLOCKS % 256 == 0 || blk < B_BLOCKS) && (!kGuard || (gk < K && gn < N))) {
-          rb[j][r] = *reinterpret_cast<const uint4*>(B + gk * ldb + gn);
-        } else {
-          rb[j][r] = make_uint4(0, 0, 0, 0);
-        }
-      }
-    }
-  };
-
-  auto store_slice = [&](int buf) {
-    uint4* As = lds[buf];
-    uint4* Bs = lds[buf] + BM * 8;
-#pragma unroll
-    for (int i = 0; i < A_LOADS; ++i) {
-      const int id = tid + 256 * i;
-      const int row = id >> 3, c = id & 7;
-      As[row * 8 + swz(row, c)] = ra[i];
-    }
-#pragma unroll
-    for (int j = 0; j < B_ITERS; ++j) {
-      const int blk = tid + 256 * j;
-      if (B_BLOCKS % 256 != 0 && blk >= B_BLOCKS) continue;
-      const int kb = blk / NB_PER_ROW, nb = blk % NB_PER_ROW;
-      uint4 t[E];
-      if constexpr (E == 8) {
-        transpose8x8_u16(rb[j], t);
-      } else {
-        transpose4x4_u32(rb[j], t);
-      }
-#pragma unroll
-      for (int c = 0; c < E; ++c) {
-        const int n = nb * E + c;
-        Bs[n * 8 + swz(n, kb)] = t[c];
-      }
-    }
-  };
-
-  f32x16_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
-  const int KT = static_cast<int>((K + BK - 1) / BK);
-  const int half = lane >> 5;
-  const int l32 = lane & 31;
-
-  load_slice(0);
-  store_slice(0);
-  __syncthreads();
-
-  for (int kt = 0; kt < KT; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < KT) load_slice(kt + 1);
-    const uint4* As = lds[cur];
-    const uint4* Bs = lds[cur] + BM * 8;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const int chunk = 2 * ks + half;
-      uint4 a[TM], b[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int row = wm * WM + i * 32 + l32;
-        a[i] = As[row * 8 + swz(row, chunk)];
-      }
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int row = wn * WN + j * 32 + l32;
-        b[j] = Bs[row * 8 + swz(row, chunk)];
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) mfma_step<T>(a[i], b[j], acc[i][j]);
-    }
-    if (kt + 1 < KT) store_slice(cur ^ 1);
-    __syncthreads();
-  }
-
-  // --- epilogue: stage the rounded tile through LDS (free after the last barrier), then each wave runs the
-  // elementwise program on 16-byte vectors and stores them coalesced. Rounding the product to T before
-  // staging loses nothing: the epilogue starts from the rounded product anyway. ---
-  constexpr int V = 16 / static_cast<int>(sizeof(S));       // elements per 16-byte vector
-  constexpr int CAP = (BM + BN) * 64 / static_cast<int>(sizeof(S));  // LDS elements owned by one wave
-  constexpr int RP_RAW = (CAP / WN) / 32 * 32;
-  constexpr int RP = RP_RAW < WM ? RP_RAW : WM;               // wave rows staged per pass
-  constexpr int PASSES = WM / RP;
-  constexpr int LPR = WN / V;                                  // lanes per staged row
-  constexpr int RPI = 64 / LPR;                                // staged rows per wave-wide access
-  static_assert(RP >= 32 && WM % RP == 0 && 64 % LPR == 0, "epilogue staging shape");
-  S* wl = reinterpret_cast<S*>(&lds[0][0]) + wave * CAP;
-#pragma unroll
-  for (int p = 0; p < PASSES; ++p) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      if (i / (RP / 32) != p) continue;
-      const int rbase = (i % (RP / 32)) * 32;
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int rr = rbase + 8 * (r >> 2) + 4 * half + (r & 3);
-          wl[rr * WN + j * 32 + l32] = Io<T>::store(acc[i][j][r]);
-        }
-    }
-    __syncthreads();
-    const int c = (lane % LPR) * V;
-    const int64_t col = n0 + wn * WN + c;
-#pragma unroll 4
-    for (int it = 0; it < RP / RPI; ++it) {
-      const int rr = it * RPI + lane / LPR;
-      const int64_t row = m0 + wm * WM + p * RP + rr;
-      if (kGuard && (row >= M || col >= N)) continue;
-      uint4 packed = *reinterpret_cast<const uint4*>(wl + rr * WN + c);
-      const int64_t idx = row * ldc + col;
-      if (args.ep.nseg > 0) packed = epilogue_vec<T>(args.ep, packed, idx);
-      *reinterpret_cast<uint4*>(C + idx) = packed;
-    }
-    if (p + 1 < PASSES) __syncthreads();
-  }
-}
-
-// Small and unaligned GEMMs (few output tiles, or rows/columns the tile kernels cannot take): one thread per
+// Small GEMMs (few output tiles, or fewer columns than the tile kernels take): one thread per
 // output of a 16 x 16 tile, its k loop strictly sequential like the reference CPU kernel (fp32 products and sums,
 // no contraction, one rounding), so the result is bit-identical to it. K is staged through LDS in chunks of kKC as
 // fp32, A row-major and B transposed, both k-contiguous so each step reads 4 k-values per operand with one
@@ -471,48 +207,26 @@ __global__ __launch_bounds__(kSplitWaves * 64) void gemm_split_kernel(GemmArgs a
   }
 }
 
-template <typename T, int BM, int BN>
-fh_status launch_tile(GemmArgs args, int64_t batch, hipStream_t stream) {
-  args.tiles_m = static_cast<int32_t>((args.M + BM - 1) / BM);
-  args.tiles_n = static_cast<int32_t>((args.N + BN - 1) / BN);
-  constexpr int BK = 8 * GemmTraits<T>::E;
-  const bool full = (args.M % BM == 0) && (args.N % BN == 0) && (args.K % BK == 0);
-  dim3 grid(static_cast<uint32_t>(args.tiles_m) * static_cast<uint32_t>(args.tiles_n),
-            static_cast<uint32_t>(batch));
-  if (full) {
-    hipLaunchKernelGGL((gemm_tile_kernel<T, BM, BN, false>), grid, dim3(256), 0, stream, args);
-  } else {
-    hipLaunchKernelGGL((gemm_tile_kernel<T, BM, BN, true>), grid, dim3(256), 0, stream, args);
-  }
-  return launch_status("gemm_tile_kernel launch");
-}
-
-bool epilogue_aligned(const EpilogueArgs& ep) {
-  for (int s = 0; s < ep.nseg; ++s)
-    if (ew_is_binary(ep.ops[s]) && reinterpret_cast<uintptr_t>(ep.ins[s]) % 16 != 0) return false;
-  return true;
-}
-
 template <typename T>
 fh_status dispatch_gemm(GemmArgs args, int64_t batch, hipStream_t stream) {
-  constexpr int E = GemmTraits<T>::E;
   const int cus = device_cu_count();
   // Few 64 x 64 tiles: the sequential kernel, whose 16 x 16 tiles spread further and whose latency is a handful
   // of K chunks. fp32 below a quarter of the CUs; 16-bit only below 16 tiles (its MFMA kernel stays faster down
   // to there: the C4 classifier, 16 tiles, 7.8 us there against 22 us sequential).
   const int64_t tiles64 = ((args.M + 63) / 64) * ((args.N + 63) / 64) * batch;
   const bool small = (std::is_same_v<T, float> ? tiles64 * 4 < cus : tiles64 < 16) && args.K <= 16384;
-  if constexpr (!std::is_same_v<T, float>) {
-    fh_status st = FH_OK;
-    if (!small && gemm16_try_launch(std::is_same_v<T, bf16_t> ? FH_BF16 : FH_F16, args, batch, stream, &st)) return st;
+  // everything else on the matrix cores: 16-bit operands of whole 16-byte vectors on the aligned pipeline, the rest on
+  // the kernel of any size and alignment
+  fh_status st = FH_OK;
+  if (!small && !args.row_softmax) {
+    if constexpr (std::is_same_v<T, float>) {
+      if (gemm_f32_try_launch(args, batch, stream, &st)) return st;
+    } else {
+      const int32_t dtype = std::is_same_v<T, bf16_t> ? FH_BF16 : FH_F16;
+      if (!args.trans_a && !args.trans_b && gemm16_try_launch(dtype, args, batch, stream, &st)) return st;
+      if (gemm_any16_try_launch(dtype, args, batch, stream, &st)) return st;
+    }
   }
-  const size_t esz = sizeof(typename Io<T>::storage);
-  const bool aligned = (reinterpret_cast<uintptr_t>(args.A) % 16 == 0) &&
-                       (reinterpret_cast<uintptr_t>(args.B) % 16 == 0) && (args.K % E == 0) &&
-                       (args.N % E == 0) && (args.lda % E == 0) && (args.ldb % E == 0) &&
-                       ((args.stride_a * esz) % 16 == 0) && ((args.stride_b * esz) % 16 == 0) &&
-                       (reinterpret_cast<uintptr_t>(args.C) % 16 == 0) && (args.ldc % E == 0) &&
-                       ((args.stride_c * esz) % 16 == 0) && epilogue_aligned(args.ep);
   const bool split_ok = args.any_order && !args.trans_a && !args.trans_b &&
                         (args.M + kSplitTM - 1) / kSplitTM <= 65535 && batch <= 65535;
   if (args.row_softmax && (!split_ok || args.N > kSplitTN))
@@ -524,19 +238,13 @@ fh_status dispatch_gemm(GemmArgs args, int64_t batch, hipStream_t stream) {
     hipLaunchKernelGGL((gemm_split_kernel<T>), grid, dim3(kSplitWaves * 64), 0, stream, args);
     return launch_status("gemm_split_kernel launch");
   }
-  // small problems, or operands the tile kernels cannot take
-  if (!aligned || small) {
-    if ((args.M + kSeqT - 1) / kSeqT > 65535 || batch > 65535)
-      return fail(FH_UNIMPLEMENTED, "fh_gemm: unaligned operands with more than 1,048,560 rows or 65,535 batches");
-    dim3 grid(static_cast<uint32_t>((args.N + kSeqT - 1) / kSeqT), static_cast<uint32_t>((args.M + kSeqT - 1) / kSeqT),
-              static_cast<uint32_t>(batch));
-    hipLaunchKernelGGL((gemm_seq_kernel<T>), grid, dim3(256), 0, stream, args);
-    return launch_status("gemm_seq_kernel launch");
-  }
-  auto tiles = [&](int64_t t) { return ((args.M + t - 1) / t) * ((args.N + t - 1) / t) * batch; };
-  if (tiles(256) >= cus) return launch_tile<T, 256, 256>(args, batch, stream);
-  if (tiles(128) >= cus / 2) return launch_tile<T, 128, 128>(args, batch, stream);
-  return launch_tile<T, 64, 64>(args, batch, stream);
+  // small problems, and the few that no MFMA kernel takes (N below 8)
+  if ((args.M + kSeqT - 1) / kSeqT > 65535 || batch > 65535)
+    return fail(FH_UNIMPLEMENTED, "fh_gemm: fewer than 8 columns with more than 1,048,560 rows or 65,535 batches");
+  dim3 grid(static_cast<uint32_t>((args.N + kSeqT - 1) / kSeqT), static_cast<uint32_t>((args.M + kSeqT - 1) / kSeqT),
+            static_cast<uint32_t>(batch));
+  hipLaunchKernelGGL((gemm_seq_kernel<T>), grid, dim3(256), 0, stream, args);
+  return launch_status("gemm_seq_kernel launch");
 }
 
 fh_status run_gemm(int32_t dtype, GemmArgs args, int64_t batch, hipStream_t stream) {

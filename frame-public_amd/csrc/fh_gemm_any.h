@@ -1,0 +1,431 @@
+// GEMM of any size and alignment, either operand transposed, for 16-bit and fp32 operands: C = op(A) · op(B) with fp32
+// accumulation on v_mfma_f32_16x16x32, one rounding per output, then the optional elementwise epilogue (semantics of
+// Frame's matmul and its gradients: reference src/backends/cpu/kernels/matmul.cpp:92-327). The kernel template; its
+// instances and their dispatch are in fh_gemm_any.hip (16-bit) and fh_gemm_f32.hip (fp32).
+//
+// Operands go global -> registers -> LDS in units of 8 elements along their contiguous index, so a unit needs element
+// alignment only (global memory takes 16-byte accesses at any alignment) and edges are handled per unit: rows past the
+// edge are clamped to the last valid one (their products land in discarded outputs), and the last k tile is loaded
+// element by element with zeros past K when K or a contiguous width leaves a remainder. Two register sets and two LDS
+// buffers: the loads of tile k+2 and the LDS writes of tile k+1 are issued around the products of tile k, with one
+// barrier per tile.
+//
+// An operand that is contiguous along k (A as stored, B transposed) lies in LDS as rows of 32 k and is read with
+// ds_read_b128; one that is contiguous along m or n (A transposed, B as stored) lies as 32 k rows and is read with the
+// LDS transpose read ds_read_b64_tr_b16: neither needs a transposed copy.
+//
+// fp32 operands are split on their way to LDS into three bf16 planes, x = x1 + x2 + x3 (each the round-to-nearest bf16
+// of what the ones before it leave: 24 bits, exact for |x| >= 2^-110), and a product is the six plane products
+// x1 y1 + x1 y2 + x2 y1 + x2 y2 + x1 y3 + x3 y1 summed in fp32. The three left out are below 2^-26 of |x y| together, under
+// the rounding of a single fp32 product. The bf16 matrix rate is 16 times the fp32 one, so six products take 6/16 of
+// the time. Operands outside the split's range (an infinity or NaN, a finite value that rounds to a bf16 infinity, a
+// nonzero value below 2^-110) send the tile to plain fp32 MFMA after the loop: the first two make the accumulators
+// non-finite, the third is tracked while splitting.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+#include <utility>
+
+#include "fh_common.h"
+#include "fh_gemm.h"
+#include "fh_mfma16.h"
+
+namespace fh {
+namespace gemm_any {
+
+using namespace mfma16;
+
+typedef u32x4_t u32x4_any __attribute__((aligned(2)));
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+
+template <typename T>
+struct AnyTraits {
+  static constexpr int P = 1;  // planes in LDS
+  using mfma_t = T;
+};
+template <>
+struct AnyTraits<float> {
+  static constexpr int P = 3;
+  using mfma_t = bf16_t;
+};
+
+// Eight consecutive elements as loaded.
+template <typename T>
+struct Unit {
+  static constexpr int R = sizeof(typename Io<T>::storage) / 2;  // 16-byte registers
+  u32x4_t v[R];
+};
+
+template <typename T>
+__device__ __forceinline__ Unit<T> load_unit(const typename Io<T>::storage* p) {
+  Unit<T> u;
+#pragma unroll
+  for (int i = 0; i < Unit<T>::R; ++i) u.v[i] = *(reinterpret_cast<const u32x4_any*>(p) + i);
+  return u;
+}
+
+// Element e of the unit at p when it is one of the first n, zero otherwise.
+template <typename T>
+__device__ __forceinline__ Unit<T> load_unit_partial(const typename Io<T>::storage* p, int n) {
+  typename Io<T>::storage e[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) e[i] = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    if (i < n) e[i] = p[i];
+  Unit<T> u;
+  __builtin_memcpy(&u, e, sizeof(u));
+  return u;
+}
+
+// 2^-110 as (bits << 1) - 1, the key that zero wraps to the top of.
+constexpr uint32_t kTinyKey = (static_cast<uint32_t>(127 - 110) << 24) - 1;
+
+// The unit's planes as packed 16-bit vectors. fp32: tracks the smallest key of its elements in `tiny`.
+template <typename T>
+__device__ __forceinline__ void split_unit(const Unit<T>& u, u32x4_t (&plane)[AnyTraits<T>::P], uint32_t& tiny) {
+  if constexpr (std::is_same_v<T, float>) {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const uint32_t b0 = u.v[d / 2][2 * (d % 2)], b1 = u.v[d / 2][2 * (d % 2) + 1];
+      tiny = min(tiny, min((b0 << 1) - 1u, (b1 << 1) - 1u));
+      float x0 = __uint_as_float(b0), x1 = __uint_as_float(b1);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        const uint32_t w = store2<bf16_t>(x0, x1);
+        plane[p][d] = w;
+        x0 -= __uint_as_float(w << 16);
+        x1 -= __uint_as_float(w & 0xffff0000u);
+      }
+    }
+  } else {
+    plane[0] = u.v[0];
+  }
+}
+
+// One operand of a tile: ROWS rows (of A) or columns (of B), BK k, held by NT threads as UNITS units each. KC: memory
+// is contiguous along k.
+template <typename T, int ROWS, int BK, int NT, bool KC>
+struct Operand {
+  using S = typename Io<T>::storage;
+  static constexpr int P = AnyTraits<T>::P;
+  static constexpr int UNITS = ROWS * BK / 8 / NT;
+  static constexpr int CHUNKS = ROWS / 8;       // units per k row (MC)
+  static constexpr int SUB = ROWS * 64;         // bytes of one plane's k32 block in LDS
+  static constexpr int PLANE = SUB * (BK / 32);
+  static constexpr int BYTES = PLANE * P;
+  static_assert(ROWS * BK / 8 % NT == 0 && UNITS >= 1, "whole units per thread");
+  static_assert(KC || CHUNKS >= 8, "the k rows' swizzle moves a chunk within eight");
+
+  const S* src[UNITS];  // unit's address at k tile 0
+  int dst[UNITS];       // its LDS offset
+  int kk[UNITS];        // its k (KC: first of 8; MC: the row) within the tile
+  int left[UNITS];      // MC: valid elements from its first (8 or more: all)
+  Unit<T> reg[2][UNITS];
+  int64_t step;         // elements from one k tile to the next
+
+  __device__ void init(const S* base, int64_t ld, int64_t r0, int64_t rows, int tid) {
+    step = KC ? BK : BK * ld;
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+      const int id = tid + NT * u;
+      if constexpr (KC) {
+        const int row = id / (BK / 8), c = id % (BK / 8);
+        kk[u] = c * 8;
+        left[u] = 8;
+        src[u] = base + min(r0 + row, rows - 1) * ld + c * 8;
+        dst[u] = (c / 4) * SUB + row * 64 + (((c % 4) ^ a_swizzle(row)) * 16);
+      } else {
+        const int row = id / CHUNKS, c = id % CHUNKS;
+        kk[u] = row;
+        // a unit past the edge reads the last whole unit's columns instead (discarded); one that straddles the edge
+        // runs into the next k row, which exists in every tile but the last
+        const int64_t col = r0 + c * 8 < rows ? r0 + c * 8 : rows - 8;
+        left[u] = static_cast<int>(min<int64_t>(rows - col, 8));
+        src[u] = base + static_cast<int64_t>(row) * ld + col;
+        dst[u] = (row / 32) * SUB + (row % 32) * (ROWS * 2) + ((c ^ b_swizzle16<CHUNKS>(row % 32)) * 16);
+      }
+    }
+  }
+  template <int SET>
+  __device__ void load(int64_t kt) {
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) reg[SET][u] = load_unit<T>(src[u] + kt * step);
+  }
+  // The last tile, k0 .. K - 1, with zeros for the rest.
+  template <int SET>
+  __device__ void load_tail(int64_t kt, int64_t left_k) {
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+      const int64_t k = left_k - kk[u];  // valid k from this unit's first
+      const int n = KC ? static_cast<int>(min<int64_t>(max<int64_t>(k, 0), 8)) : (k > 0 ? left[u] : 0);
+      reg[SET][u] = load_unit_partial<T>(src[u] + kt * step, n);
+    }
+  }
+  template <int SET>
+  __device__ void store(unsigned char* lds, uint32_t& tiny) {
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+      u32x4_t plane[P];
+      split_unit<T>(reg[SET][u], plane, tiny);
+#pragma unroll
+      for (int p = 0; p < P; ++p) *reinterpret_cast<u32x4_t*>(lds + p * PLANE + dst[u]) = plane[p];
+    }
+  }
+
+  // Fragment of the 16 rows (columns) from w on, in the k32 block at `sub`: lane l holds row w + l % 16, k 8 (l / 16)..+7.
+  __device__ static u32x4_t fragment(const unsigned char* sub, int w, int lane) {
+    if constexpr (KC) {
+      const int row = w + (lane & 15);
+      return *reinterpret_cast<const u32x4_t*>(sub + row * 64 + (((lane >> 4) ^ a_swizzle(row)) * 16));
+    } else {
+      const int q = lane & 3, e = (lane >> 2) & 3;
+      const int col = w + 4 * q, krow = 8 * (lane >> 4) + e;
+      const unsigned char* p = sub + krow * (ROWS * 2) + (((col >> 3) ^ b_swizzle16<CHUNKS>(krow)) * 16) + (col & 7) * 2;
+      const auto lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FH_LDS s16x4_t*)(p));
+      const auto hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FH_LDS s16x4_t*)(p + 4 * ROWS * 2));
+      const u32x2_t a = __builtin_bit_cast(u32x2_t, lo), b = __builtin_bit_cast(u32x2_t, hi);
+      return u32x4_t{a[0], a[1], b[0], b[1]};
+    }
+  }
+};
+
+// Barrier over LDS traffic only: the register prefetch stays in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <typename T, int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool TA, bool TB, int E>
+__global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_any_kernel(GemmArgs args) {
+  using S = typename Io<T>::storage;
+  using M16 = typename AnyTraits<T>::mfma_t;
+  constexpr bool F32 = std::is_same_v<T, float>;
+  constexpr int P = AnyTraits<T>::P;
+  constexpr int NT = WAVES_M * WAVES_N * 64;
+  constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
+  constexpr int TM = WM / 16, TN = WN / 16;
+  using OpA = Operand<T, BM, BK, NT, !TA>;
+  using OpB = Operand<T, BN, BK, NT, TB>;
+  constexpr int BUF = OpA::BYTES + OpB::BYTES;
+  constexpr int STAGED = WAVES_M * WAVES_N * WM * WN * static_cast<int>(sizeof(S));
+  static_assert(STAGED <= 2 * BUF, "the wave tiles fit in the buffers");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * BUF];
+  __shared__ int tiny_seen;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+
+  // tile id: consecutive tiles on one XCD (any tile count), in groups of 8 tile rows
+  const int tiles = args.tiles_m * args.tiles_n;
+  const int xcd = blockIdx.x & 7;
+  int bid = xcd * (tiles >> 3) + min(xcd, tiles & 7) + static_cast<int>(blockIdx.x >> 3);
+  constexpr int GROUP_M = 8;
+  const int group = bid / (GROUP_M * args.tiles_n);
+  const int gsize = min(args.tiles_m - group * GROUP_M, GROUP_M);
+  const int in_group = bid % (GROUP_M * args.tiles_n);
+  const int64_t m0 = static_cast<int64_t>(group * GROUP_M + in_group % gsize) * BM;
+  const int64_t n0 = static_cast<int64_t>(in_group / gsize) * BN;
+
+  const S* __restrict__ A = static_cast<const S*>(args.A) + blockIdx.y * args.stride_a;
+  const S* __restrict__ B = static_cast<const S*>(args.B) + blockIdx.y * args.stride_b;
+  S* __restrict__ C = static_cast<S*>(args.C) + blockIdx.y * args.stride_c;
+  const int64_t M = args.M, N = args.N, K = args.K;
+  const int KT = static_cast<int>((K + BK - 1) / BK);
+  const bool tail = K % BK != 0 || (TA && M % 8 != 0) || (!TB && N % 8 != 0);
+  const int whole = tail ? KT - 1 : KT;  // tiles without a remainder
+
+  OpA a;
+  OpB b;
+  a.init(A, args.lda, m0, M, tid);
+  b.init(B, args.ldb, n0, N, tid);
+  uint32_t tiny = ~0u;
+  if (F32 && tid == 0) tiny_seen = 0;
+
+  auto load = [&]<int SET>(int kt) {
+    if (kt < whole) {
+      a.template load<SET>(kt);
+      b.template load<SET>(kt);
+    } else if (kt < KT) {
+      a.template load_tail<SET>(kt, K - static_cast<int64_t>(kt) * BK);
+      b.template load_tail<SET>(kt, K - static_cast<int64_t>(kt) * BK);
+    }
+  };
+  auto store = [&]<int SET>(unsigned char* buf) {
+    a.template store<SET>(buf, tiny);
+    b.template store<SET>(buf + OpA::BYTES, tiny);
+  };
+
+  f32x4_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+  auto products = [&](const unsigned char* buf) {
+#pragma unroll
+    for (int s = 0; s < BK / 32; ++s) {
+      u32x4_t fa[P][TM], fb[P][TN];
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+          fa[p][i] = OpA::fragment(buf + p * OpA::PLANE + s * OpA::SUB, wm * WM + i * 16, lane);
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          fb[p][j] = OpB::fragment(buf + OpA::BYTES + p * OpB::PLANE + s * OpB::SUB, wn * WN + j * 16, lane);
+      }
+      auto pair = [&]<int PA, int PB>() {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) mfma16x<M16>(fa[PA][i], fb[PB][j], acc[i][j]);
+      };
+      pair.template operator()<0, 0>();
+      if constexpr (F32) {
+        pair.template operator()<0, 1>();
+        pair.template operator()<1, 0>();
+        pair.template operator()<1, 1>();
+        pair.template operator()<0, 2>();
+        pair.template operator()<2, 0>();
+      }
+    }
+  };
+
+  // step kt: loads of kt + 2 into the set that tile kt left, products of kt, LDS writes of kt + 1, barrier
+  auto step = [&]<int SET>(int kt) {
+    load.template operator()<SET>(kt + 2);
+    products(lds + SET * BUF);
+    if (kt + 1 < KT) store.template operator()<1 - SET>(lds + (1 - SET) * BUF);
+    lds_barrier();
+  };
+  if (KT > 0) {
+    load.template operator()<0>(0);
+    load.template operator()<1>(1);
+    store.template operator()<0>(lds);
+    lds_barrier();
+    for (int kt = 0; kt < KT; kt += 2) {
+      step.template operator()<0>(kt);
+      if (kt + 1 < KT) step.template operator()<1>(kt + 1);
+    }
+  }
+
+  const int g = lane >> 4, r = lane & 15;
+  if constexpr (F32) {
+    if (tiny < kTinyKey) tiny_seen = 1;
+    __syncthreads();
+    bool bad = tiny_seen != 0;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) bad |= !(__builtin_fabsf(acc[i][j][x]) <= 3.4028234663852886e38f);
+    if (__any(bad)) {
+      // outside the split's range: this wave's tile again, on fp32 operands from memory
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int64_t k0 = 0; k0 < K; k0 += 4) {
+        const int64_t k = k0 + g;
+        float va[TM], vb[TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const int64_t row = min(m0 + wm * WM + i * 16 + r, M - 1);
+          va[i] = k < K ? A[TA ? k * args.lda + row : row * args.lda + k] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int64_t col = min(n0 + wn * WN + j * 16 + r, N - 1);
+          vb[j] = k < K ? B[TB ? col * args.ldb + k : k * args.ldb + col] : 0.0f;
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[i], vb[j], acc[i][j], 0, 0, 0);
+      }
+    }
+  }
+
+  // epilogue: each wave stages its rounded tile in LDS (free: every wave is past its last read), then runs the program
+  // on 8 or 4 outputs at a time; the columns of a vector that straddles the edge go one by one
+  S* wl = reinterpret_cast<S*>(lds) + wave * (WM * WN);
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) wl[(i * 16 + 4 * g + x) * WN + j * 16 + r] = Io<T>::store(acc[i][j][x]);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+  constexpr int V = 16 / static_cast<int>(sizeof(S));
+  constexpr int LPR = WN / V, RPI = 64 / LPR;
+  static_assert(64 % LPR == 0 && WM % RPI == 0, "epilogue access shape");
+  const int c = (lane % LPR) * V;
+  const int64_t col = n0 + wn * WN + c;
+  const EpilogueArgs& ep = args.ep;
+  for (int it = 0; it < WM / RPI; ++it) {
+    const int rr = it * RPI + lane / LPR;
+    const int64_t row = m0 + wm * WM + rr;
+    if (row >= M || col >= N) continue;
+    const int64_t idx = row * args.ldc + col;
+    if (col + V <= N) {
+      const uint4 out = epi_vec<E, T>(ep, *reinterpret_cast<const uint4*>(wl + rr * WN + c), idx);
+      *reinterpret_cast<u32x4_any*>(C + idx) = u32x4_t{out.x, out.y, out.z, out.w};
+    } else {
+      for (int x = 0; x < N - col; ++x)
+        C[idx + x] = Io<T>::store(epi_one<E, T>(ep, Io<T>::load(wl[rr * WN + c + x]), idx + x));
+    }
+  }
+}
+
+template <typename T, int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool TA, bool TB>
+fh_status launch(GemmArgs args, int64_t batch, hipStream_t stream) {
+  args.tiles_m = static_cast<int32_t>((args.M + BM - 1) / BM);
+  args.tiles_n = static_cast<int32_t>((args.N + BN - 1) / BN);
+  const dim3 grid(static_cast<uint32_t>(args.tiles_m) * static_cast<uint32_t>(args.tiles_n),
+                  static_cast<uint32_t>(batch));
+  auto go = [&]<int E>() {
+    hipLaunchKernelGGL((gemm_any_kernel<T, BM, BN, BK, WAVES_M, WAVES_N, TA, TB, E>), grid,
+                       dim3(WAVES_M * WAVES_N * 64), 0, stream, args);
+    return launch_status("gemm_any_kernel launch");
+  };
+  // the programs that Linear layers carry have kernels of their own, the rest takes the interpreter (see EpiKind);
+  // gradients (a transposed operand) carry none
+  if constexpr (!TA && !TB && !std::is_same_v<T, f16_t>) {
+    switch (epi_kind(args.ep)) {
+      case kEpiNone: return go.template operator()<kEpiNone>();
+      case kEpiAdd: return go.template operator()<kEpiAdd>();
+      case kEpiAddRelu: return go.template operator()<kEpiAddRelu>();
+      case kEpiAddGelu: return go.template operator()<kEpiAddGelu>();
+      default: break;
+    }
+  } else {
+    if (args.ep.nseg == 0) return go.template operator()<kEpiNone>();
+  }
+  return go.template operator()<kEpiAny>();
+}
+
+// What the kernel accepts: an operand contiguous along m or n needs 8 of them (its units are moved back to the edge)
+// and a row stride of as many (a unit that straddles the edge runs into the next row).
+inline bool accepts(const GemmArgs& args, int64_t batch) {
+  if (args.K <= 0 || args.groups > 0 || args.row_softmax || batch > 65535) return false;
+  if (args.trans_a ? args.M < 8 : false) return false;
+  if (args.trans_b ? false : args.N < 8) return false;
+  const int64_t tiles = ((args.M + 63) / 64) * ((args.N + 63) / 64);
+  return args.K <= (int64_t{1} << 30) && tiles <= 0x7fffffff;
+}
+
+}  // namespace gemm_any
+
+// Launches the kernel and returns true, with the launch's status in *status; false (and nothing launched) for a
+// problem it does not accept.
+bool gemm_any16_try_launch(int32_t dtype, const GemmArgs& args, int64_t batch, hipStream_t stream, fh_status* status);
+bool gemm_f32_try_launch(const GemmArgs& args, int64_t batch, hipStream_t stream, fh_status* status);
+
+}  // namespace fh

@@ -67,8 +67,8 @@ __device__ __forceinline__ float softmax_div(float e, float s, float r) {
 // is moved back to end at the row's end; the elements it then shares with the vector before it ("dup" of them) are
 // left out of the sums, and both lanes store them with the same value.
 // What bounds these kernels is HBM once the accesses are vectors (softmax bf16, us, one element per lane and access
-// before): [32768, 1000] 52.7 -> 25.5 (5.1 TB/s), [32768, 1001] 53.5 -> 26.5, [65536, 47] f32 12.7 -> 6.9; rows of
-// more than 2,048 elements, in three passes over memory before: [4096, 8192] f16 98 -> 30.
+// before): [32768, 1000] 53.0 -> 23.6 (5.6 TB/s), [32768, 1001] 53.7 -> 26.4, [65536, 47] f32 12.7 -> 6.9; rows of
+// more than 2,048 elements, in three passes over memory before: [4096, 8192] f16 98 -> 24.
 enum RowMode { kRowFull, kRowVectors, kRowRagged };
 
 template <int V, int NV, int L, int MODE>

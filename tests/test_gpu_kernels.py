@@ -97,6 +97,83 @@ def test_gemm_small_bit_exact(hip, dtype, shape):
     assert_bitwise(run_gemm(hip, dtype, a, b), orc.matmul(dtype, a, b), f"small gemm {shape}")
 
 
+# GEMMs whose sizes are no whole tiles or vectors, on the MFMA kernel of any alignment: every tile size's edges, K shorter
+# than, equal to and just past a step of 32 and 64 k, one row or column left over, N of one vector and one element more.
+# A, B, C and the epilogue operand start one element into their buffers, and the elements around C stay as they were.
+ANY_SHAPES = [(257, 31, 1025), (1024, 1, 1024), (513, 33, 520), (1030, 64, 8), (1030, 65, 9), (513, 129, 511),
+              (1111, 97, 1001), (1025, 63, 2049), (2100, 32, 2051), (65, 777, 4097)]
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16, F16])
+@pytest.mark.parametrize("shape", ANY_SHAPES)
+def test_gemm_any_alignment(hip, dtype, shape):
+    m, k, n = shape
+    say(f"gemm any alignment dtype={dtype} m={m} k={k} n={n}")
+    a, b = synth.tensor(15, (m, k), dtype, "uniform"), synth.tensor(16, (k, n), dtype, "uniform")
+    bias = synth.tensor(17, (m, n), dtype, "normal")
+    pad, e = np.full(1, 7, a.dtype), a.itemsize
+    da, db, dbias = (dev(hip, np.concatenate([pad, t.ravel()])) for t in (a, b, bias))
+    ep = hip.make_epilogue([(hip.EW_ADD, dbias.value + e), (hip.EW_RELU, None)])
+    # float64 reference rounded to the type: the fp32 sums are within k * 2^-24 of it, far below the rule of 1e-5 / 1e-2
+    want = synth.to_float(a, dtype).astype(np.float64) @ synth.to_float(b, dtype)
+    want = synth.to_storage(want.astype(np.float32), dtype)
+    for segs, exp in [(None, want), (ep, None)]:
+        dc = dev(hip, np.full(m * n + 2, 7, a.dtype))
+        hip.check(hip.lib().fh_gemm(dtype, da.value + e, db.value + e, dc.value + e, m, n, k,
+                                    ctypes.byref(segs) if segs else None, None), "fh_gemm")
+        got = dc.download((m * n + 2,), a.dtype)
+        assert got[0] == 7 and got[-1] == 7, "an element outside C was written"
+        got = got[1:-1].reshape(m, n)
+        if exp is not None:
+            assert_close(got, exp, dtype, what=f"gemm {shape}")
+            plain = got
+        else:  # the fused program equals the separate one on the same product
+            assert_bitwise(got, run_ew(hip, dtype, [1, 3], [2, 1], [plain, bias]), "epilogue vs separate program")
+
+
+def test_gemm_f32_outside_the_split_range(hip):
+    # operands that three bf16 planes do not hold: infinities, NaN, values that round to a bf16 infinity, and values
+    # below 2^-110 (whole rows, so that the result is theirs). Rows without them keep their values next to them
+    m, k, n = 640, 100, 640
+    say("gemm f32: infinities, NaN, FLT_MAX and tiny operands")
+    a, b = synth.tensor(18, (m, k), F32, "uniform"), np.abs(synth.tensor(19, (k, n), F32, "uniform")) + np.float32(0.01)
+    flt_max = np.float32(3.4028234663852886e38)
+    a[3, 5], a[70, 0], a[200, 99] = np.inf, -np.inf, np.nan
+    a[300, :] = 0
+    a[300, 7] = -flt_max
+    a[310, :] *= np.float32(2.0 ** -118)
+    a[639, :] *= np.float32(2.0 ** -125)
+    b[:, 600] = np.float32(2.0 ** -20)
+    a[301, :], a[301, 3] = 0, flt_max  # times b[3, 600] finite, times b[3, j] finite (b < 1.01 may overflow)
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
+    got = run_gemm(hip, F32, a, b)
+    assert np.array_equal(np.isnan(got), np.isnan(want)), "NaN positions"
+    assert np.array_equal(np.isinf(got), np.isinf(want)), "infinities"
+    for r in range(m):
+        ok = np.isfinite(want[r])
+        if ok.any():
+            # fp32 sums of 100 terms: 100 * 2^-24 of the sum of magnitudes, which is at most 100 max|a| max|b|; tiny rows
+            # also lose what fp32 cannot hold below 2^-149
+            mag = np.abs(a[r].astype(np.float64)[np.isfinite(a[r])]).sum() * 1.01
+            err = np.abs(got[r][ok].astype(np.float64) - want[r][ok])
+            assert err.max() <= 100 * 2.0 ** -24 * mag + 100 * 2.0 ** -149, (r, err.max(), mag)
+
+
+@pytest.mark.parametrize("k", [64, 1000, 4096])
+def test_gemm_f32_error_against_float64(hip, k):
+    # the split product is no further from float64 than fp32 products summed in fp32 are: 2^-24 sqrt(k) relative to the
+    # result's norm for sums of random signs (measured 0.2 of it), at ordinary and at very small and large scales
+    for scale in (1.0, 2.0 ** -60, 2.0 ** 60):
+        say(f"gemm f32 error k={k} scale={scale}")
+        a = (synth.tensor(20, (640, k), F32, "uniform") * np.float32(scale)).astype(np.float32)
+        b = (synth.tensor(21, (k, 648), F32, "uniform") * np.float32(scale)).astype(np.float32)
+        want = a.astype(np.float64) @ b.astype(np.float64)
+        got = run_gemm(hip, F32, a, b).astype(np.float64)
+        rel = np.linalg.norm(got - want) / np.linalg.norm(want)
+        assert rel <= 2.0 ** -24 * np.sqrt(k), rel
+
+
 def test_gemm_known_answer(hip):
     # reference: tests/cpp/ops/test_op_matmul.cpp:208-230 — [[1,2],[3,4]]·[[5,6],[7,8]] = [[19,22],[43,50]]
     a = np.array([[1, 2], [3, 4]], np.float32)

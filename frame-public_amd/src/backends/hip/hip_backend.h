@@ -165,6 +165,8 @@ inline void* stream_handle(const ops::KernelContext& ctx) {
 
 // Internal op names produced by HipBackend::compile's lowering (never user-visible).
 inline constexpr std::string_view kGemmEpilogueOp = "hip_matmul_epilogue_internal";
+// kGemmEpilogueOp attribute: 1: operand A is stored transposed, 2: operand B is (fh_gemm_transposed).
+inline constexpr const char* kTransposedAttr = "transposed";
 inline constexpr std::string_view kConvEpilogueOp = "hip_conv2d_epilogue_internal";
 // Up to FH_GEMM_MAX_GROUPS matmuls (each optionally with the same epilogue program) that read one A operand, as one
 // fh_gemm_grouped launch: inputs [A, B_0 .. B_{g-1}, epilogue operands of group 0, of group 1, ...], outputs C_0 ..

@@ -1456,27 +1456,41 @@ class HipExecutable final : public hal::Executable {
 
 }  // namespace
 
-// Whether a matmul_grad node's GEMM is large enough for the tiled kernels: the same threshold as fh_gemm's
-// dispatch on a 256-CU device (fp32 from 64 tiles of 64 x 64, 16-bit from 16). Smaller ones stay
-// matmul_grad_*_internal and run on fh_matmul_grad's sequential kernel, which reads the transposed operand in place.
-bool matmul_grad_wants_gemm(const ir::Node* n) {
+// How a matmul_grad node's GEMM runs.
+enum class MatmulGrad {
+  kNone,       // not a matmul gradient
+  kKeep,       // small: matmul_grad_*_internal on fh_matmul_grad's sequential kernel, in the reference's order
+  kInPlace,    // kGemmEpilogueOp with kTransposedAttr: the transposed operand read as it is stored
+  kTranspose,  // a transpose of that operand, then a plain matmul
+};
+
+// The tiled kernels take a gradient from the same size on as fh_gemm's dispatch on a 256-CU device does (fp32 from 64
+// tiles of 64 x 64, 16-bit from 16); at opt_level >= 1, where the k order is free, smaller ones with k >= 128 as well (the
+// sequential kernel spends 35 ns per k). Of these, large 16-bit ones of whole vectors are transposed: the aligned pipeline
+// makes up for the copy above about 2^30 multiplications (1024^3: 11.5 us in place, 7 + 4.5 us with the copy).
+MatmulGrad plan_matmul_grad(const ir::Node* n, int32_t opt_level) {
   const bool lhs = n->op() == "matmul_grad_lhs_internal";
-  if (!lhs && n->op() != "matmul_grad_rhs_internal") return false;
+  if (!lhs && n->op() != "matmul_grad_rhs_internal") return MatmulGrad::kNone;
   const Shape& p = n->inputs()[0]->type().shape;
   const Shape& q = n->inputs()[1]->type().shape;
   const int64_t M = lhs ? p.dim(0) : p.dim(1), N = lhs ? q.dim(0) : q.dim(1), K = lhs ? p.dim(1) : p.dim(0);
   const int64_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
   const bool f32 = n->inputs()[0]->type().dtype.code() == DTypeCode::kFloat32;
-  return (f32 ? tiles64 >= 64 : tiles64 >= 16) || K > 16384;
+  const bool tiled = (f32 ? tiles64 >= 64 : tiles64 >= 16) || K > 16384;
+  if (!tiled && !(opt_level >= 1 && K >= 128 && M >= 8 && N >= 8)) return MatmulGrad::kKeep;
+  const bool vectors = K % 32 == 0 && N % 8 == 0 && N >= 64;
+  const double work = static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(K);
+  if (!f32 && vectors && tiled && work > static_cast<double>(int64_t{1} << 30)) return MatmulGrad::kTranspose;
+  return MatmulGrad::kInPlace;
 }
 
-// matmul_grad_lhs_internal(gy, b) = gy * b^T and matmul_grad_rhs_internal(a, gy) = a^T * gy, when large, become a
-// transpose of the transposed operand plus a plain matmul, so they run on the tiled GEMM kernels with the same
-// products and fp32 accumulation as the reference (src/backends/cpu/kernels/matmul.cpp:187-327). Returns a clone
-// of the source when no node qualifies.
-Result<ir::Graph> lower_matmul_grads(const ir::Graph& src) {
+// matmul_grad_lhs_internal(gy, b) = gy * b^T and matmul_grad_rhs_internal(a, gy) = a^T * gy on the MFMA GEMM kernels where
+// plan_matmul_grad says so: the same products and fp32 accumulation as the reference
+// (src/backends/cpu/kernels/matmul.cpp:187-327). Returns a clone of the source when no node qualifies.
+Result<ir::Graph> lower_matmul_grads(const ir::Graph& src, int32_t opt_level) {
   const auto& order = src.topological_order();
-  const bool any = std::any_of(order.begin(), order.end(), matmul_grad_wants_gemm);
+  const bool any = std::any_of(order.begin(), order.end(),
+                               [&](const ir::Node* n) { return plan_matmul_grad(n, opt_level) >= MatmulGrad::kInPlace; });
   if (!any) return ir::clone_graph(src);
   std::unordered_map<const ir::Value*, ir::Value*> map;
   ir::Graph out{std::string(src.name())};
@@ -1489,7 +1503,19 @@ Result<ir::Graph> lower_matmul_grads(const ir::Graph& src) {
     }
     std::vector<ir::Value*> ins;
     for (const ir::Value* in : n->inputs()) ins.push_back(map.at(in));
-    if (matmul_grad_wants_gemm(n)) {
+    const MatmulGrad how = plan_matmul_grad(n, opt_level);
+    if (how == MatmulGrad::kInPlace) {
+      Result<ir::Node*> mm = out.create_node(std::string(kGemmEpilogueOp), std::move(ins), {n->outputs()[0].type()});
+      if (!mm.is_ok()) return mm.status();
+      const bool lhs = n->op() == "matmul_grad_lhs_internal";
+      mm.value()->set_attr(kTransposedAttr, ir::AttrValue{int64_t{lhs ? 2 : 1}});
+      mm.value()->set_attr("any_order", ir::AttrValue{int64_t{opt_level >= 1 ? 1 : 0}});
+      mm.value()->set_attr("ep_ops", ir::AttrValue{std::vector<int64_t>{}});
+      mm.value()->set_attr("n_main_inputs", ir::AttrValue{int64_t{2}});
+      map[&n->outputs()[0]] = mm.value()->output(0);
+      continue;
+    }
+    if (how == MatmulGrad::kTranspose) {
       const bool lhs = n->op() == "matmul_grad_lhs_internal";
       ir::Value* t_in = lhs ? ins[1] : ins[0];  // b of gy*b^T, a of a^T*gy
       ir::TensorType tt = t_in->type();
@@ -1611,6 +1637,7 @@ Status lower_gemm_softmax(ir::Graph& g) {
     const auto* any = attr_of<int64_t>(p, "any_order");
     const auto* n_main = attr_of<int64_t>(p, "n_main_inputs");
     if (any == nullptr || *any == 0 || n_main == nullptr || *n_main != 2) continue;
+    if (attr_of<int64_t>(p, kTransposedAttr) != nullptr) continue;
     const ir::TensorType& ot = p->outputs()[0].type();
     if (ot.shape.rank() != 2 || ot.shape.dim(1) > 16 || ot.shape.dim(0) > 262140) continue;
     const ir::TensorType& st = sm->outputs()[0].type();
@@ -1645,7 +1672,9 @@ Status lower_grouped_gemms(ir::Graph& g) {
     const bool mm = n->op() == "matmul" && n->inputs().size() == 2;
     const auto* n_main = attr_of<int64_t>(n, "n_main_inputs");
     const bool epi = n->op() == kGemmEpilogueOp && n_main != nullptr && *n_main == 2;
-    if ((!mm && !epi) || n->outputs().size() != 1 || attr_of<int64_t>(n, "row_softmax") != nullptr) continue;
+    if ((!mm && !epi) || n->outputs().size() != 1 || attr_of<int64_t>(n, "row_softmax") != nullptr ||
+        attr_of<int64_t>(n, kTransposedAttr) != nullptr)
+      continue;
     const ir::TensorType& ot = n->outputs()[0].type();
     if (ot.dtype.code() != DTypeCode::kBFloat16 && ot.dtype.code() != DTypeCode::kFloat16) continue;
     const ir::TensorType& bt = n->inputs()[1]->type();
@@ -1691,7 +1720,7 @@ Status lower_grouped_gemms(ir::Graph& g) {
 }
 
 Result<ir::Graph> lower_for_hip(const ir::Graph& graph, int32_t opt_level) {
-  Result<ir::Graph> work = lower_matmul_grads(graph);
+  Result<ir::Graph> work = lower_matmul_grads(graph, opt_level);
   if (!work.is_ok()) return work.status();
   // Attention runs at every level (like the conv lowering), before the epilogue fusion would claim its matmuls.
   FRAME_RETURN_IF_ERROR(lower_attention(work.value()));

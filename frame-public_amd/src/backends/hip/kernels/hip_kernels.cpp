@@ -164,8 +164,12 @@ Status gemm_impl(KernelContext& ctx, const std::string& op, size_t n_main) {
   const Tensor& b = ctx.inputs[1];
   Tensor& c = ctx.outputs[0];
   if (a.shape().rank() != 2 || b.shape().rank() != 2 || c.shape().rank() != 2) return invalid(op, "operands must be rank-2");
-  const int64_t m = a.shape().dim(0), k = a.shape().dim(1), n = b.shape().dim(1);
-  if (b.shape().dim(0) != k || c.shape().dim(0) != m || c.shape().dim(1) != n)
+  // kTransposedAttr: 1: A is stored [k, m], 2: B is stored [n, k] (lowered matmul gradients)
+  const auto* stored = attr<int64_t>(ctx, kTransposedAttr);
+  const int32_t transposed = stored != nullptr ? static_cast<int32_t>(*stored) : 0;
+  const int64_t m = a.shape().dim(transposed == 1 ? 1 : 0), k = a.shape().dim(transposed == 1 ? 0 : 1);
+  const int64_t n = b.shape().dim(transposed == 2 ? 0 : 1);
+  if (b.shape().dim(transposed == 2 ? 1 : 0) != k || c.shape().dim(0) != m || c.shape().dim(1) != n)
     return invalid(op, "shape mismatch " + a.shape().to_string() + " x " + b.shape().to_string() + " -> " + c.shape().to_string());
   FRAME_RETURN_IF_ERROR(same_dtype(ctx, op));
   Result<int32_t> dt = float_code(op, c.dtype());
@@ -176,9 +180,13 @@ Status gemm_impl(KernelContext& ctx, const std::string& op, size_t n_main) {
   const auto* row_softmax = attr<int64_t>(ctx, "row_softmax");
   const int32_t flags = ((any != nullptr && *any != 0) ? FH_GEMM_ANY_ORDER : 0) |
                         ((row_softmax != nullptr && *row_softmax != 0) ? FH_GEMM_ROW_SOFTMAX : 0);
-  FRAME_HIP_RETURN_IF_ERROR(fh_gemm_ex(dt.value(), a.raw_data(), b.raw_data(), c.raw_data(), m, n, k,
-                                       ep.value().nseg > 0 ? &ep.value() : nullptr, flags, stream_handle(ctx)),
-                            "op '" + op + "' (hip)");
+  const fh_epilogue* program = ep.value().nseg > 0 ? &ep.value() : nullptr;
+  FRAME_HIP_RETURN_IF_ERROR(
+      transposed == 0
+          ? fh_gemm_ex(dt.value(), a.raw_data(), b.raw_data(), c.raw_data(), m, n, k, program, flags, stream_handle(ctx))
+          : fh_gemm_transposed(dt.value(), transposed, a.raw_data(), b.raw_data(), c.raw_data(), m, n, k, program, flags,
+                               stream_handle(ctx)),
+      "op '" + op + "' (hip)");
   return Status::ok();
 }
 

@@ -145,6 +145,13 @@ fh_status fh_gemm(int32_t dtype, const void* A, const void* B, void* C, int64_t 
 fh_status fh_gemm_ex(int32_t dtype, const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K,
                      const fh_epilogue* epilogue, int32_t flags, void* stream);
 
+/* fh_gemm_ex with transposed operand storage: transposed = 1: A is stored [K,M] (A(m, k) = A[k * M + m]);
+ * transposed = 2: B is stored [N,K] (B(k, n) = B[n * K + k]). Neither is copied: the kernels read the stored layout. The
+ * gradients of matmul (reference: src/backends/cpu/kernels/matmul.cpp:187-327) with the epilogue HipBackend::compile
+ * fuses into them. */
+fh_status fh_gemm_transposed(int32_t dtype, int32_t transposed, const void* A, const void* B, void* C, int64_t M,
+                             int64_t N, int64_t K, const fh_epilogue* epilogue, int32_t flags, void* stream);
+
 /* `groups` GEMMs sharing A[M,K] and one shape, in one launch: C_g[M,N] = A · B_g[K,N], then epilogues[g]
  * (every group the same program, its own operands). Used where HipBackend::compile merges the Q/K/V
  * projections of an attention block, which read the same normalised input (the reference runs three

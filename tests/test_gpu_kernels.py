@@ -131,6 +131,34 @@ def test_gemm_any_alignment(hip, dtype, shape):
             assert_bitwise(got, run_ew(hip, dtype, [1, 3], [2, 1], [plain, bias]), "epilogue vs separate program")
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16, F16])
+@pytest.mark.parametrize("transposed", [1, 2])
+def test_gemm_transposed_operand(hip, dtype, transposed):
+    # A stored [K,M] or B stored [N,K], read in place: tile edges, ragged K, widths of one vector and one element more, and
+    # the small sizes of the any-order rule (K >= 128), with an epilogue; the sequential kernel below it
+    for m, k, n in [(257, 33, 1025), (1030, 65, 9), (513, 129, 511), (1024, 512, 768), (64, 1000, 512), (8, 128, 8),
+                    (10, 200, 300), (64, 64, 10)]:
+        say(f"gemm transposed={transposed} dtype={dtype} m={m} k={k} n={n}")
+        a, b = synth.tensor(22, (m, k), dtype, "uniform"), synth.tensor(23, (k, n), dtype, "uniform")
+        bias = synth.tensor(24, (m, n), dtype, "normal")
+        want = synth.to_float(a, dtype).astype(np.float64) @ synth.to_float(b, dtype)
+        want = synth.to_storage(want.astype(np.float32), dtype)
+        da, db = dev(hip, a.T if transposed == 1 else a), dev(hip, b.T if transposed == 2 else b)
+        dbias = dev(hip, bias)
+        ep = hip.make_epilogue([(hip.EW_ADD, dbias.value)])
+        dc = hip.DeviceBuffer(m * n * a.itemsize)
+        for program in (None, ctypes.byref(ep)):
+            hip.check(hip.lib().fh_gemm_transposed(dtype, transposed, da.value, db.value, dc.value, m, n, k, program, 1, None))
+            got = dc.download((m, n), a.dtype)
+            if program is None:
+                assert_close(got, want, dtype, what=f"transposed {(m, k, n)}")
+                plain = got
+            else:
+                assert_bitwise(got, run_ew(hip, dtype, [1], [2], [plain, bias]), "epilogue")
+    for bad in (0, 3):
+        assert hip.lib().fh_gemm_transposed(dtype, bad, da.value, db.value, dc.value, m, n, k, None, 1, None) == 1
+
+
 def test_gemm_f32_outside_the_split_range(hip):
     # operands that three bf16 planes do not hold: infinities, NaN, values that round to a bf16 infinity, and values
     # below 2^-110 (whole rows, so that the result is theirs). Rows without them keep their values next to them

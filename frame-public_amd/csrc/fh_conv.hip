@@ -1,14 +1,15 @@
 // Conv2d forward, NCHW (reference semantics: src/backends/cpu/kernels/conv.cpp:223-314).
 //
 // conv2d_direct_kernel: one thread per output element, products summed over (ci, kh, kw) in the reference's
-// order, bias added last inside the fp32 accumulator, one rounding. It serves every geometry (groups,
-// strides, padding, odd channel counts, fp32) on NCHW operands. The MFMA implicit-GEMM path over
-// channels-last operands is fh_conv2d_nhwc_fwd (fh_conv_igemm.hip), selected at graph compile time.
+// order, bias added last inside the fp32 accumulator, one rounding. It serves grouped convolutions and sizes past the
+// MFMA kernel's 32-bit offsets; every other geometry runs on the implicit GEMM over NCHW operands (fh_conv_any.hip). The
+// kernels over channels-last operands are fh_conv2d_nhwc_fwd's (fh_conv_igemm.hip), selected at graph compile time.
 #include <hip/hip_runtime.h>
 
 #include <string>
 
 #include "fh_common.h"
+#include "fh_conv_any.h"
 #include "fh_conv_direct.h"
 
 namespace fh {
@@ -64,12 +65,6 @@ fh_status launch_direct(const void* x, const void* w, const void* bias, void* y,
   return launch_status("conv2d_direct_kernel launch");
 }
 
-template <typename T>
-fh_status conv_typed(const void* x, const void* w, const void* bias, void* y, const ConvGeom& g,
-                     const ConvEpilogue& ep, hipStream_t s) {
-  return launch_direct<T>(x, w, bias, y, g, ep, s);
-}
-
 }  // namespace
 }  // namespace fh
 
@@ -119,12 +114,14 @@ extern "C" fh_status fh_conv2d_fwd(int32_t dtype, const void* x, const void* w, 
   if (g.n * g.cout * g.oh * g.ow == 0) return FH_OK;
   if (x == nullptr || w == nullptr || y == nullptr) return fail(FH_INVALID_ARGUMENT, "fh_conv2d_fwd: null pointer");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  fh_status st = FH_OK;
+  if (conv_any_try_launch(dtype, x, w, bias, y, g, ep, s, &st)) return st;
   switch (dtype) {
     case FH_F32:
-      return conv_typed<float>(x, w, bias, y, g, ep, s);
+      return launch_direct<float>(x, w, bias, y, g, ep, s);
     case FH_BF16:
-      return conv_typed<bf16_t>(x, w, bias, y, g, ep, s);
+      return launch_direct<bf16_t>(x, w, bias, y, g, ep, s);
     default:
-      return conv_typed<f16_t>(x, w, bias, y, g, ep, s);
+      return launch_direct<f16_t>(x, w, bias, y, g, ep, s);
   }
 }

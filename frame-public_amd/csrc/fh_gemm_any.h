@@ -199,12 +199,107 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-template <typename T, int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool TA, bool TB, int E>
-__global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_any_kernel(GemmArgs args) {
-  using S = typename Io<T>::storage;
-  using M16 = typename AnyTraits<T>::mfma_t;
+// The k loop of one tile: KT steps of BK. whole_load<SET>(kt) issues the loads of tile kt < whole into register set SET,
+// any_load<SET>(kt) those of any tile (nothing from KT on). Step kt: loads of kt + 2 into the set that tile kt left,
+// products of kt, LDS writes of kt + 1, barrier. The main loop has no branch: where a path might have left a load of the
+// same registers in flight, the compiler waits for every load before issuing the next (4095^3 bf16: 278 us against 180).
+// (Spreading the LDS writes between the products in fixed order was slower for fp32: 98 us against 94 at 2048^3.)
+template <typename T, typename OpA, typename OpB, int BK, int TM, int TN, typename Whole, typename Any>
+__device__ __forceinline__ void k_loop(OpA& a, OpB& b, unsigned char* lds, int KT, int whole, int m_off, int n_off,
+                                       int lane, Whole&& whole_load, Any&& any_load, uint32_t& tiny,
+                                       f32x4_t (&acc)[TM][TN]) {
   constexpr bool F32 = std::is_same_v<T, float>;
   constexpr int P = AnyTraits<T>::P;
+  constexpr int BUF = OpA::BYTES + OpB::BYTES;
+  using M16 = typename AnyTraits<T>::mfma_t;
+  auto store = [&]<int SET>(unsigned char* buf) {
+    a.template store<SET>(buf, tiny);
+    b.template store<SET>(buf + OpA::BYTES, tiny);
+  };
+  auto products = [&](const unsigned char* buf) {
+#pragma unroll
+    for (int s = 0; s < BK / 32; ++s) {
+      u32x4_t fa[P][TM], fb[P][TN];
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+          fa[p][i] = OpA::fragment(buf + p * OpA::PLANE + s * OpA::SUB, m_off + i * 16, lane);
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          fb[p][j] = OpB::fragment(buf + OpA::BYTES + p * OpB::PLANE + s * OpB::SUB, n_off + j * 16, lane);
+      }
+      auto pair = [&]<int PA, int PB>() {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) mfma16x<M16>(fa[PA][i], fb[PB][j], acc[i][j]);
+      };
+      if constexpr (F32) {  // small terms first: a short sum then rounds once at its full size
+        pair.template operator()<2, 0>();
+        pair.template operator()<0, 2>();
+        pair.template operator()<1, 1>();
+        pair.template operator()<1, 0>();
+        pair.template operator()<0, 1>();
+      }
+      pair.template operator()<0, 0>();
+    }
+  };
+  auto whole_step = [&]<int SET>(int kt) {
+    whole_load.template operator()<SET>(kt + 2);
+    products(lds + SET * BUF);
+    store.template operator()<1 - SET>(lds + (1 - SET) * BUF);
+    lds_barrier();
+  };
+  auto any_step = [&]<int SET>(int kt) {
+    any_load.template operator()<SET>(kt + 2);
+    products(lds + SET * BUF);
+    if (kt + 1 < KT) store.template operator()<1 - SET>(lds + (1 - SET) * BUF);
+    lds_barrier();
+  };
+  if (KT <= 0) return;
+  any_load.template operator()<0>(0);
+  any_load.template operator()<1>(1);
+  store.template operator()<0>(lds);
+  lds_barrier();
+  int kt = 0;
+  for (; kt + 3 < whole; kt += 2) {
+    whole_step.template operator()<0>(kt);
+    whole_step.template operator()<1>(kt + 1);
+  }
+  for (; kt < KT; kt += 2) {
+    any_step.template operator()<0>(kt);
+    if (kt + 1 < KT) any_step.template operator()<1>(kt + 1);
+  }
+}
+
+// Whether this wave's fp32 tile has to be taken again on fp32 operands: an operand below the split's range, or a result
+// that is not finite.
+template <int TM, int TN>
+__device__ __forceinline__ bool outside_split(int* tiny_seen, uint32_t tiny, const f32x4_t (&acc)[TM][TN]) {
+  if (tiny < kTinyKey) *tiny_seen = 1;
+  __syncthreads();
+  bool bad = *tiny_seen != 0;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) bad |= !(__builtin_fabsf(acc[i][j][x]) <= 3.4028234663852886e38f);
+  return __any(bad);
+}
+
+// Waves per SIMD a kernel is compiled for: two workgroups of eight waves share a CU's 16-bit LDS buffers, which 128
+// registers per lane allow and 130 (the compiler's own choice at 128x128x64) do not: 4095^3 bf16 181 us against 206.
+template <typename T, int WAVES>
+constexpr int min_waves() {
+  return std::is_same_v<T, float> || WAVES < 8 ? 1 : 4;
+}
+
+template <typename T, int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool TA, bool TB, int E>
+__global__ __launch_bounds__(WAVES_M* WAVES_N * 64, (min_waves<T, WAVES_M * WAVES_N>())) void gemm_any_kernel(GemmArgs args) {
+  using S = typename Io<T>::storage;
+  constexpr bool F32 = std::is_same_v<T, float>;
   constexpr int NT = WAVES_M * WAVES_N * 64;
   constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
   constexpr int TM = WM / 16, TN = WN / 16;
@@ -246,86 +341,29 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_any_kernel(GemmArg
   uint32_t tiny = ~0u;
   if (F32 && tid == 0) tiny_seen = 0;
 
-  auto load = [&]<int SET>(int kt) {
+  auto whole_load = [&]<int SET>(int kt) {
+    a.template load<SET>(kt);
+    b.template load<SET>(kt);
+  };
+  auto any_load = [&]<int SET>(int kt) {
     if (kt < whole) {
-      a.template load<SET>(kt);
-      b.template load<SET>(kt);
+      whole_load.template operator()<SET>(kt);
     } else if (kt < KT) {
       a.template load_tail<SET>(kt, K - static_cast<int64_t>(kt) * BK);
       b.template load_tail<SET>(kt, K - static_cast<int64_t>(kt) * BK);
     }
   };
-  auto store = [&]<int SET>(unsigned char* buf) {
-    a.template store<SET>(buf, tiny);
-    b.template store<SET>(buf + OpA::BYTES, tiny);
-  };
-
   f32x4_t acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-  auto products = [&](const unsigned char* buf) {
-#pragma unroll
-    for (int s = 0; s < BK / 32; ++s) {
-      u32x4_t fa[P][TM], fb[P][TN];
-#pragma unroll
-      for (int p = 0; p < P; ++p) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-          fa[p][i] = OpA::fragment(buf + p * OpA::PLANE + s * OpA::SUB, wm * WM + i * 16, lane);
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          fb[p][j] = OpB::fragment(buf + OpA::BYTES + p * OpB::PLANE + s * OpB::SUB, wn * WN + j * 16, lane);
-      }
-      auto pair = [&]<int PA, int PB>() {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) mfma16x<M16>(fa[PA][i], fb[PB][j], acc[i][j]);
-      };
-      pair.template operator()<0, 0>();
-      if constexpr (F32) {
-        pair.template operator()<0, 1>();
-        pair.template operator()<1, 0>();
-        pair.template operator()<1, 1>();
-        pair.template operator()<0, 2>();
-        pair.template operator()<2, 0>();
-      }
-    }
-  };
-
-  // step kt: loads of kt + 2 into the set that tile kt left, products of kt, LDS writes of kt + 1, barrier
-  auto step = [&]<int SET>(int kt) {
-    load.template operator()<SET>(kt + 2);
-    products(lds + SET * BUF);
-    if (kt + 1 < KT) store.template operator()<1 - SET>(lds + (1 - SET) * BUF);
-    lds_barrier();
-  };
-  if (KT > 0) {
-    load.template operator()<0>(0);
-    load.template operator()<1>(1);
-    store.template operator()<0>(lds);
-    lds_barrier();
-    for (int kt = 0; kt < KT; kt += 2) {
-      step.template operator()<0>(kt);
-      if (kt + 1 < KT) step.template operator()<1>(kt + 1);
-    }
-  }
+  k_loop<T, OpA, OpB, BK>(a, b, lds, KT, whole, wm * WM, wn * WN, lane, whole_load, any_load, tiny, acc);
 
   const int g = lane >> 4, r = lane & 15;
   if constexpr (F32) {
-    if (tiny < kTinyKey) tiny_seen = 1;
-    __syncthreads();
-    bool bad = tiny_seen != 0;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int x = 0; x < 4; ++x) bad |= !(__builtin_fabsf(acc[i][j][x]) <= 3.4028234663852886e38f);
-    if (__any(bad)) {
+    if (outside_split(&tiny_seen, tiny, acc)) {
       // outside the split's range: this wave's tile again, on fp32 operands from memory
 #pragma unroll
       for (int i = 0; i < TM; ++i)

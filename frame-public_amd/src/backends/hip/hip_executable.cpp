@@ -458,6 +458,23 @@ std::optional<std::vector<int64_t>> nhwc_sum_axes(const ir::Node* n) {
   return out;
 }
 
+// Whether an fp32 conv of a forward graph runs on the NCHW implicit GEMM: with output rows of whole vectors; gathering
+// single pixels for a stride along the row only on enough tiles to hide it. Output rows under 8 stay channels-last
+// ([64,256,7,7] x [256,256,3,3]: 72 us there, 76 gathered; [8,64,7,7] x [256,64,5,5] 49 and 55).
+bool f32_conv_nchw(const int64_t geom[12]) {
+  const int64_t oh = (geom[2] + 2 * geom[9] - geom[5]) / geom[7] + 1;
+  const int64_t ow = (geom[3] + 2 * geom[10] - geom[6]) / geom[8] + 1;
+  const int64_t tiles64 = ((geom[0] * oh * ow + 63) / 64) * ((geom[4] + 63) / 64);
+  return ow >= 8 && (geom[8] == 1 || tiles64 >= 128);
+}
+
+// Whether a graph computes no gradients.
+bool is_forward(const ir::Graph& g) {
+  for (const ir::Node* n : g.topological_order())
+    if (n->op().find("grad") != std::string::npos) return false;
+  return true;
+}
+
 // A conv the band kernel takes when its activation, output and residual operand are NCHW and its filter stays in
 // the graph's [Cout][Cin][KH][KW] layout (fh_conv2d_w_oihw_supported on its geometry and epilogue program).
 bool band_conv(const ir::Node* n, const ConvLowering& p) {
@@ -566,14 +583,12 @@ std::unordered_set<const ir::Value*> plan_channels_last(const ir::Graph& src) {
     }
     if (!producer_ok || !uses_ok || !rank4(v)) bad.insert(root);
   }
+  // fp32 convs of forward graphs stay NCHW throughout (see f32_nchw in lower_convs).
   // Forward graphs: a group that a band conv produces stays NCHW when every conv producing into it is a band conv
   // or a C8 stem conv (both write NCHW), so the band kernel (NCHW in and out, the filter read as it is) runs it:
   // ResNet's 56x56 layer, whose channels-last convs took 32-37 us each, against 24-26 us on the band kernel. Its
   // pool runs the NCHW kernel; a non-band conv reading such a value gets one channels-last copy of it.
-  bool forward = true;
-  for (const ir::Node* n : src.topological_order())
-    if (n->op().find("grad") != std::string::npos) forward = false;
-  if (forward) {
+  if (is_forward(src)) {
     std::unordered_map<const ir::Value*, std::pair<bool, bool>> group;  // root -> (band producer, other conv producer)
     for (const auto& [v, unused] : parent) {
       (void)unused;
@@ -581,7 +596,7 @@ std::unordered_set<const ir::Value*> plan_channels_last(const ir::Graph& src) {
       auto it = p != nullptr ? convs.find(p) : convs.end();
       if (it == convs.end()) continue;
       auto& g = group[find(v)];
-      if (band_conv(p, it->second)) g.first = true;
+      if (band_conv(p, it->second) || (conv_dtype_code(v->type()) == FH_F32 && f32_conv_nchw(it->second.geom))) g.first = true;
       else if (!it->second.c8) g.second = true;
     }
     for (const auto& [root, g] : group)
@@ -667,11 +682,20 @@ Result<ir::Graph> lower_convs(const ir::Graph& src) {
 
   // Whether a lowered conv reads its NCHW activation (FH_CONV_IN_NCHW) and, writing NCHW, takes its filter in the
   // graph's own [Cout][Cin][KH][KW] layout too (FH_CONV_W_OIHW, the band kernel): then neither operand is copied.
+  // fp32 convs of forward graphs read both operands as they are too and write NCHW, on fh_conv2d_fwd's implicit GEMM over
+  // split operands ([32,64,56,56] x [64,64,3,3]: 67 us, against 102 channels-last with its two transposes).
+  const bool forward = is_forward(src);
+  auto f32_nchw = [&](const ir::Node* n, const ConvLowering& p) {
+    return p.ok && forward && conv_dtype_code(n->inputs()[0]->type()) == FH_F32 && f32_conv_nchw(p.geom) &&
+           !nhwc.count(n->inputs()[0]) && !nhwc.count(&n->outputs()[0]);
+  };
   auto reads_nchw = [&](const ir::Node* n, const ConvLowering& p) {
+    if (f32_nchw(n, p)) return true;
     return p.ok && !p.c8 && !nhwc.count(n->inputs()[0]) &&
            fh_conv2d_nchw_in_supported(conv_dtype_code(n->inputs()[0]->type()), p.geom) != 0;
   };
   auto takes_oihw = [&](const ir::Node* n, const ConvLowering& p) {
+    if (f32_nchw(n, p)) return true;
     if (!reads_nchw(n, p) || nhwc.count(&n->outputs()[0])) return false;
     fh_epilogue qe{};
     if (const auto* prog = attr_of<std::vector<int64_t>>(n, "ep_ops")) {

@@ -268,7 +268,8 @@ Result<bool> conv_via_channels_last(const KernelContext& ctx, const std::string&
                                     const Tensor* bias, const fh_epilogue& ep) {
   const Tensor& x = ctx.inputs[0];
   const Tensor& w = ctx.inputs[1];
-  const bool c8 = dt != FH_F32 && geom[1] <= 8 && geom[11] == 1;
+  if (dt == FH_F32) return false;  // fh_conv2d_fwd's implicit GEMM needs no copies
+  const bool c8 = geom[1] <= 8 && geom[11] == 1;
   int64_t g[12];
   std::copy(geom, geom + 12, g);
   if (c8) g[1] = 8;
@@ -407,6 +408,13 @@ Status conv_nhwc_kernel(KernelContext& ctx) {
                                                        y.raw_data(), geom, ep.value().nseg > 0 ? &ep.value() : nullptr,
                                                        FH_CONV_OUT_NHWC, 0, ws.raw_data(),
                                                        ws.numel() * static_cast<int64_t>(sizeof(float)), stream_handle(ctx)),
+                              "op '" + op + "' (hip)");
+    return Status::ok();
+  }
+  if (dt.value() == FH_F32 && in_nchw && w_oihw && !out_nhwc) {  // fp32 on operands as they are: the NCHW implicit GEMM
+    FRAME_HIP_RETURN_IF_ERROR(fh_conv2d_fwd(dt.value(), x.raw_data(), w.raw_data(), bias ? bias->raw_data() : nullptr,
+                                            y.raw_data(), geom, ep.value().nseg > 0 ? &ep.value() : nullptr,
+                                            stream_handle(ctx)),
                               "op '" + op + "' (hip)");
     return Status::ok();
   }

@@ -689,6 +689,74 @@ def test_conv2d(hip, dtype, geom, with_bias):
     assert_close(got, want, dtype, what=f"conv {geom}")
 
 
+# The implicit GEMM over NCHW operands: output rows of whole vectors, rows that a vector runs over, gathers (stride along the
+# row, rows shorter than 8), padding wider than a row's start, one pixel, K below / at / past a step, channels past a tile,
+# pixels past a tile and vectors over an image's end.
+CONV_ANY_CASES = [
+    # N, Cin, H, W, Cout, KH, KW, sh, sw, ph, pw, groups
+    (2, 5, 16, 24, 65, 3, 3, 1, 1, 1, 1, 1),
+    (3, 5, 17, 23, 70, 3, 5, 1, 1, 2, 1, 1),
+    (1, 7, 9, 30, 64, 2, 4, 3, 1, 0, 3, 1),
+    (2, 16, 15, 15, 130, 1, 1, 2, 2, 0, 0, 1),
+    (5, 64, 7, 7, 33, 3, 3, 1, 1, 1, 1, 1),
+    (2, 3, 31, 18, 8, 7, 7, 2, 2, 3, 3, 1),
+    (1, 1, 1, 1, 1, 1, 1, 1, 1, 0, 0, 1),
+    (1, 32, 5, 8, 16, 1, 1, 1, 1, 0, 0, 1),
+    (4, 11, 8, 9, 100, 3, 3, 1, 1, 1, 1, 1),
+]
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16, F16])
+@pytest.mark.parametrize("geom", CONV_ANY_CASES)
+def test_conv2d_any_geometry(hip, dtype, geom):
+    say(f"conv any geometry dtype={dtype} {geom}")
+    n, cin, h, w, cout, kh, kw = geom[:7]
+    x = synth.tensor(104, (n, cin, h, w), dtype, "normal")
+    wt = synth.tensor(105, (cout, cin, kh, kw), dtype, "normal", (2.0 / (cin * kh * kw)) ** 0.5)
+    bias = synth.tensor(106, (cout,), dtype, "normal", 0.1)
+    want = orc.conv2d(dtype, x, wt, bias, geom)
+    res = synth.tensor(107, want.shape, dtype, "normal")
+    pad, e = np.full(1, 7, x.dtype), x.itemsize  # every pointer one element into its buffer
+    dx, dw, db, dres = (dev(hip, np.concatenate([pad, t.ravel()])) for t in (x, wt, bias, res))
+    programs = [([], None), ([(hip.EW_RELU, None)], ([3], [1], [])),
+                ([(hip.EW_ADD, dres.value + e), (hip.EW_RELU, None)], ([1, 3], [2, 1], [res]))]
+    for segs, check in programs:
+        dy = dev(hip, np.full(want.size + 2, 7, x.dtype))
+        ep = hip.make_epilogue(segs)
+        hip.check(hip.lib().fh_conv2d_fwd(dtype, dx.value + e, dw.value + e, db.value + e, dy.value + e,
+                                          hip.i64_array(geom), ctypes.byref(ep) if segs else None, None))
+        got = dy.download((want.size + 2,), x.dtype)
+        assert got[0] == 7 and got[-1] == 7, "an element outside y was written"
+        got = got[1:-1].reshape(want.shape)
+        if check is None:
+            assert_close(got, want, dtype, what=f"conv {geom}")
+            plain = got
+        else:
+            ops, arities, ins = check
+            assert_bitwise(got, run_ew(hip, dtype, ops, arities, [plain] + ins), "epilogue vs separate program")
+
+
+def test_conv2d_f32_outside_the_split_range(hip):
+    # an image with an infinity, one with NaN, one of values below 2^-110 and one whose largest value rounds to a bf16
+    # infinity: their results are the oracle's, the other images' are untouched
+    geom = (6, 8, 12, 12, 16, 3, 3, 1, 1, 1, 1, 1)
+    say(f"conv f32 outside the split range {geom}")
+    x = synth.tensor(108, geom[:4], F32, "normal")
+    wt = np.abs(synth.tensor(109, (16, 8, 3, 3), F32, "normal", 0.1)) + np.float32(0.01)
+    x[1, 3, 5, 5], x[2, 0, 0, 0] = np.inf, np.nan
+    x[3] *= np.float32(2.0 ** -118)
+    x[4] = 0
+    x[4, 2, 6, 6] = -3.4028234663852886e38
+    want = orc.conv2d(F32, x, wt, None, geom)
+    dx, dw, dy = dev(hip, x), dev(hip, wt), hip.DeviceBuffer(want.nbytes)
+    hip.check(hip.lib().fh_conv2d_fwd(F32, dx.value, dw.value, None, dy.value, hip.i64_array(geom), None, None))
+    got = dy.download(want.shape, want.dtype)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    for i in range(6):
+        ok = np.isfinite(want[i])
+        assert_close(got[i][ok], want[i][ok], F32, what=f"image {i}")
+
+
 # paths: whole planes through LDS (rows * cols <= 8192: filters), 16-byte tiles (16-bit, rows and cols multiples
 # of 8; full and partial tiles), element tiles (everything else, e.g. thin late-stage activations)
 @pytest.mark.parametrize("itemsize,shape", [(2, (3, 64, 3136)), (2, (2, 72, 200)), (2, (5, 70, 9)), (4, (2, 33, 130)),

@@ -24,6 +24,9 @@ struct GemmArgs {
   int64_t M, N, K;
   int64_t lda, ldb, ldc;                 // row strides in elements
   int64_t stride_a, stride_b, stride_c;  // batch strides in elements (blockIdx.y)
+  // inner > 1 (kernel of any alignment only): blockIdx.y = outer * inner + i, the batch strides are the outer ones and
+  // these the strides of i (the heads of an attention inside its rows).
+  int64_t inner, inner_a, inner_b, inner_c;
   int32_t tiles_m, tiles_n;
   EpilogueArgs ep;
   // Transposed operand storage, honoured by the sequential kernel and the kernel of any alignment:

@@ -326,9 +326,11 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64, (min_waves<T, WAVES_M * WAVE
   const int64_t m0 = static_cast<int64_t>(group * GROUP_M + in_group % gsize) * BM;
   const int64_t n0 = static_cast<int64_t>(in_group / gsize) * BN;
 
-  const S* __restrict__ A = static_cast<const S*>(args.A) + blockIdx.y * args.stride_a;
-  const S* __restrict__ B = static_cast<const S*>(args.B) + blockIdx.y * args.stride_b;
-  S* __restrict__ C = static_cast<S*>(args.C) + blockIdx.y * args.stride_c;
+  const int inner = args.inner > 1 ? static_cast<int>(args.inner) : 1;
+  const int64_t outer_y = blockIdx.y / inner, inner_y = blockIdx.y % inner;
+  const S* __restrict__ A = static_cast<const S*>(args.A) + outer_y * args.stride_a + inner_y * args.inner_a;
+  const S* __restrict__ B = static_cast<const S*>(args.B) + outer_y * args.stride_b + inner_y * args.inner_b;
+  S* __restrict__ C = static_cast<S*>(args.C) + outer_y * args.stride_c + inner_y * args.inner_c;
   const int64_t M = args.M, N = args.N, K = args.K;
   const int KT = static_cast<int>((K + BK - 1) / BK);
   const bool tail = K % BK != 0 || (TA && M % 8 != 0) || (!TB && N % 8 != 0);

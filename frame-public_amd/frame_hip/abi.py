@@ -93,6 +93,8 @@ _SIGS = {
                                 c_void_p, c_int64, c_int32, c_void_p]),
     "fh_attention_fwd": (c_int32, [c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64,
                                    c_float, c_void_p]),
+    "fh_attention_grad_workspace": (c_int64, [c_int64, c_int64, c_int64]),
+    "fh_attention_grad": (c_int32, [c_int32] + [c_void_p] * 8 + [c_int64] * 5 + [c_float, c_void_p]),
     "fh_attention_supported": (c_int32, [c_int32, c_int64, c_int64]),
     "fh_softmax_rows": (c_int32, [c_int32, c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
     "fh_layer_norm_rows": (c_int32, [c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_float,

@@ -220,6 +220,8 @@ inline constexpr std::string_view kConvWgradOp = "hip_conv2d_wgrad_nhwc_internal
 // attention(q, k, v) [batch*seq, heads*dh] -> [batch*seq, heads*dh]: the per-(batch, head) slice / matmul / mul /
 // softmax / matmul / concat decomposition in one kernel (attrs batch, seq, heads, dh, scale; see fh_attention_fwd).
 inline constexpr std::string_view kAttentionOp = "hip_attention_internal";
+// attention_grad(q, k, v, dout) -> dq, dk, dv, workspace (the same attributes; see fh_attention_grad).
+inline constexpr std::string_view kAttentionGradOp = "hip_attention_grad_internal";
 
 // The graph HipBackend::compile plans for `graph` (already through the pass pipeline): attention, epilogue
 // (opt_level >= 1) and channels-last conv lowering applied to a copy. Host-only; used by compile and by

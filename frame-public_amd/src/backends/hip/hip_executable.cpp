@@ -8,7 +8,8 @@
 //
 // Lowering (allowed inside Backend::compile by the HAL contract, include/frame/hal/backend.h:45-63):
 //  * attention (every opt_level): the per-(batch, head) decomposition of multi-head attention becomes one
-// attention node (see lower_attention);
+// attention node (see lower_attention); at opt_level >= 1 its gradients in a training graph become one too (see
+// lower_attention_grads);
 //  * epilogue fusion (opt_level >= 1): a matmul
 // or conv2d whose only consumer is an elementwise node (add, mul, relu, square, gelu or a fused chain) that
 // takes the contraction result as its first operand is replaced by one internal node that applies the
@@ -1010,6 +1011,10 @@ struct AttentionMatch {
   int64_t batch = 0, seq = 0, heads = 0, dh = 0;
   float scale = 0.0f;
   std::vector<const ir::Node*> absorbed;  // every node of the decomposition, the batch concat included
+  struct Head {
+    const ir::Value *q, *kt, *v, *probs;  // the head's Q, transposed K, V and softmax
+  };
+  std::vector<Head> head;  // of (b, h), b * heads + h
 };
 
 // Matches the decomposition the reference's MultiHeadAttention emits (reference: src/nn/layers.cpp:1014-1080),
@@ -1081,12 +1086,254 @@ std::optional<AttentionMatch> match_attention(const ir::Node* root) {
         m.absorbed.push_back(col);
       }
       m.absorbed.insert(m.absorbed.end(), {pv, sm, mul, qk, kt});
+      m.head.push_back({heads_in[0], qk->inputs()[1], heads_in[2], pv->inputs()[0]});
     }
   }
   for (const ir::Value* x : {m.q, m.k, m.v})
     if (x->type().shape != ot.shape || !(x->type().dtype == ot.dtype)) return std::nullopt;
   m.scale = *scale;
   return m;
+}
+
+// The gradients of one attention: the three assembled values [batch*seq, heads*dh] in the gradient graph and the output
+// gradient they come from.
+struct AttentionGradMatch {
+  AttentionMatch fwd;
+  ir::Value* dout = nullptr;
+  const ir::Value* grads[3] = {nullptr, nullptr, nullptr};  // dq, dk, dv
+};
+
+// The other input of a two-input node with op `op` that reads x, else nullptr.
+const ir::Value* partner(const ir::Node* n, std::string_view op, const ir::Value* x) {
+  if (n == nullptr || n->op() != op || n->inputs().size() != 2 || n->outputs().size() != 1) return nullptr;
+  if (n->inputs()[0] == x) return n->inputs()[1];
+  return n->inputs()[1] == x ? n->inputs()[0] : nullptr;
+}
+
+// Matches the gradients of the decomposition `m` (reference: src/ops/schemas/sequence.cpp:358-406 and the matmul, slice and
+// transpose gradients around it), per (batch, head):
+//   dP = matmul_grad_lhs(dO_bh, V), dV = matmul_grad_rhs(P, dO_bh), s = reshape(sum_axis1(mul(P, dP))),
+//   dS = fused mul;mul(P, add(dP, mul(matmul(s, ones), -1)), C), dQ = matmul_grad_lhs(dS, K^T),
+//   dK = transpose(matmul_grad_rhs(Q, dS)),
+// placed by concats with zeros and added up to [batch*seq, heads*dh]. Any deviation leaves the graph as it is.
+std::optional<AttentionGradMatch> match_attention_grad(
+    const ir::Graph& g, AttentionMatch m,
+    const std::unordered_map<const ir::Value*, std::vector<const ir::Node*>>& users) {
+  struct Place {
+    int which;
+    int64_t row, col;  // offset from the block's own place
+  };
+  const DType dtype = m.q->type().dtype;
+  std::unordered_map<const ir::Node*, std::optional<float>> splats;
+  auto splat = [&](const ir::Value* v) {
+    const ir::Node* p = v->producer();
+    auto it = splats.find(p);
+    if (it == splats.end()) it = splats.emplace(p, splat_value(p, dtype)).first;
+    return it->second;
+  };
+  auto user = [&](const ir::Value* v, std::string_view op, size_t index) -> const ir::Node* {
+    const ir::Node* found = nullptr;
+    auto it = users.find(v);
+    if (it == users.end()) return nullptr;
+    for (const ir::Node* n : it->second) {
+      if (n->op() != op || n->inputs().size() <= index || n->inputs()[index] != v || n->outputs().size() != 1) continue;
+      if (found != nullptr) return nullptr;  // one gradient only
+      found = n;
+    }
+    return found;
+  };
+  AttentionGradMatch out;
+  std::unordered_map<const ir::Value*, std::vector<Place>> placed;                        // the blocks in a value
+  std::unordered_map<const ir::Value*, std::vector<std::pair<int64_t, int64_t>>> blocks;  // and their own places
+  for (int64_t b = 0; b < m.batch; ++b) {
+    for (int64_t h = 0; h < m.heads; ++h) {
+      const AttentionMatch::Head& hd = m.head[static_cast<size_t>(b * m.heads + h)];
+      const ir::Node* dv = user(hd.probs, "matmul_grad_rhs_internal", 0);
+      if (dv == nullptr) return std::nullopt;
+      const ir::Value* doh = dv->inputs()[1];
+      const ir::Node* dp = user(hd.v, "matmul_grad_lhs_internal", 1);
+      if (dp == nullptr || dp->inputs()[0] != doh) return std::nullopt;
+      const ir::Value* dpv = &dp->outputs()[0];
+      const ir::Node* col = slice_of(doh, 1, h * m.dh, (h + 1) * m.dh);
+      const ir::Node* row = col ? slice_of(col->inputs()[0], 0, b * m.seq, (b + 1) * m.seq) : nullptr;
+      if (row == nullptr || (out.dout != nullptr && out.dout != row->inputs()[0])) return std::nullopt;
+      out.dout = row->inputs()[0];
+      // dS = P * (dP + -1 * broadcast(sum(P * dP))) * C
+      const ir::Node* ds = user(hd.probs, ops::kFusedElementwiseOpName, 0);
+      if (ds == nullptr || ds->inputs().size() != 3) return std::nullopt;
+      ops::FusedElementwiseChain chain;
+      if (!ops::decode_and_validate_fused_chain(ds->attrs(), 3, chain).is_ok() || chain.sub_ops.size() != 2 ||
+          chain.sub_ops[0] != "mul" || chain.sub_ops[1] != "mul" || chain.arities[0] != 2 || chain.arities[1] != 2)
+        return std::nullopt;
+      const std::optional<float> c = splat(ds->inputs()[2]);
+      if (!c || *c != m.scale) return std::nullopt;
+      const ir::Value* neg = partner(ds->inputs()[1]->producer(), "add", dpv);
+      const ir::Node* negn = neg ? producer_op(neg, "mul", 2) : nullptr;
+      if (negn == nullptr) return std::nullopt;
+      const bool first = splat(negn->inputs()[0]).has_value();
+      const std::optional<float> minus = splat(negn->inputs()[first ? 0 : 1]);
+      const ir::Node* wide = producer_op(negn->inputs()[first ? 1 : 0], "matmul", 2);
+      if (!minus || *minus != -1.0f || wide == nullptr) return std::nullopt;
+      const std::optional<float> ones = splat(wide->inputs()[1]);
+      const ir::Node* rs = producer_op(wide->inputs()[0], "reshape", 1);
+      if (!ones || *ones != 1.0f || rs == nullptr || rs->outputs()[0].type().shape != Shape({m.seq, 1})) return std::nullopt;
+      const ir::Node* sum = producer_op(rs->inputs()[0], "sum", 1);
+      const auto* axes = sum ? attr_of<std::vector<int64_t>>(sum, "axes") : nullptr;
+      if (axes == nullptr || *axes != std::vector<int64_t>{1}) return std::nullopt;
+      if (partner(sum->inputs()[0]->producer(), "mul", hd.probs) != dpv) return std::nullopt;
+      const ir::Value* dsv = &ds->outputs()[0];
+      const ir::Node* dq = user(dsv, "matmul_grad_lhs_internal", 0);
+      const ir::Node* dkt = user(dsv, "matmul_grad_rhs_internal", 1);
+      if (dq == nullptr || dq->inputs()[1] != hd.kt || dkt == nullptr || dkt->inputs()[0] != hd.q) return std::nullopt;
+      const ir::Node* dk = user(&dkt->outputs()[0], "transpose", 0);
+      const auto* perm = dk ? attr_of<std::vector<int64_t>>(dk, "perm") : nullptr;
+      if (perm == nullptr || *perm != std::vector<int64_t>{1, 0}) return std::nullopt;
+      const std::pair<int64_t, int64_t> at{b * m.seq, h * m.dh};
+      const ir::Value* block[3] = {&dq->outputs()[0], &dk->outputs()[0], &dv->outputs()[0]};
+      for (int i = 0; i < 3; ++i) {
+        placed[block[i]] = {{i, -at.first, -at.second}};
+        blocks[block[i]] = {at};
+      }
+    }
+  }
+  for (const ir::Node* n : g.topological_order()) {
+    if (n->outputs().size() != 1 || n->inputs().empty()) continue;
+    const ir::Value* o = &n->outputs()[0];
+    std::vector<Place> places;
+    std::vector<std::pair<int64_t, int64_t>> homes;
+    bool ok = true;
+    if (n->op() == "concat") {
+      const int64_t* axis = attr_of<int64_t>(n, "axis");
+      if (axis == nullptr || *axis > 1 || o->type().shape.rank() != 2) continue;
+      int64_t at = 0;
+      for (const ir::Value* in : n->inputs()) {
+        if (auto it = placed.find(in); it != placed.end()) {
+          for (Place p : it->second) {
+            (*axis == 0 ? p.row : p.col) += at;
+            places.push_back(p);
+          }
+          homes.insert(homes.end(), blocks[in].begin(), blocks[in].end());
+        } else if (const auto z = splat(in); !z || *z != 0.0f) {
+          ok = false;
+          break;
+        }
+        at += in->type().shape.dim(static_cast<int32_t>(*axis));
+      }
+    } else {
+      bool adds = n->op() == "add";
+      if (n->op() == ops::kFusedElementwiseOpName) {
+        ops::FusedElementwiseChain chain;
+        adds = ops::decode_and_validate_fused_chain(n->attrs(), static_cast<int64_t>(n->inputs().size()), chain).is_ok() &&
+               std::all_of(chain.sub_ops.begin(), chain.sub_ops.end(), [](const auto& s) { return s == "add"; });
+      }
+      if (!adds) continue;
+      for (const ir::Value* in : n->inputs()) {
+        auto it = placed.find(in);
+        if (it == placed.end()) {
+          ok = false;
+          break;
+        }
+        places.insert(places.end(), it->second.begin(), it->second.end());
+        homes.insert(homes.end(), blocks[in].begin(), blocks[in].end());
+      }
+    }
+    if (!ok || places.empty()) continue;
+    const int which = places[0].which;
+    if (std::any_of(places.begin(), places.end(), [&](const Place& p) { return p.which != which; })) continue;
+    std::sort(homes.begin(), homes.end());
+    if (std::adjacent_find(homes.begin(), homes.end()) != homes.end()) continue;  // a block twice: not an assembly
+    placed[o] = places;
+    blocks[o] = homes;
+    if (out.grads[which] == nullptr && static_cast<int64_t>(homes.size()) == m.batch * m.heads &&
+        o->type().shape == m.q->type().shape && o->type().dtype == dtype &&
+        std::all_of(places.begin(), places.end(), [](const Place& p) { return p.row == 0 && p.col == 0; }))
+      out.grads[which] = o;
+  }
+  for (const ir::Value* v : out.grads)
+    if (v == nullptr) return std::nullopt;
+  if (out.dout->type().shape != m.q->type().shape || !(out.dout->type().dtype == dtype)) return std::nullopt;
+  out.fwd = std::move(m);
+  return out;
+}
+
+// Replaces the gradients of every matched attention by one kAttentionGradOp node, at the first of the three assembled
+// values. The forward decomposition, which then serves the forward only, is lower_attention's.
+Status lower_attention_grads(ir::Graph& g) {
+  const std::vector<ir::Node*> order = g.topological_order();
+  if (is_forward(g)) return Status::ok();
+  std::unordered_map<const ir::Value*, std::vector<const ir::Node*>> users;
+  for (const ir::Node* n : order)
+    for (const ir::Value* v : n->inputs()) users[v].push_back(n);
+  std::vector<AttentionGradMatch> matches;
+  std::unordered_map<const ir::Node*, size_t> roots;  // producers of the assembled gradients
+  for (const ir::Node* n : order) {
+    std::optional<AttentionMatch> m = match_attention(n);
+    if (!m) continue;
+    std::optional<AttentionGradMatch> grad = match_attention_grad(g, std::move(*m), users);
+    if (!grad) continue;
+    bool fresh = true;
+    for (const ir::Value* v : grad->grads) fresh = fresh && !roots.count(v->producer());
+    if (!fresh) continue;
+    for (const ir::Value* v : grad->grads) roots[v->producer()] = matches.size();
+    matches.push_back(std::move(*grad));
+  }
+  if (matches.empty()) return Status::ok();
+
+  auto inputs_of = [&](const ir::Node* n) {
+    std::vector<ir::Value*> in(n->inputs().begin(), n->inputs().end());
+    if (auto r = roots.find(n); r != roots.end()) {
+      const AttentionGradMatch& m = matches[r->second];
+      in = {m.fwd.q, m.fwd.k, m.fwd.v, m.dout};
+    }
+    return in;
+  };
+  std::unordered_set<const ir::Node*> live;
+  for (const ir::Value* o : g.outputs())
+    if (o->producer()) live.insert(o->producer());
+  for (auto it = order.rbegin(); it != order.rend(); ++it) {
+    if (!live.count(*it)) continue;
+    for (const ir::Value* x : inputs_of(*it))
+      if (x->producer()) live.insert(x->producer());
+  }
+  std::unordered_map<const ir::Value*, ir::Value*> map;
+  std::unordered_set<size_t> emitted;
+  ir::Graph out{std::string(g.name())};
+  for (const ir::Node* n : order) {
+    if (n->op() == ir::kGraphInputOp) {
+      Result<ir::Value*> v = out.add_graph_input(n->outputs()[0].type());
+      if (!v.is_ok()) return v.status();
+      map[&n->outputs()[0]] = v.value();
+      continue;
+    }
+    if (!live.count(n)) continue;
+    std::vector<ir::Value*> ins;
+    for (const ir::Value* in : inputs_of(n)) ins.push_back(map.at(in));
+    if (auto r = roots.find(n); r != roots.end()) {
+      if (!emitted.insert(r->second).second) continue;
+      const AttentionGradMatch& m = matches[r->second];
+      ir::TensorType ws = m.fwd.q->type();
+      ws.shape = Shape({2 * m.fwd.batch * m.fwd.heads * m.fwd.seq, m.fwd.seq});
+      const ir::TensorType t = m.fwd.q->type();
+      Result<ir::Node*> a = out.create_node(std::string(kAttentionGradOp), std::move(ins), {t, t, t, ws});
+      if (!a.is_ok()) return a.status();
+      a.value()->set_attr("batch", ir::AttrValue{m.fwd.batch});
+      a.value()->set_attr("seq", ir::AttrValue{m.fwd.seq});
+      a.value()->set_attr("heads", ir::AttrValue{m.fwd.heads});
+      a.value()->set_attr("dh", ir::AttrValue{m.fwd.dh});
+      a.value()->set_attr("scale", ir::AttrValue{static_cast<double>(m.fwd.scale)});
+      for (int32_t i = 0; i < 3; ++i) map[m.grads[i]] = a.value()->output(i);
+      continue;
+    }
+    std::vector<ir::TensorType> types;
+    for (const ir::Value& o : n->outputs()) types.push_back(o.type());
+    Result<ir::Node*> c = out.create_node(std::string(n->op()), std::move(ins), std::move(types));
+    if (!c.is_ok()) return c.status();
+    for (const auto& [k, v] : n->attrs()) c.value()->set_attr(k, v);
+    for (size_t i = 0; i < n->outputs().size(); ++i) map[&n->outputs()[i]] = c.value()->output(static_cast<int32_t>(i));
+  }
+  for (const ir::Value* o : g.outputs()) FRAME_RETURN_IF_ERROR(out.mark_output(map.at(o)));
+  g = std::move(out);
+  return Status::ok();
 }
 
 // Replaces every matched attention decomposition by one kAttentionOp node. Nodes of a decomposition whose
@@ -1744,7 +1991,10 @@ Status lower_grouped_gemms(ir::Graph& g) {
 }
 
 Result<ir::Graph> lower_for_hip(const ir::Graph& graph, int32_t opt_level) {
-  Result<ir::Graph> work = lower_matmul_grads(graph, opt_level);
+  Result<ir::Graph> source = ir::clone_graph(graph);
+  if (!source.is_ok()) return source.status();
+  if (opt_level >= 1) FRAME_RETURN_IF_ERROR(lower_attention_grads(source.value()));
+  Result<ir::Graph> work = lower_matmul_grads(source.value(), opt_level);
   if (!work.is_ok()) return work.status();
   // Attention runs at every level (like the conv lowering), before the epilogue fusion would claim its matmuls.
   FRAME_RETURN_IF_ERROR(lower_attention(work.value()));

@@ -592,6 +592,34 @@ Status attention_kernel(KernelContext& ctx) {
   return Status::ok();
 }
 
+// The gradients of such an attention (fh_attention_grad): inputs q, k, v, dout, outputs dq, dk, dv and the workspace.
+Status attention_grad_kernel(KernelContext& ctx) {
+  const std::string op(kAttentionGradOp);
+  FRAME_RETURN_IF_ERROR(arity(ctx, op, 4, 4));
+  FRAME_RETURN_IF_ERROR(same_dtype(ctx, op));
+  const auto* batch = attr<int64_t>(ctx, "batch");
+  const auto* seq = attr<int64_t>(ctx, "seq");
+  const auto* heads = attr<int64_t>(ctx, "heads");
+  const auto* dh = attr<int64_t>(ctx, "dh");
+  const auto* scale = attr<double>(ctx, "scale");
+  if (!batch || !seq || !heads || !dh || !scale) return invalid(op, "missing batch/seq/heads/dh/scale attributes");
+  const Shape want({*batch * *seq, *heads * *dh});
+  for (const Tensor& t : ctx.inputs)
+    if (t.shape() != want) return invalid(op, "q, k, v, dout must be [batch*seq, heads*dh]");
+  for (size_t i = 0; i < 3; ++i)
+    if (ctx.outputs[i].shape() != want) return invalid(op, "dq, dk, dv must be [batch*seq, heads*dh]");
+  Result<int32_t> dt = float_code(op, ctx.outputs[0].dtype());
+  if (!dt.is_ok()) return dt.status();
+  Tensor& ws = ctx.outputs[3];
+  FRAME_HIP_RETURN_IF_ERROR(
+      fh_attention_grad(dt.value(), ctx.inputs[0].raw_data(), ctx.inputs[1].raw_data(), ctx.inputs[2].raw_data(),
+                        ctx.inputs[3].raw_data(), ctx.outputs[0].raw_data(), ctx.outputs[1].raw_data(),
+                        ctx.outputs[2].raw_data(), ws.raw_data(), ws.numel() * 2, *batch, *seq, *heads, *dh,
+                        static_cast<float>(*scale), stream_handle(ctx)),
+      "op '" + op + "' (hip)");
+  return Status::ok();
+}
+
 Status layer_norm_kernel(KernelContext& ctx) {
   FRAME_RETURN_IF_ERROR(arity(ctx, "layer_norm", 3, 1));
   FRAME_RETURN_IF_ERROR(same_dtype(ctx, "layer_norm"));
@@ -1095,6 +1123,7 @@ FRAME_REGISTER_KERNEL(kPackInputC8Op, kHipBackendName, &pack_input_c8_kernel);
 FRAME_REGISTER_KERNEL(kPackFilterC8Op, kHipBackendName, &pack_filter_c8_kernel);
 FRAME_REGISTER_KERNEL("softmax", kHipBackendName, &softmax_kernel);
 FRAME_REGISTER_KERNEL(kAttentionOp, kHipBackendName, &attention_kernel);
+FRAME_REGISTER_KERNEL(kAttentionGradOp, kHipBackendName, &attention_grad_kernel);
 FRAME_REGISTER_KERNEL("layer_norm", kHipBackendName, &layer_norm_kernel);
 FRAME_REGISTER_KERNEL("max_pool2d", kHipBackendName, &pool_kernel<0>);
 FRAME_REGISTER_KERNEL("avg_pool2d", kHipBackendName, &pool_kernel<1>);

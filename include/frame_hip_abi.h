@@ -311,6 +311,16 @@ fh_status fh_attention_fwd(int32_t dtype, const void* q, const void* k, const vo
 /* 1 if fh_attention_fwd accepts (dtype, seq, dh), else 0. Host-only query; no counterpart in the reference. */
 int32_t fh_attention_supported(int32_t dtype, int64_t seq, int64_t dh);
 
+/* Gradients of fh_attention_fwd's result with respect to q, k and v for the output gradient dout, all [batch*seq, heads*dh]:
+ * the per-(batch, head) chain of matmul gradients, softmax gradient (mul, sum, mul by -1, add, mul) and scaling that the
+ * gradient graph of the decomposition holds, with its roundings (reference: src/backends/cpu/kernels/matmul.cpp:187-327,
+ * softmax gradient src/ops/schemas/sequence.cpp:358-406). The probabilities and their gradient go through `workspace`
+ * (fh_attention_grad_workspace bytes, 16-byte aligned). Accepts what fh_attention_supported accepts. */
+int64_t fh_attention_grad_workspace(int64_t batch, int64_t seq, int64_t heads);
+fh_status fh_attention_grad(int32_t dtype, const void* q, const void* k, const void* v, const void* dout, void* dq, void* dk,
+                            void* dv, void* workspace, int64_t workspace_bytes, int64_t batch, int64_t seq, int64_t heads,
+                            int64_t dh, float scale, void* stream);
+
 /* 2-D pooling, NCHW. mode 0 = max (-inf padding, first max wins), 1 = average (include padding).
  * geom = {N, C, H, W, KH, KW, stride_h, stride_w, pad_h, pad_w}.
  * Replaces cudnnPoolingForward (reference: src/backends/cuda/kernels/pool.cpp:172-244);

@@ -421,3 +421,20 @@ def test_sgd_update_lowers_to_multi_tensor_launches():
     assert " mul(" not in low and " add(" not in low and "constant(" not in low
     assert "scales=[" in low
     assert host.hip_lowered(sgd, 0).count(" mul(") == len(specs)
+
+
+@pytest.mark.parametrize("shape", [dict(batch=2, seq=64, heads=4), dict(batch=1, seq=128, heads=2),
+                                   dict(batch=3, seq=64, heads=1)])
+def test_attention_gradients_lower_to_one_node(shape):
+    # the per-(batch, head) gradients of every block become one node, the forward the fused attention; at opt_level 0, and
+    # for a sequence the kernels do not take, the decomposition stays
+    d = 64 * shape["heads"]
+    g, shapes = graphs.transformer_block(ffn=128, d_model=d, dtype=BF16, train=True, **shape)
+    text = host.backward(g.text(), 0, list(range(1, len(shapes) + 1)))
+    low = host.hip_lowered(text, 1)
+    assert low.count("hip_attention_grad_internal(") == 1 and low.count("hip_attention_internal(") == 1
+    assert " slice(" not in low and " softmax(" not in low
+    assert "hip_attention_grad_internal(" not in host.hip_lowered(text, 0)
+    g, shapes = graphs.transformer_block(batch=1, seq=40, d_model=128, heads=2, ffn=128, dtype=BF16, train=True)
+    low = host.hip_lowered(host.backward(g.text(), 0, list(range(1, len(shapes) + 1))), 1)
+    assert "hip_attention_grad_internal(" not in low and " softmax(" in low

@@ -1470,6 +1470,48 @@ def test_attention_matches_decomposition(hip, case):
     print(f"  bit-identical fraction {same:.4f}, max abs err {stats['max_abs']:.3g} (rms {stats['rms']:.3g})")
 
 
+ATTENTION_GRAD_CASES = [(BF16, 2, 64, 3, 0.125), (F16, 1, 128, 2, 0.125), (BF16, 1, 192, 1, 0.1), (BF16, 1, 256, 2, 0.125),
+                        (F16, 3, 64, 1, 0.1), (BF16, 1, 512, 2, 0.125)]
+
+
+@pytest.mark.parametrize("case", ATTENTION_GRAD_CASES, ids=lambda c: "-".join(str(x) for x in c))
+def test_attention_grad_matches_decomposition(hip, case):
+    """fh_attention_grad against the gradient graph's chain evaluated per (batch, head) with its roundings (float64 sums,
+    so each result differs by fp32 sums of up to 512 terms and the roundings they push over: the file's 1e-2 rule)."""
+    dtype, batch, seq, heads, scale = case
+    say(f"attention grad dtype={dtype} batch={batch} seq={seq} heads={heads} scale={scale}")
+    shape = (batch * seq, heads * 64)
+    q, k, v, do = (synth.tensor(70 + i, shape, dtype, "normal") for i in range(4))
+
+    def rnd(a):
+        return synth.to_float(synth.to_storage(a.astype(np.float32), dtype), dtype).astype(np.float64)
+
+    c = float(rnd(np.array([scale]))[0])
+    want = [np.zeros(shape) for _ in range(3)]
+    for b in range(batch):
+        for h in range(heads):
+            at = (slice(b * seq, (b + 1) * seq), slice(h * 64, (h + 1) * 64))
+            qh, kh, vh, oh = (synth.to_float(t[at], dtype).astype(np.float64) for t in (q, k, v, do))
+            s = rnd(rnd(qh @ kh.T) * c)
+            e = np.exp(s - s.max(1, keepdims=True))
+            p = rnd(e / e.sum(1, keepdims=True))
+            dp = rnd(oh @ vh.T)
+            ds = rnd(rnd(p * rnd(dp - rnd(rnd(p * dp).sum(1, keepdims=True)))) * c)
+            for w, g in zip(want, (ds @ kh, ds.T @ qh, p.T @ oh)):
+                w[at] = g
+    dev_in = [dev(hip, t) for t in (q, k, v, do)]
+    outs = [hip.DeviceBuffer(q.nbytes) for _ in range(3)]
+    need = hip.lib().fh_attention_grad_workspace(batch, seq, heads)
+    ws = hip.DeviceBuffer(need)
+    args = [dtype, *[d.value for d in dev_in], *[d.value for d in outs], ws.value]
+    assert hip.lib().fh_attention_grad(*args, need - 1, batch, seq, heads, 64, c, None) == 1  # workspace too small
+    assert hip.lib().fh_attention_grad(*args, need, batch, seq + 1, heads, 64, c, None) == 4  # unsupported sequence
+    hip.check(hip.lib().fh_attention_grad(*args, need, batch, seq, heads, 64, c, None))
+    for name, d, w in zip("qkv", outs, want):
+        got = d.download(shape, q.dtype)
+        assert_close(got, synth.to_storage(w.astype(np.float32), dtype), dtype, what=f"d{name}")
+
+
 def test_attention_rejects_unsupported(hip):
     # shapes outside the kernel's envelope are refused without a launch
     for dtype, seq, dh in [(F32, 128, 64), (BF16, 128, 32), (BF16, 96, 64), (BF16, 576, 64), (BF16, 0, 64)]:

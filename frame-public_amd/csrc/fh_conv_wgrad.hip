@@ -6,15 +6,18 @@
 // dW in the reference's [Cout][Cin][KH][KW] layout with one rounding.
 //
 // Both operands are k-major (rows of p), so both MFMA fragments come from ds_read_b64_tr_b16 transpose reads of
-// [BK][cols] LDS tiles (the B-operand path of the GEMM kernel, used for A as well). Tiles: WM (co) x 128 (a,b,ci)
-// per workgroup with WM = 128 when Cout >= 128 (4 waves of 64 x 64, four 32x32x16 MFMA tiles each) and WM = 64
-// otherwise (4 waves of 32 x 64, two tiles), register-staged loads with zero fill for rows past the split and
-// taps in the padding, two LDS stages of 64 p-rows. The larger tile loads 1.5x fewer bytes per MFMA, which is
-// what limits this kernel: operands come from L2 (x is read once per filter tap).
+// [BK][cols] LDS tiles; the k loop is the one of the GEMMs of any alignment (fh_gemm_any.h: v_mfma_f32_16x16x32, two LDS
+// buffers of 64 p-rows, two register sets, loads two tiles ahead, no branch). Loads are unconditional: rows past the split
+// and taps in the padding read the operand's first vector and are zeroed on their way to LDS, because a load behind a
+// branch is waited for before the next one is issued. Tiles: WM (co) x 128 (a,b,ci) per workgroup of 4 waves, WM = 128 when
+// Cout >= 128 and 64 otherwise; two workgroups per CU. What bounds it is the operands' way from L2, as x is read once per
+// filter tap: ResNet-18's layers move 230-385 MB through it per gradient, 6-7.7 TB/s. us per gradient at batch 64, bf16
+// (before: conditional loads one tile ahead, 32x32x16 tiles): WM 64 72.0 -> 64.4, WM 128 30.8 -> 30.5.
 #include <algorithm>
 #include <mutex>
 #include <string>
 
+#include "fh_gemm_any.h"
 #include "fh_mfma16.h"
 
 namespace fh {
@@ -48,20 +51,64 @@ __device__ __forceinline__ int32_t div_by(int32_t n, uint64_t m, uint32_t s) {
   return static_cast<int32_t>((static_cast<uint64_t>(static_cast<uint32_t>(n)) * m) >> s);
 }
 
-__device__ __forceinline__ int swz8(int krow) { return 2 * (krow & 3); }
-__device__ __forceinline__ int swz16(int krow) { return (2 * (krow & 3)) ^ (8 * (krow & 1)); }
-
 // Workgroup tile rows for a filter of cout output channels (the host's and the kernel's choice must agree).
 inline int wgrad_wm(int64_t cout) { return cout >= 128 ? 128 : 64; }
+
+// One operand of a tile, COLS columns of rows p: thread t holds the column vector t % CHUNKS of the p-rows
+// t / CHUNKS + u * NT / CHUNKS.
+template <typename T, int COLS>
+struct RowsOperand : gemm_any::Operand<T, COLS, kWK, kWThreads, false> {
+  using Base = gemm_any::Operand<T, COLS, kWK, kWThreads, false>;
+  using S = typename Io<T>::storage;
+  static constexpr int U = Base::UNITS, STEP = kWThreads / Base::CHUNKS;
+  static_assert(kWThreads % Base::CHUNKS == 0, "a thread's units are the same columns");
+  uint32_t live[2];  // bit u: unit u holds values (zero otherwise)
+
+  __device__ void init(int tid) {
+    const int c = tid % Base::CHUNKS;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int row = tid / Base::CHUNKS + u * STEP;
+      this->kk[u] = row;
+      this->dst[u] = (row / 32) * Base::SUB + (row % 32) * (COLS * 2) + ((c ^ b_swizzle16<Base::CHUNKS>(row % 32)) * 16);
+    }
+  }
+  // address(p): the unit's vector in row p, or null where it is zero
+  template <int SET, typename Address>
+  __device__ void load(int32_t p0, const S* base, Address&& address) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const S* at = address(p0 + this->kk[u]);
+      m |= at != nullptr ? 1u << u : 0u;
+      this->reg[SET][u].v[0] = *reinterpret_cast<const u32x4_t*>(at != nullptr ? at : base);
+    }
+    live[SET] = m;
+  }
+  template <int SET>
+  __device__ void store(unsigned char* lds, uint32_t&) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool on = (live[SET] >> u) & 1u;
+      u32x4_t v = this->reg[SET][u].v[0];
+#pragma unroll
+      for (int d = 0; d < 4; ++d) v[d] = on ? v[d] : 0u;
+      *reinterpret_cast<u32x4_t*>(lds + this->dst[u]) = v;
+    }
+  }
+};
 
 template <typename T, int kWM>
 __global__ __launch_bounds__(kWThreads) void conv_wgrad_kernel(WgradArgs a) {
   static_assert(kWM == 64 || kWM == 128, "tile rows");
-  constexpr int MT = kWM / 64;  // 32-row MFMA tiles per wave
   using S = typename Io<T>::storage;
-  __shared__ __attribute__((aligned(16))) S As[2][kWK * kWM];
-  __shared__ __attribute__((aligned(16))) S Bs[2][kWK * kWN];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  using OpA = RowsOperand<T, kWM>;
+  using OpB = RowsOperand<T, kWN>;
+  constexpr int WM = kWM / 2, WN = kWN / 2, TM = WM / 16, TN = WN / 16;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * (OpA::BYTES + OpB::BYTES)];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
   const int tm = blockIdx.x / a.tiles_n, tn = blockIdx.x % a.tiles_n;
   const int m0 = tm * kWM, n0 = tn * kWN;
   // p fits 32 bits (checked by the host)
@@ -70,145 +117,58 @@ __global__ __launch_bounds__(kWThreads) void conv_wgrad_kernel(WgradArgs a) {
   const S* __restrict__ X = static_cast<const S*>(a.x);
   const S* __restrict__ DY = static_cast<const S*>(a.dy);
 
-  // A loads: kWK*(WM/8) chunks, rows t/(WM/8) + A_STEP i, column chunk t%(WM/8); B loads: kWK*16 chunks, rows
-  // t/16 + 16 i, column chunk t%16 (a fixed filter tap and ci block per thread)
-  constexpr int A_CH = kWM / 8, A_STEP = kWThreads / A_CH;
-  // A rows of 8 chunks swizzle like the GEMM's A, rows of 16 chunks like B
-  auto swza = [](int krow) { return kWM == 64 ? swz8(krow) : swz16(krow); };
-  constexpr int A_LOADS = kWK * A_CH / kWThreads, B_LOADS = kWK * (kWN / 8) / kWThreads;
-  const int a_row = tid / A_CH, a_chunk = tid % A_CH;
-  const bool a_col_ok = m0 + 8 * a_chunk < a.cout;
-  const int b_row = tid >> 4, b_chunk = tid & 15;
-  const int ncol = n0 + 8 * b_chunk;
-  const bool b_col_ok = ncol < a.nc;
-  const int tap = b_col_ok ? ncol / a.cin : 0;
-  const int ci = b_col_ok ? ncol - tap * a.cin : 0;
+  OpA oa;
+  OpB ob;
+  oa.init(tid);
+  ob.init(tid);
+  // this thread's columns: 8 output channels of dy, 8 input channels of one filter tap of x
+  const int mcol = m0 + 8 * (tid % OpA::CHUNKS);
+  const bool a_ok = mcol < a.cout;
+  const int ncol = n0 + 8 * (tid % OpB::CHUNKS);
+  const bool b_ok = ncol < a.nc;
+  const int tap = b_ok ? ncol / a.cin : 0;
+  const int ci = b_ok ? ncol - tap * a.cin : 0;
   const int ta = tap / a.kw, tb = tap - ta * a.kw;
   const int32_t plane = a.oh * a.ow;
-
-  uint4 ra[A_LOADS], rb[B_LOADS];
-  auto load = [&](int32_t p0) {
-#pragma unroll
-    for (int i = 0; i < A_LOADS; ++i) {
-      const int32_t p = p0 + a_row + A_STEP * i;
-      ra[i] = (p < p_end && a_col_ok) ? *reinterpret_cast<const uint4*>(DY + static_cast<int64_t>(p) * a.cout + m0 + 8 * a_chunk)
-                                      : uint4{0, 0, 0, 0};
-    }
-#pragma unroll
-    for (int i = 0; i < B_LOADS; ++i) {
-      const int32_t p = p0 + b_row + 16 * i;
-      uint4 v{0, 0, 0, 0};
-      if (p < p_end && b_col_ok) {
-        const int32_t n = div_by(p, a.plane_m, a.plane_s);
-        const int32_t rem = p - n * plane;
-        const int32_t oh = div_by(rem, a.ow_m, a.ow_s), ow = rem - oh * a.ow;
-        const int32_t ih = oh * a.sh - a.ph + ta, iw = ow * a.sw - a.pw + tb;
-        if (ih >= 0 && ih < a.h && iw >= 0 && iw < a.w)
-          v = *reinterpret_cast<const uint4*>(X + ((static_cast<int64_t>(n) * a.h + ih) * a.w + iw) * a.cin + ci);
-      }
-      rb[i] = v;
-    }
+  auto dy_at = [&](int32_t p) -> const S* {
+    return p < p_end && a_ok ? DY + static_cast<int64_t>(p) * a.cout + mcol : nullptr;
   };
-  auto store = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < A_LOADS; ++i) {
-      const int r = a_row + A_STEP * i;
-      *reinterpret_cast<uint4*>(&As[buf][r * kWM + ((a_chunk ^ swza(r)) * 8)]) = ra[i];
-    }
-#pragma unroll
-    for (int i = 0; i < B_LOADS; ++i) {
-      const int r = b_row + 16 * i;
-      *reinterpret_cast<uint4*>(&Bs[buf][r * kWN + ((b_chunk ^ swz16(r)) * 8)]) = rb[i];
-    }
+  auto x_at = [&](int32_t p) -> const S* {
+    const int32_t n = div_by(p, a.plane_m, a.plane_s);
+    const int32_t rem = p - n * plane;
+    const int32_t oh = div_by(rem, a.ow_m, a.ow_s), ow = rem - oh * a.ow;
+    const int32_t ih = oh * a.sh - a.ph + ta, iw = ow * a.sw - a.pw + tb;
+    const bool in = p < p_end && b_ok && ih >= 0 && ih < a.h && iw >= 0 && iw < a.w;
+    return in ? X + ((static_cast<int64_t>(n) * a.h + ih) * a.w + iw) * a.cin + ci : nullptr;
+  };
+  auto load = [&]<int SET>(int kt) {  // (rows past the split are zero, so any tile number will do)
+    const int32_t p0 = p_begin + kt * kWK;
+    oa.template load<SET>(p0, DY, dy_at);
+    ob.template load<SET>(p0, X, x_at);
   };
 
-  // transpose-read addressing (bytes within a tile): lane group g = lane/16 covers 16 columns and 4 k rows;
-  // lane q + 4e of the group points at row (kbase + e), columns 4q .. 4q+3 of the group's 16
-  const int wm = wave >> 1, wn = wave & 1;
-  const int g = lane >> 4, r16 = lane & 15, q = r16 & 3, e = r16 >> 2;
-  const int krow0 = 8 * (g >> 1) + e;  // + 16 s + 4 h: krow & 3 and krow & 1 unchanged
-  int a_off[MT], b_off[2];
-  {
+  f32x4_t acc[TM][TN];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int col = wm * (kWM / 2) + 32 * mt + 16 * (g & 1) + 4 * q;
-      a_off[mt] = krow0 * (kWM * 2) + ((col >> 3) ^ swza(krow0)) * 16 + (col & 7) * 2;
-    }
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int c = wn * 64 + 32 * j + 16 * (g & 1) + 4 * q;
-      b_off[j] = krow0 * (kWN * 2) + ((c >> 3) ^ swz16(krow0)) * 16 + (c & 7) * 2;
-    }
-  }
-
-  f32x16_t acc[MT][2];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int x = 0; x < 16; ++x) acc[mt][j][x] = 0.0f;
-
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
   const int32_t steps = (p_end - p_begin + kWK - 1) / kWK;
-  if (steps > 0) {
-    load(p_begin);
-    store(0);
-  }
-  __syncthreads();
-  asm volatile("" ::: "memory");  // the transpose reads below are asm: keep them after the barrier
-  for (int32_t it = 0; it < steps; ++it) {
-    const int buf = it & 1;
-    if (it + 1 < steps) load(p_begin + (it + 1) * kWK);
-    const uint32_t abase = lds_addr((const FH_LDS void*)&As[buf][0]);
-    const uint32_t bbase = lds_addr((const FH_LDS void*)&Bs[buf][0]);
-    [&]<int... K_>(std::integer_sequence<int, K_...>) {
-      (
-          [&] {
-            constexpr int s = K_;  // 16-row k-step within the stage
-            u32x2_t al[MT], ah[MT], bl[2], bh[2];
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-              al[mt] = lds_read_tr16_b64<(16 * s) * kWM * 2>(abase + a_off[mt]);
-              ah[mt] = lds_read_tr16_b64<(16 * s + 4) * kWM * 2>(abase + a_off[mt]);
-            }
-            bl[0] = lds_read_tr16_b64<(16 * s) * kWN * 2>(bbase + b_off[0]);
-            bh[0] = lds_read_tr16_b64<(16 * s + 4) * kWN * 2>(bbase + b_off[0]);
-            bl[1] = lds_read_tr16_b64<(16 * s) * kWN * 2>(bbase + b_off[1]);
-            bh[1] = lds_read_tr16_b64<(16 * s + 4) * kWN * 2>(bbase + b_off[1]);
-            if constexpr (MT == 1)
-              asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(al[0]), "+v"(ah[0]), "+v"(bl[0]), "+v"(bh[0]), "+v"(bl[1]), "+v"(bh[1]));
-            else
-              asm volatile("s_waitcnt lgkmcnt(0)"
-                           : "+v"(al[0]), "+v"(ah[0]), "+v"(al[1]), "+v"(ah[1]), "+v"(bl[0]), "+v"(bh[0]), "+v"(bl[1]),
-                             "+v"(bh[1]));
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-              const u32x4_t af{al[mt][0], al[mt][1], ah[mt][0], ah[mt][1]};
-#pragma unroll
-              for (int j = 0; j < 2; ++j) mfma32<T>(af, u32x4_t{bl[j][0], bl[j][1], bh[j][0], bh[j][1]}, acc[mt][j]);
-            }
-          }(),
-          ...);
-    }(std::make_integer_sequence<int, kWK / 16>{});
-    // buf^1 was last read in the previous iteration, before its closing barrier: safe to refill now
-    if (it + 1 < steps) store(buf ^ 1);
-    __syncthreads();
-    asm volatile("" ::: "memory");
-  }
+  uint32_t unused = 0;
+  gemm_any::k_loop<T, OpA, OpB, kWK>(oa, ob, lds, steps, steps, wm * WM, wn * WN, lane, load, load, unused, acc);
 
-  // fp32 partial tile: row m = 8*(x/4) + 4*(lane/32) + x%4 of the wave's 32, column lane%32 of each 32-wide tile
+  // fp32 partial tile
   float* out = a.part + static_cast<int64_t>(blockIdx.y) * a.cout * a.nc;
-  const int hi = lane >> 5, l32 = lane & 31;
+  const int g = lane >> 4, r = lane & 15;
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = n0 + wn * 64 + 32 * j + l32;
+    for (int j = 0; j < TN; ++j) {
+      const int col = n0 + wn * WN + j * 16 + r;
       if (col >= a.nc) continue;
 #pragma unroll
-      for (int x = 0; x < 16; ++x) {
-        const int row = m0 + wm * (kWM / 2) + 32 * mt + 8 * (x >> 2) + 4 * hi + (x & 3);
-        if (row < a.cout) out[static_cast<int64_t>(row) * a.nc + col] = acc[mt][j][x];
+      for (int x = 0; x < 4; ++x) {
+        const int row = m0 + wm * WM + i * 16 + 4 * g + x;
+        if (row < a.cout) out[static_cast<int64_t>(row) * a.nc + col] = acc[i][j][x];
       }
     }
 }

@@ -454,7 +454,7 @@ fh_status launch(GemmArgs args, int64_t batch, hipStream_t stream) {
 // What the kernel accepts: an operand contiguous along m or n needs 8 of them (its units are moved back to the edge)
 // and a row stride of as many (a unit that straddles the edge runs into the next row).
 inline bool accepts(const GemmArgs& args, int64_t batch) {
-  if (args.K <= 0 || args.groups > 0 || args.row_softmax || batch > 65535) return false;
+  if (args.K < 0 || args.groups > 0 || args.row_softmax || batch > 65535) return false;  // (K = 0: zeros)
   if (args.trans_a ? args.M < 8 : false) return false;
   if (args.trans_b ? false : args.N < 8) return false;
   const int64_t tiles = ((args.M + 63) / 64) * ((args.N + 63) / 64);

@@ -131,6 +131,17 @@ def test_gemm_any_alignment(hip, dtype, shape):
             assert_bitwise(got, run_ew(hip, dtype, [1, 3], [2, 1], [plain, bias]), "epilogue vs separate program")
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+def test_gemm_without_k(hip, dtype):
+    # K = 0: an empty sum, then the epilogue; A and B may be null
+    say(f"gemm K=0 dtype={dtype}")
+    bias = synth.tensor(25, (700, 601), dtype, "normal")
+    dc, dbias = hip.DeviceBuffer(bias.nbytes), dev(hip, bias)
+    ep = hip.make_epilogue([(hip.EW_ADD, dbias.value)])
+    hip.check(hip.lib().fh_gemm(dtype, None, None, dc.value, 700, 601, 0, ctypes.byref(ep), None))
+    assert_bitwise(dc.download(bias.shape, bias.dtype), bias, "bias alone")
+
+
 @pytest.mark.parametrize("dtype", [F32, BF16, F16])
 @pytest.mark.parametrize("transposed", [1, 2])
 def test_gemm_transposed_operand(hip, dtype, transposed):

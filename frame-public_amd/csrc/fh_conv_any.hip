@@ -250,35 +250,30 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void conv_any_kernel(ConvAny
   k_loop<T, OpA, OpB, BK>(a, b, lds, KT, whole, wm * WM, wn * WN, lane, whole_load, any_load, tiny, acc);
 
   const int q = lane >> 4, r = lane & 15;
-  if constexpr (std::is_same_v<T, float>) {
-    if (outside_split(&tiny_seen, tiny, acc)) {
-      const float* x = static_cast<const float*>(g.x);
-      const float* w = static_cast<const float*>(g.w);
+  // Results that are not finite (and fp32 operands below the split's range) are taken again one product at a time, in the
+  // reference's order: it skips the taps in the padding, where a matrix product would add zero times the filter's value,
+  // NaN for an infinite one.
+  if (outside_split(&tiny_seen, tiny, acc)) {
+    const S* x = static_cast<const S*>(g.x);
+    const S* w = static_cast<const S*>(g.w);
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+    for (int j = 0; j < TN; ++j) {
+      const Pixel px = pixel_of(g, min(n0 + wn * WN + j * 16 + r, g.p - 1));
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-      for (int k0 = 0; k0 < g.k; k0 += 4) {
-        const int k = k0 + q;
-        const Tap t = tap_of(g, min(k, g.k - 1));
-        float va[TM], vb[TN];
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const int64_t row = min(m0 + wm * WM + i * 16 + r, g.cout - 1);
-          va[i] = k < g.k ? w[row * g.k + k] : 0.0f;
-        }
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const Pixel px = pixel_of(g, min(n0 + wn * WN + j * 16 + r, g.p - 1));
-          const bool in = k < g.k && static_cast<unsigned>(px.ih + t.a) < static_cast<unsigned>(g.h) &&
-                          static_cast<unsigned>(px.iw + t.b) < static_cast<unsigned>(g.wd);
-          vb[j] = 0.0f;
-          if (in) vb[j] = x[px.base + t.delta];
-        }
+      for (int i = 0; i < TM; ++i) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int k = 0; k < g.k; ++k) {
+        const Tap t = tap_of(g, k);
+        if (static_cast<unsigned>(px.ih + t.a) >= static_cast<unsigned>(g.h) ||
+            static_cast<unsigned>(px.iw + t.b) >= static_cast<unsigned>(g.wd))
+          continue;
+        const float v = Io<T>::load(x[px.base + t.delta]);
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[i], vb[j], acc[i][j], 0, 0, 0);
+          for (int e = 0; e < 4; ++e) {
+            const int64_t row = min(m0 + wm * WM + i * 16 + 4 * q + e, g.cout - 1);
+            acc[i][j][e] = acc[i][j][e] + v * Io<T>::load(w[row * g.k + k]);
+          }
       }
     }
   }

@@ -747,6 +747,27 @@ def test_conv2d_any_geometry(hip, dtype, geom):
             assert_bitwise(got, run_ew(hip, dtype, ops, arities, [plain] + ins), "epilogue vs separate program")
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16, F16])
+@pytest.mark.parametrize("hw,stride", [(16, 1), (11, 1), (9, 2)])
+def test_conv2d_infinite_filter_value_in_the_padding(hip, dtype, hw, stride):
+    # taps in the padding are skipped, not multiplied by zero: an infinite filter value reaches only the pixels whose tap
+    # lies inside the plane, bit for bit the oracle's infinities and NaN
+    geom = (2, 5, hw, hw, 20, 3, 3, stride, stride, 1, 1, 1)
+    say(f"conv with an infinite filter value dtype={dtype} {geom}")
+    x = np.abs(synth.to_float(synth.tensor(110, geom[:4], dtype, "normal"), dtype)) + np.float32(0.5)
+    wt = synth.to_float(synth.tensor(111, (20, 5, 3, 3), dtype, "normal", 0.2), dtype).copy()
+    wt[3, 2, 0, 0], wt[19, 4, 2, 1] = np.inf, -np.inf
+    x, wt = synth.to_storage(x, dtype), synth.to_storage(wt, dtype)
+    want = orc.conv2d(dtype, x, wt, None, geom)
+    dx, dw, dy = dev(hip, x), dev(hip, wt), hip.DeviceBuffer(want.nbytes)
+    hip.check(hip.lib().fh_conv2d_fwd(dtype, dx.value, dw.value, None, dy.value, hip.i64_array(geom), None, None))
+    got, exp = (synth.to_float(t, dtype) for t in (dy.download(want.shape, want.dtype), want))
+    ok = np.isfinite(exp)
+    assert 0 < ok[:, 3].sum() < ok[:, 3].size and np.array_equal(np.isfinite(got), ok)
+    assert np.array_equal(got[~ok], exp[~ok])  # infinities with their sign (no NaN: x > 0)
+    assert_close(synth.to_storage(got[ok], dtype), synth.to_storage(exp[ok], dtype), dtype, what="finite outputs")
+
+
 def test_conv2d_f32_outside_the_split_range(hip):
     # an image with an infinity, one with NaN, one of values below 2^-110 and one whose largest value rounds to a bf16
     # infinity: their results are the oracle's, the other images' are untouched

@@ -25,7 +25,7 @@ for p in (os.path.join(REPO, "frame-public_amd"), os.path.join(REPO, "tests")):
 import numpy as np  # noqa: E402
 
 PEAK_BF16_TFLOPS = 2516.6  # dense bf16 MFMA, 256 CU x 2.4 GHz x 4096 FLOP/clk/CU
-PEAK_F32_TFLOPS = PEAK_BF16_TFLOPS / 6  # fp32 products as six bf16 ones (fp32 MFMA itself: 157.3)
+PEAK_F32_TFLOPS = PEAK_BF16_TFLOPS / 8  # fp32 products as eight bf16 ones (fp32 MFMA itself: 157.3)
 PEAK_HBM_GBS = 8000.0
 GRAPH_SETTLE_MS = 200.0  # untimed wall time each secondary measurement runs before its timed region
 

@@ -200,8 +200,17 @@ struct Im2col : Operand<T, BN, BK, NT, false> {
   }
 };
 
+// Waves per SIMD, as min_waves; a gather of fp32 pixels needs more registers than three leave (stride 2, [32,64,56,56] to
+// 128 channels: 80 us with them, 57 without).
+template <typename T, int WAVES, int LDS, int RUNS>
+constexpr int conv_waves() {
+  return RUNS == kGather ? 1 : min_waves<T, WAVES, LDS>();
+}
+
 template <typename T, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int RUNS, int E>
-__global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void conv_any_kernel(ConvAnyArgs g) {
+__global__ __launch_bounds__(WAVES_M* WAVES_N * 64,
+                             (conv_waves<T, WAVES_M * WAVES_N, (BM + BN) * BK * 4 * AnyTraits<T>::P, RUNS>())) void
+conv_any_kernel(ConvAnyArgs g) {
   using S = typename Io<T>::storage;
   constexpr int NT = WAVES_M * WAVES_N * 64;
   constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
@@ -242,12 +251,10 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void conv_any_kernel(ConvAny
       b.template load<SET>(g, kt);
     }
   };
-  f32x4_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  k_loop<T, OpA, OpB, BK>(a, b, lds, KT, whole, wm * WM, wn * WN, lane, whole_load, any_load, tiny, acc);
+  f32x4_t sums[AnyTraits<T>::Q][TM][TN];
+  clear(sums);
+  k_loop<T, OpA, OpB, BK>(a, b, lds, KT, whole, wm * WM, wn * WN, lane, whole_load, any_load, tiny, sums);
+  f32x4_t(&acc)[TM][TN] = total(sums);
 
   const int q = lane >> 4, r = lane & 15;
   // Results that are not finite (and fp32 operands below the split's range) are taken again one product at a time, in the

@@ -147,14 +147,12 @@ __global__ __launch_bounds__(kWThreads) void conv_wgrad_kernel(WgradArgs a) {
     ob.template load<SET>(p0, X, x_at);
   };
 
-  f32x4_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4_t sums[1][TM][TN];
+  gemm_any::clear(sums);
   const int32_t steps = (p_end - p_begin + kWK - 1) / kWK;
   uint32_t unused = 0;
-  gemm_any::k_loop<T, OpA, OpB, kWK>(oa, ob, lds, steps, steps, wm * WM, wn * WN, lane, load, load, unused, acc);
+  gemm_any::k_loop<T, OpA, OpB, kWK>(oa, ob, lds, steps, steps, wm * WM, wn * WN, lane, load, load, unused, sums);
+  const f32x4_t(&acc)[TM][TN] = sums[0];
 
   // fp32 partial tile
   float* out = a.part + static_cast<int64_t>(blockIdx.y) * a.cout * a.nc;

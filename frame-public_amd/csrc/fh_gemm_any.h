@@ -15,12 +15,18 @@
 // LDS transpose read ds_read_b64_tr_b16: neither needs a transposed copy.
 //
 // fp32 operands are split on their way to LDS into three bf16 planes, x = x1 + x2 + x3 (each the round-to-nearest bf16
-// of what the ones before it leave: 24 bits, exact for |x| >= 2^-110), and a product is the six plane products
-// x1 y1 + x1 y2 + x2 y1 + x2 y2 + x1 y3 + x3 y1 summed in fp32. The three left out are below 2^-26 of |x y| together, under
-// the rounding of a single fp32 product. The bf16 matrix rate is 16 times the fp32 one, so six products take 6/16 of
-// the time. Operands outside the split's range (an infinity or NaN, a finite value that rounds to a bf16 infinity, a
-// nonzero value below 2^-110) send the tile to plain fp32 MFMA after the loop: the first two make the accumulators
-// non-finite, the third is tracked while splitting.
+// of what the ones before it leave: 24 bits, exact for |x| >= 2^-110), and a product is the eight plane products
+// x1 y1 + x1 y2 + x2 y1 + x2 y2 + x1 y3 + x3 y1 + x2 y3 + x3 y2. With |x2| <= 2^-8 and |x3| <= 2^-17 of x's power of two,
+// the one left out is at most 2^-34 of |x y|; without the last two it would be 2^-24, as much again as a product's own
+// rounding (and of one sign where an operand repeats). The instruction does not round to nearest when it adds to its
+// accumulator, so x1 y1, whose 16 bits rarely meet the end of the sum, has an accumulator of its own and the small terms
+// another, added up once. Error against float64 (fp32 MFMA before; one accumulator and six products): N(0,1), K 4096
+// 4.0e-7 (1.1e-6; 1.0e-6 with a bias of -2.7e-7), U(0,1), K 4096 3.0e-7 (8.5e-7; 5.3e-7), U(-1,1), K 1 2.5e-8 (2.5e-8;
+// 3.1e-8), equal operands, K 4096 5.9e-8 (5.9e-8; 3.8e-6). The bf16 matrix rate is 16 times the fp32 one, so
+// eight products take half of the time (2048^3: 109 us; 92 with six in one accumulator, 187 on fp32 MFMA). Operands outside
+// the split's range (an infinity or NaN, a finite value that rounds to a bf16 infinity, a nonzero value below 2^-110) send
+// the tile to plain fp32 MFMA after the loop: the first two make the accumulators non-finite, the third is tracked while
+// splitting.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -43,11 +49,13 @@ typedef short s16x4_t __attribute__((ext_vector_type(4)));
 template <typename T>
 struct AnyTraits {
   static constexpr int P = 1;  // planes in LDS
+  static constexpr int Q = 1;  // accumulators per output
   using mfma_t = T;
 };
 template <>
 struct AnyTraits<float> {
   static constexpr int P = 3;
+  static constexpr int Q = 2;  // x1 y1, and the small terms
   using mfma_t = bf16_t;
 };
 
@@ -199,15 +207,36 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+template <int Q, int TM, int TN>
+__device__ __forceinline__ void clear(f32x4_t (&sums)[Q][TM][TN]) {
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) sums[q][i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+}
+// The accumulators of each output added up, in the first of them.
+template <int Q, int TM, int TN>
+__device__ __forceinline__ auto total(f32x4_t (&sums)[Q][TM][TN]) -> f32x4_t (&)[TM][TN] {
+#pragma unroll
+  for (int q = 1; q < Q; ++q)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) sums[0][i][j] += sums[q][i][j];
+  return sums[0];
+}
+
 // The k loop of one tile: KT steps of BK. whole_load<SET>(kt) issues the loads of tile kt < whole into register set SET,
 // any_load<SET>(kt) those of any tile (nothing from KT on). Step kt: loads of kt + 2 into the set that tile kt left,
 // products of kt, LDS writes of kt + 1, barrier. The main loop has no branch: where a path might have left a load of the
 // same registers in flight, the compiler waits for every load before issuing the next (4095^3 bf16: 278 us against 180).
-// (Spreading the LDS writes between the products in fixed order was slower for fp32: 98 us against 94 at 2048^3.)
+// (Spreading the LDS writes between the products in fixed order was slower for fp32.)
 template <typename T, typename OpA, typename OpB, int BK, int TM, int TN, typename Whole, typename Any>
 __device__ __forceinline__ void k_loop(OpA& a, OpB& b, unsigned char* lds, int KT, int whole, int m_off, int n_off,
                                        int lane, Whole&& whole_load, Any&& any_load, uint32_t& tiny,
-                                       f32x4_t (&acc)[TM][TN]) {
+                                       f32x4_t (&acc)[AnyTraits<T>::Q][TM][TN]) {
   constexpr bool F32 = std::is_same_v<T, float>;
   constexpr int P = AnyTraits<T>::P;
   constexpr int BUF = OpA::BYTES + OpB::BYTES;
@@ -233,9 +262,11 @@ __device__ __forceinline__ void k_loop(OpA& a, OpB& b, unsigned char* lds, int K
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j) mfma16x<M16>(fa[PA][i], fb[PB][j], acc[i][j]);
+          for (int j = 0; j < TN; ++j) mfma16x<M16>(fa[PA][i], fb[PB][j], acc[PA + PB > 0][i][j]);
       };
-      if constexpr (F32) {  // small terms first: a short sum then rounds once at its full size
+      if constexpr (F32) {
+        pair.template operator()<2, 1>();
+        pair.template operator()<1, 2>();
         pair.template operator()<2, 0>();
         pair.template operator()<0, 2>();
         pair.template operator()<1, 1>();
@@ -291,13 +322,17 @@ __device__ __forceinline__ bool outside_split(int* tiny_seen, uint32_t tiny, con
 
 // Waves per SIMD a kernel is compiled for: two workgroups of eight waves share a CU's 16-bit LDS buffers, which 128
 // registers per lane allow and 130 (the compiler's own choice at 128x128x64) do not: 4095^3 bf16 181 us against 206.
-template <typename T, int WAVES>
+// Three workgroups of four waves share its fp32 buffers at 64x64x32.
+template <typename T, int WAVES, int LDS>
 constexpr int min_waves() {
-  return std::is_same_v<T, float> || WAVES < 8 ? 1 : 4;
+  if (std::is_same_v<T, float>) return WAVES < 8 && 3 * LDS <= 160 * 1024 ? 3 : 1;
+  return WAVES < 8 ? 1 : 4;
 }
 
 template <typename T, int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool TA, bool TB, int E>
-__global__ __launch_bounds__(WAVES_M* WAVES_N * 64, (min_waves<T, WAVES_M * WAVES_N>())) void gemm_any_kernel(GemmArgs args) {
+__global__ __launch_bounds__(WAVES_M* WAVES_N * 64,
+                             (min_waves<T, WAVES_M * WAVES_N, (BM + BN) * BK * 4 * AnyTraits<T>::P>())) void
+gemm_any_kernel(GemmArgs args) {
   using S = typename Io<T>::storage;
   constexpr bool F32 = std::is_same_v<T, float>;
   constexpr int NT = WAVES_M * WAVES_N * 64;
@@ -355,13 +390,11 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64, (min_waves<T, WAVES_M * WAVE
       b.template load_tail<SET>(kt, K - static_cast<int64_t>(kt) * BK);
     }
   };
-  f32x4_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4_t sums[AnyTraits<T>::Q][TM][TN];
+  clear(sums);
 
-  k_loop<T, OpA, OpB, BK>(a, b, lds, KT, whole, wm * WM, wn * WN, lane, whole_load, any_load, tiny, acc);
+  k_loop<T, OpA, OpB, BK>(a, b, lds, KT, whole, wm * WM, wn * WN, lane, whole_load, any_load, tiny, sums);
+  f32x4_t(&acc)[TM][TN] = total(sums);
 
   const int g = lane >> 4, r = lane & 15;
   if constexpr (F32) {

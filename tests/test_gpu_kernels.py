@@ -213,6 +213,41 @@ def test_gemm_f32_error_against_float64(hip, k):
         assert rel <= 2.0 ** -24 * np.sqrt(k), rel
 
 
+def test_gemm_f32_single_products(hip):
+    # K = 1: every output is one product, x y in fp32. The operands are the mantissas whose second and third bf16 planes
+    # are largest, of either sign, and random ones. What three planes and eight plane products may lose next to the one
+    # rounding: a few sums of the small terms, each rounded at 2^-7 of the product (2^-7 of its half ulp), and x3 y3
+    # (2^-34); without x2 y3 and x3 y2 the worst pairs here are nearly two half ulps off
+    say("gemm f32 single products")
+    m = (np.arange(1 << 23, dtype=np.uint32) | np.uint32(0x3F800000)).view(np.float32)
+
+    def bf16(x):
+        u = x.view(np.uint32)
+        return ((u + np.uint32(0x7FFF) + ((u >> 16) & 1)) & np.uint32(0xFFFF0000)).view(np.float32)
+
+    x2 = bf16(m - bf16(m))
+    x3 = m - bf16(m) - x2
+    order = np.argsort(x2 * x3)
+    rng = np.random.default_rng(31)
+    x = np.concatenate([m[order[:160]], m[order[-160:]], rng.choice(m, 320, replace=False)])
+    a, b = np.ascontiguousarray(x[:, None]), np.ascontiguousarray(rng.permutation(x)[None, :])
+    want = a.astype(np.float64) * b.astype(np.float64)
+    err = np.abs(run_gemm(hip, F32, a, b) - want) / (np.spacing(want.astype(np.float32)) / 2)
+    assert err.max() <= 1 + 2.0 ** -5, err.max()
+
+
+def test_gemm_f32_equal_operands(hip):
+    # every product is the same: what planes lose, and what sums that are not rounded to nearest lose, has one sign over all
+    # of k. The small terms (2^-7 of the whole) are added 7 times per step of 32 k, each time at most an ulp (2^-23) off;
+    # then comes one rounding. (One accumulator for all products was 3.8e-6 off.)
+    k = 4096
+    say("gemm f32 equal operands")
+    v = np.float32(float.fromhex("0x1.00ff8p+0"))
+    got = run_gemm(hip, F32, np.full((640, k), v), np.full((k, 640), v))
+    want = k * float(v) ** 2
+    assert np.abs(got / want - 1).max() <= k / 32 * 7 * 2.0 ** -30 + 2.0 ** -24, np.abs(got / want - 1).max()
+
+
 def test_gemm_known_answer(hip):
     # reference: tests/cpp/ops/test_op_matmul.cpp:208-230 — [[1,2],[3,4]]·[[5,6],[7,8]] = [[19,22],[43,50]]
     a = np.array([[1, 2], [3, 4]], np.float32)

@@ -86,7 +86,7 @@ struct RowsOperand : gemm_any::Operand<T, COLS, kWK, kWThreads, false> {
     live[SET] = m;
   }
   template <int SET>
-  __device__ void store(unsigned char* lds, uint32_t&) {
+  __device__ void store(unsigned char* lds) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const bool on = (live[SET] >> u) & 1u;
@@ -150,8 +150,7 @@ __global__ __launch_bounds__(kWThreads) void conv_wgrad_kernel(WgradArgs a) {
   f32x4_t sums[1][TM][TN];
   gemm_any::clear(sums);
   const int32_t steps = (p_end - p_begin + kWK - 1) / kWK;
-  uint32_t unused = 0;
-  gemm_any::k_loop<T, OpA, OpB, kWK>(oa, ob, lds, steps, steps, wm * WM, wn * WN, lane, load, load, unused, sums);
+  gemm_any::k_loop<T, OpA, OpB, kWK>(oa, ob, lds, steps, steps, wm * WM, wn * WN, lane, load, load, sums);
   const f32x4_t(&acc)[TM][TN] = sums[0];
 
   // fp32 partial tile

@@ -14,8 +14,9 @@
 // ds_read_b128; one that is contiguous along m or n (A transposed, B as stored) lies as 32 k rows and is read with the
 // LDS transpose read ds_read_b64_tr_b16: neither needs a transposed copy.
 //
-// fp32 operands are split on their way to LDS into three bf16 planes, x = x1 + x2 + x3 (each the round-to-nearest bf16
-// of what the ones before it leave: 24 bits, exact for |x| >= 2^-110), and a product is the eight plane products
+// fp32 operands are scaled by 2^24 and split on their way to LDS into three bf16 planes, 2^24 x = x1 + x2 + x3 (each the
+// round-to-nearest bf16 of what the ones before it leave: all 24 bits of every |x| < 2^104, denormals included, in planes
+// that are no denormals themselves); the sum is scaled back by 2^-48. A product is the eight plane products
 // x1 y1 + x1 y2 + x2 y1 + x2 y2 + x1 y3 + x3 y1 + x2 y3 + x3 y2. With |x2| <= 2^-8 and |x3| <= 2^-17 of x's power of two,
 // the one left out is at most 2^-34 of |x y|; without the last two it would be 2^-24, as much again as a product's own
 // rounding (and of one sign where an operand repeats). The instruction does not round to nearest when it adds to its
@@ -23,10 +24,9 @@
 // another, added up once. Error against float64 (fp32 MFMA before; one accumulator and six products): N(0,1), K 4096
 // 4.0e-7 (1.1e-6; 1.0e-6 with a bias of -2.7e-7), U(0,1), K 4096 3.0e-7 (8.5e-7; 5.3e-7), U(-1,1), K 1 2.5e-8 (2.5e-8;
 // 3.1e-8), equal operands, K 4096 5.9e-8 (5.9e-8; 3.8e-6). The bf16 matrix rate is 16 times the fp32 one, so
-// eight products take half of the time (2048^3: 109 us; 92 with six in one accumulator, 187 on fp32 MFMA). Operands outside
-// the split's range (an infinity or NaN, a finite value that rounds to a bf16 infinity, a nonzero value below 2^-110) send
-// the tile to plain fp32 MFMA after the loop: the first two make the accumulators non-finite, the third is tracked while
-// splitting.
+// eight products take half of the time (2048^3: 109 us; 92 with six in one accumulator, 187 on fp32 MFMA). Infinities,
+// NaN, operands of 2^104 or more and sums of 2^80 or more make the accumulators non-finite: those outputs, and no others, are
+// taken again on fp32 MFMA after the loop (one NaN in an operand of 2048^3: 276 us).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -88,18 +88,16 @@ __device__ __forceinline__ Unit<T> load_unit_partial(const typename Io<T>::stora
   return u;
 }
 
-// 2^-110 as (bits << 1) - 1, the key that zero wraps to the top of.
-constexpr uint32_t kTinyKey = (static_cast<uint32_t>(127 - 110) << 24) - 1;
+constexpr float kSplitScale = 0x1p24f, kSplitUnscale = 0x1p-48f;
 
-// The unit's planes as packed 16-bit vectors. fp32: tracks the smallest key of its elements in `tiny`.
+// The unit's planes as packed 16-bit vectors.
 template <typename T>
-__device__ __forceinline__ void split_unit(const Unit<T>& u, u32x4_t (&plane)[AnyTraits<T>::P], uint32_t& tiny) {
+__device__ __forceinline__ void split_unit(const Unit<T>& u, u32x4_t (&plane)[AnyTraits<T>::P]) {
   if constexpr (std::is_same_v<T, float>) {
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
-      const uint32_t b0 = u.v[d / 2][2 * (d % 2)], b1 = u.v[d / 2][2 * (d % 2) + 1];
-      tiny = min(tiny, min((b0 << 1) - 1u, (b1 << 1) - 1u));
-      float x0 = __uint_as_float(b0), x1 = __uint_as_float(b1);
+      float x0 = __uint_as_float(u.v[d / 2][2 * (d % 2)]) * kSplitScale;
+      float x1 = __uint_as_float(u.v[d / 2][2 * (d % 2) + 1]) * kSplitScale;
 #pragma unroll
       for (int p = 0; p < 3; ++p) {
         const uint32_t w = store2<bf16_t>(x0, x1);
@@ -173,11 +171,11 @@ struct Operand {
     }
   }
   template <int SET>
-  __device__ void store(unsigned char* lds, uint32_t& tiny) {
+  __device__ void store(unsigned char* lds) {
 #pragma unroll
     for (int u = 0; u < UNITS; ++u) {
       u32x4_t plane[P];
-      split_unit<T>(reg[SET][u], plane, tiny);
+      split_unit<T>(reg[SET][u], plane);
 #pragma unroll
       for (int p = 0; p < P; ++p) *reinterpret_cast<u32x4_t*>(lds + p * PLANE + dst[u]) = plane[p];
     }
@@ -235,15 +233,14 @@ __device__ __forceinline__ auto total(f32x4_t (&sums)[Q][TM][TN]) -> f32x4_t (&)
 // (Spreading the LDS writes between the products in fixed order was slower for fp32.)
 template <typename T, typename OpA, typename OpB, int BK, int TM, int TN, typename Whole, typename Any>
 __device__ __forceinline__ void k_loop(OpA& a, OpB& b, unsigned char* lds, int KT, int whole, int m_off, int n_off,
-                                       int lane, Whole&& whole_load, Any&& any_load, uint32_t& tiny,
-                                       f32x4_t (&acc)[AnyTraits<T>::Q][TM][TN]) {
+                                       int lane, Whole&& whole_load, Any&& any_load, f32x4_t (&acc)[AnyTraits<T>::Q][TM][TN]) {
   constexpr bool F32 = std::is_same_v<T, float>;
   constexpr int P = AnyTraits<T>::P;
   constexpr int BUF = OpA::BYTES + OpB::BYTES;
   using M16 = typename AnyTraits<T>::mfma_t;
   auto store = [&]<int SET>(unsigned char* buf) {
-    a.template store<SET>(buf, tiny);
-    b.template store<SET>(buf + OpA::BYTES, tiny);
+    a.template store<SET>(buf);
+    b.template store<SET>(buf + OpA::BYTES);
   };
   auto products = [&](const unsigned char* buf) {
 #pragma unroll
@@ -304,20 +301,10 @@ __device__ __forceinline__ void k_loop(OpA& a, OpB& b, unsigned char* lds, int K
   }
 }
 
-// Whether this wave's fp32 tile has to be taken again on fp32 operands: an operand below the split's range, or a result
-// that is not finite.
-template <int TM, int TN>
-__device__ __forceinline__ bool outside_split(int* tiny_seen, uint32_t tiny, const f32x4_t (&acc)[TM][TN]) {
-  if (tiny < kTinyKey) *tiny_seen = 1;
-  __syncthreads();
-  bool bad = *tiny_seen != 0;
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int x = 0; x < 4; ++x) bad |= !(__builtin_fabsf(acc[i][j][x]) <= 3.4028234663852886e38f);
-  return __any(bad);
+__device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) <= 3.4028234663852886e38f; }
+// Whether the wave's 16x16 tile holds a result that is not finite (the same answer on every lane).
+__device__ __forceinline__ bool any_not_finite(const f32x4_t& acc) {
+  return __any(!(finite(acc[0]) && finite(acc[1]) && finite(acc[2]) && finite(acc[3])));
 }
 
 // Waves per SIMD a kernel is compiled for: two workgroups of eight waves share a CU's 16-bit LDS buffers, which 128
@@ -344,7 +331,6 @@ gemm_any_kernel(GemmArgs args) {
   constexpr int STAGED = WAVES_M * WAVES_N * WM * WN * static_cast<int>(sizeof(S));
   static_assert(STAGED <= 2 * BUF, "the wave tiles fit in the buffers");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * BUF];
-  __shared__ int tiny_seen;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -375,8 +361,6 @@ gemm_any_kernel(GemmArgs args) {
   OpB b;
   a.init(A, args.lda, m0, M, tid);
   b.init(B, args.ldb, n0, N, tid);
-  uint32_t tiny = ~0u;
-  if (F32 && tid == 0) tiny_seen = 0;
 
   auto whole_load = [&]<int SET>(int kt) {
     a.template load<SET>(kt);
@@ -393,35 +377,49 @@ gemm_any_kernel(GemmArgs args) {
   f32x4_t sums[AnyTraits<T>::Q][TM][TN];
   clear(sums);
 
-  k_loop<T, OpA, OpB, BK>(a, b, lds, KT, whole, wm * WM, wn * WN, lane, whole_load, any_load, tiny, sums);
+  k_loop<T, OpA, OpB, BK>(a, b, lds, KT, whole, wm * WM, wn * WN, lane, whole_load, any_load, sums);
   f32x4_t(&acc)[TM][TN] = total(sums);
 
   const int g = lane >> 4, r = lane & 15;
   if constexpr (F32) {
-    if (outside_split(&tiny_seen, tiny, acc)) {
-      // outside the split's range: this wave's tile again, on fp32 operands from memory
+    // the sums scaled back; those that are not finite again, on fp32 operands from memory, a row of 16x16 tiles at a time
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i) {
+      f32x4_t plain[TN];
+      bool again = false;
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-      for (int64_t k0 = 0; k0 < K; k0 += 4) {
-        const int64_t k = k0 + g;
-        float va[TM], vb[TN];
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const int64_t row = min(m0 + wm * WM + i * 16 + r, M - 1);
-          va[i] = k < K ? A[TA ? k * args.lda + row : row * args.lda + k] : 0.0f;
-        }
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const int64_t col = min(n0 + wn * WN + j * 16 + r, N - 1);
-          vb[j] = k < K ? B[TB ? col * args.ldb + k : k * args.ldb + col] : 0.0f;
-        }
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[i], vb[j], acc[i][j], 0, 0, 0);
+      for (int j = 0; j < TN; ++j) {
+        plain[j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        again |= any_not_finite(acc[i][j]);
       }
+      if (again) {
+        constexpr int U = 4;  // k4 steps whose loads are in flight together
+        const int64_t row = min(m0 + wm * WM + i * 16 + r, M - 1);
+        for (int64_t k0 = 0; k0 < K; k0 += 4 * U) {
+          float va[U], vb[U][TN];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int64_t k = min(k0 + 4 * u + g, K - 1);
+            va[u] = A[TA ? k * args.lda + row : row * args.lda + k];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+              const int64_t col = min(n0 + wn * WN + j * 16 + r, N - 1);
+              vb[u][j] = B[TB ? col * args.ldb + k : k * args.ldb + col];
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const bool live = k0 + 4 * u + g < K;
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+              plain[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(live ? va[u] : 0.0f, live ? vb[u][j] : 0.0f, plain[j], 0, 0, 0);
+          }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) acc[i][j][x] = finite(acc[i][j][x]) ? acc[i][j][x] * kSplitUnscale : plain[j][x];
     }
   }
 

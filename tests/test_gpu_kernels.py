@@ -248,6 +248,38 @@ def test_gemm_f32_equal_operands(hip):
     assert np.abs(got / want - 1).max() <= k / 32 * 7 * 2.0 ** -30 + 2.0 ** -24, np.abs(got / want - 1).max()
 
 
+@pytest.mark.parametrize("exponent", [-149, -140, -126, -118, -112, -109, -106, -103, 60, 100, 103])
+def test_gemm_f32_operands_at_every_scale(hip, exponent):
+    # operands down to single denormals keep all their bits, next to ordinary ones in the same rows, and so do those up to
+    # the largest that three planes hold: each output is no further from float64 than fp32 sums of 64 terms are
+    say(f"gemm f32 operands near 2^{exponent}")
+    k = 64
+    a = synth.tensor(32, (640, k), F32, "uniform").astype(np.float64) * 2.0 ** exponent
+    a = a.astype(np.float32)
+    a[300:, k // 2:] = synth.tensor(33, (340, k // 2), F32, "uniform")
+    b = synth.tensor(34, (k, 640), F32, "uniform")
+    b[: k // 2] *= np.float32(2.0 ** min(-exponent, 100) if exponent < 0 else 2.0 ** -40)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    got = run_gemm(hip, F32, a, b).astype(np.float64)
+    for rows in (slice(0, 300), slice(300, 640)):
+        rel = np.linalg.norm(got[rows] - want[rows]) / np.linalg.norm(want[rows])
+        assert rel <= 2.0 ** -24 * np.sqrt(k), (rows, rel)
+
+
+def test_gemm_f32_outputs_do_not_depend_on_their_neighbours(hip):
+    # whatever is elsewhere in the operands, an output is made from its own row and column alone, bit for bit
+    say("gemm f32 with tiny, infinite, NaN and huge operands in other rows and columns")
+    a, b = synth.tensor(35, (640, 200), F32, "uniform"), synth.tensor(36, (200, 520), F32, "uniform")
+    plain = run_gemm(hip, F32, a, b)
+    rows, cols = np.ones(640, bool), np.ones(520, bool)
+    for r, v in ((5, 1e-36), (130, np.inf), (300, np.nan), (511, 1e38), (630, 1e-45)):
+        a[r, r % 200], rows[r] = v, False
+    for c, v in ((7, 1e-36), (300, -np.inf)):
+        b[c % 200, c], cols[c] = v, False
+    got = run_gemm(hip, F32, a, b)
+    assert_bitwise(got[np.ix_(rows, cols)], plain[np.ix_(rows, cols)], "outputs of unchanged rows and columns")
+
+
 def test_gemm_known_answer(hip):
     # reference: tests/cpp/ops/test_op_matmul.cpp:208-230 — [[1,2],[3,4]]·[[5,6],[7,8]] = [[19,22],[43,50]]
     a = np.array([[1, 2], [3, 4]], np.float32)
@@ -822,6 +854,29 @@ def test_conv2d_f32_outside_the_split_range(hip):
     for i in range(6):
         ok = np.isfinite(want[i])
         assert_close(got[i][ok], want[i][ok], F32, what=f"image {i}")
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16, F16])
+@pytest.mark.parametrize("pad", [0, 1])
+def test_conv2d_outputs_do_not_depend_on_their_neighbours(hip, dtype, pad):
+    # an infinite, a NaN and a tiny filter value reach their own channels' outputs only, and such inputs their own image's
+    geom = (4, 5, 14, 14, 40, 3, 3, 1, 1, pad, pad, 1)
+    say(f"conv with special values in other channels and images dtype={dtype} pad={pad}")
+    x = synth.to_float(synth.tensor(112, geom[:4], dtype, "normal"), dtype).copy()
+    wt = synth.to_float(synth.tensor(113, (40, 5, 3, 3), dtype, "normal", 0.2), dtype).copy()
+    out = (4, 40, 12 + 2 * pad, 12 + 2 * pad)
+
+    def run():
+        dx, dw = dev(hip, synth.to_storage(x, dtype)), dev(hip, synth.to_storage(wt, dtype))
+        dy = hip.DeviceBuffer(int(np.prod(out)) * (4 if dtype == F32 else 2))
+        hip.check(hip.lib().fh_conv2d_fwd(dtype, dx.value, dw.value, None, dy.value, hip.i64_array(geom), None, None))
+        return dy.download(out, hip.storage_dtype(dtype))
+
+    plain = run()
+    wt[3, 2, 0, 0], wt[17, 0, 1, 1], wt[30, 4, 2, 2] = np.inf, np.nan, 1e-36 if dtype != F16 else 6e-8
+    x[2, 1, 5, 5], x[3, 4, 13, 0] = np.nan, 1e-36 if dtype != F16 else 6e-8
+    keep = np.setdiff1d(np.arange(40), [3, 17, 30])
+    assert_bitwise(run()[:2][:, keep], plain[:2][:, keep], "outputs of unchanged channels and images")
 
 
 # paths: whole planes through LDS (rows * cols <= 8192: filters), 16-byte tiles (16-bit, rows and cols multiples

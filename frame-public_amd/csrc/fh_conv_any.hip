@@ -198,6 +198,8 @@ struct Im2col : Operand<T, BN, BK, NT, false> {
       for (int p = 0; p < Base::P; ++p) *reinterpret_cast<u32x4_t*>(lds + p * Base::PLANE + this->dst[n]) = plane[p];
     }
   }
+  template <int SET>
+  __device__ void store_any(unsigned char* lds) { store<SET>(lds); }
 };
 
 // Waves per SIMD, as min_waves; a gather of fp32 pixels needs more registers than three leave (stride 2, [32,64,56,56] to
@@ -232,7 +234,7 @@ conv_any_kernel(ConvAnyArgs g) {
 
   OpA a;
   OpB b;
-  a.init(static_cast<const S*>(g.w), g.k, m0, g.cout, tid);
+  a.init(static_cast<const S*>(g.w), g.k, m0, g.cout, g.k, tid);
   b.init(g, n0, tid);
   const int KT = (g.k + BK - 1) / BK;
   const int whole = g.k % BK != 0 ? KT - 1 : KT;

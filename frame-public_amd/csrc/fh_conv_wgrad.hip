@@ -96,6 +96,8 @@ struct RowsOperand : gemm_any::Operand<T, COLS, kWK, kWThreads, false> {
       *reinterpret_cast<u32x4_t*>(lds + this->dst[u]) = v;
     }
   }
+  template <int SET>
+  __device__ void store_any(unsigned char* lds) { store<SET>(lds); }
 };
 
 template <typename T, int kWM>

@@ -218,6 +218,13 @@ fh_status dispatch_gemm(GemmArgs args, int64_t batch, hipStream_t stream) {
   // A transposed operand in any order: the sequential kernel takes 3 us + 35 ns per k, the MFMA kernels 3.5 us + 10 ns per
   // k on few tiles (64x512x1000 bf16, B transposed: 40 us against 14)
   const bool long_k = args.any_order && (args.trans_a || args.trans_b) && args.K >= 128;
+  // 16-bit operands that are not whole vectors and little work: the sequential kernel takes 3 us + 20 ns per k + (0.3 us + 5
+  // ns per k) for every 65,536 outputs, an MFMA tile of any alignment 4.3-5 us at the least (bf16 2001x20x101 3.7 us against
+  // 5.1, 4001x33x47 4.3 / 5.4, 600x33x333 4.2 / 4.7; past the line 1501x64x131 4.9 / 4.4, 511x63x513 7.2 / 5.0, 300x264x200
+  // 9.6 / 5.5). fp32 stays on the planes, which are closer to the exact sum than fp32 sums in order are.
+  const double outputs = static_cast<double>(args.M) * static_cast<double>((args.N + 15) / 16 * 16) * batch;
+  const bool little = !std::is_same_v<T, float> && !args.trans_a && !args.trans_b && args.K <= 64 &&
+                      outputs / 65536 * (0.3 + 0.005 * static_cast<double>(args.K)) <= 1.7;
   // everything else on the matrix cores: 16-bit operands of whole 16-byte vectors on the aligned pipeline, the rest on
   // the kernel of any size and alignment
   fh_status st = FH_OK;
@@ -227,7 +234,7 @@ fh_status dispatch_gemm(GemmArgs args, int64_t batch, hipStream_t stream) {
     } else {
       const int32_t dtype = std::is_same_v<T, bf16_t> ? FH_BF16 : FH_F16;
       if (!args.trans_a && !args.trans_b && gemm16_try_launch(dtype, args, batch, stream, &st)) return st;
-      if (gemm_any16_try_launch(dtype, args, batch, stream, &st)) return st;
+      if (!little && gemm_any16_try_launch(dtype, args, batch, stream, &st)) return st;
     }
   }
   const bool split_ok = args.any_order && !args.trans_a && !args.trans_b &&

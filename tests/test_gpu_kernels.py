@@ -101,7 +101,8 @@ def test_gemm_small_bit_exact(hip, dtype, shape):
 # than, equal to and just past a step of 32 and 64 k, one row or column left over, N of one vector and one element more.
 # A, B, C and the epilogue operand start one element into their buffers, and the elements around C stay as they were.
 ANY_SHAPES = [(257, 31, 1025), (1024, 1, 1024), (513, 33, 520), (1030, 64, 8), (1030, 65, 9), (513, 129, 511),
-              (1111, 97, 1001), (1025, 63, 2049), (2100, 32, 2051), (65, 777, 4097)]
+              (1111, 97, 1001), (1025, 63, 2049), (2100, 32, 2051), (65, 777, 4097), (20011, 64, 8), (20011, 65, 9),
+              (20011, 70, 15), (2000, 40, 1024), (2000, 72, 1030), (7001, 7, 70)]
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16, F16])
@@ -129,6 +130,33 @@ def test_gemm_any_alignment(hip, dtype, shape):
             plain = got
         else:  # the fused program equals the separate one on the same product
             assert_bitwise(got, run_ew(hip, dtype, [1, 3], [2, 1], [plain, bias]), "epilogue vs separate program")
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("shape", [(2001, 20, 101), (4001, 33, 47), (600, 33, 333), (20001, 9, 11), (1000, 1, 401)])
+def test_gemm_little_work_bit_exact(hip, dtype, shape):
+    # little work on operands that are not whole vectors runs in the reference's order, past the few tiles that always do
+    m, k, n = shape
+    say(f"gemm little work dtype={dtype} m={m} k={k} n={n}")
+    a, b = synth.tensor(26, (m, k), dtype, "uniform"), synth.tensor(27, (k, n), dtype, "uniform")
+    assert_bitwise(run_gemm(hip, dtype, a, b), orc.matmul(dtype, a, b), f"little gemm {shape}")
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16, F16])
+def test_gemm_epilogue_operand_in_place(hip, dtype):
+    # C holds the epilogue's operand: every output reads its own before it is written, also where a row's last vector
+    # overlaps the one before it
+    for m, k, n in [(700, 50, 1001), (20011, 65, 9), (640, 100, 999)]:
+        say(f"gemm epilogue in place dtype={dtype} m={m} k={k} n={n}")
+        a, b = synth.tensor(28, (m, k), dtype, "uniform"), synth.tensor(29, (k, n), dtype, "uniform")
+        bias = synth.tensor(30, (m, n), dtype, "normal")
+        da, db, dc = dev(hip, a), dev(hip, b), dev(hip, bias)
+        plain = run_gemm(hip, dtype, a, b)
+        for op in (hip.EW_SQUARE, hip.EW_GELU):
+            dc.upload(bias)
+            ep = hip.make_epilogue([(hip.EW_ADD, dc.value), (op, None)])
+            hip.check(hip.lib().fh_gemm(dtype, da.value, db.value, dc.value, m, n, k, ctypes.byref(ep), None))
+            assert_bitwise(dc.download((m, n), a.dtype), run_ew(hip, dtype, [1, op], [2, 1], [plain, bias]), f"op {op}")
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])

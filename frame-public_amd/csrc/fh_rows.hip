@@ -8,12 +8,12 @@
 // softmax (reference: src/backends/cpu/kernels/sequence.cpp:114-174): m = max, e = exp(x - m), s = sum(e),
 // y = round(e / s). LayerNorm (reference: src/backends/cpu/kernels/sequence.cpp:182-279): two-pass mean and
 // variance, r = 1 / sqrt(var + eps), y = round(gamma * ((x - mean) * r) + beta). All arithmetic in fp32;
-// multiplies and adds are not contracted, division and sqrt are correctly rounded. For 16-bit outputs the softmax
-// of the register-resident kernels evaluates e as 2^((x - m) log2 e) on v_exp_f32 and y as round(e * (1 / s)): the
+// multiplies and adds are not contracted, division and sqrt are correctly rounded. For 16-bit rows of up to 2,048
+// elements softmax evaluates e as 2^((x - m) log2 e) on v_exp_f32 and y as round(e * (1 / s)): the
 // same d = x - m as the reference, an exponential within a few fp32 ulps of expf and a quotient within one, which
 // changes a stored 8- or 11-bit probability only where it lies that close to a rounding boundary. expf and the
 // correctly rounded division cost about 25 VALU instructions per element and made the [65536, 512] bf16 softmax
-// instruction-bound (30.7 us for 134 MB); fp32 outputs keep them.
+// instruction-bound (30.7 us for 134 MB); longer rows and fp32 keep them ([4096, 8192] f16 35.1 us, 23.9 without).
 #include <hip/hip_runtime.h>
 
 #include <string>
@@ -41,23 +41,28 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 constexpr int kRowsPerBlock = 4;  // 4 waves, one row each
 
-// softmax's e = exp(d) for d = x - m: expf for fp32 outputs, 2^(d log2 e) on v_exp_f32 for 16-bit ones
-template <typename T>
+// softmax's e = exp(d) for d = x - m: expf, or (FAST) 2^(d log2 e) on v_exp_f32
+template <bool FAST>
 __device__ __forceinline__ float softmax_exp(float d) {
-  if constexpr (std::is_same_v<T, float>) {
-    return expf(d);
-  } else {
+  if constexpr (FAST) {
     return __builtin_amdgcn_exp2f(d * 1.44269504088896340736f);
+  } else {
+    return expf(d);
   }
 }
-// y = e / s: correctly rounded for fp32 outputs, e * (1 / s) (r passed in) for 16-bit ones
-template <typename T>
+// y = e / s: correctly rounded, or (FAST) e * (1 / s) (r passed in)
+template <bool FAST>
 __device__ __forceinline__ float softmax_div(float e, float s, float r) {
-  if constexpr (std::is_same_v<T, float>) {
-    return e / s;
-  } else {
+  if constexpr (FAST) {
     return e * r;
+  } else {
+    return e / s;
   }
+}
+// 16-bit rows of up to 2,048 elements take the fast forms; longer ones and fp32 do not.
+template <typename T, int L>
+constexpr bool softmax_fast() {
+  return !std::is_same_v<T, float> && L <= 64;
 }
 
 // A row's 16-byte vectors over its L lanes (256 / L rows per workgroup): lane l holds the elements
@@ -68,7 +73,7 @@ __device__ __forceinline__ float softmax_div(float e, float s, float r) {
 // left out of the sums, and both lanes store them with the same value.
 // What bounds these kernels is HBM once the accesses are vectors (softmax bf16, us, one element per lane and access
 // before): [32768, 1000] 53.0 -> 23.6 (5.6 TB/s), [32768, 1001] 53.7 -> 26.4, [65536, 47] f32 12.7 -> 6.9; rows of
-// more than 2,048 elements, in three passes over memory before: [4096, 8192] f16 98 -> 24.
+// more than 2,048 elements, in three passes over memory before: [4096, 8192] f16 81 -> 35 (LayerNorm 64 -> 27).
 enum RowMode { kRowFull, kRowVectors, kRowRagged };
 
 template <int V, int NV, int L, int MODE>
@@ -146,6 +151,7 @@ __global__ __launch_bounds__(256) void softmax_row_kernel(const typename Io<T>::
                                                           typename Io<T>::storage* __restrict__ y, int64_t rows,
                                                           int64_t cols) {
   constexpr int V = 16 / static_cast<int>(sizeof(typename Io<T>::storage));
+  constexpr bool FAST = softmax_fast<T, L>();
   __shared__ float scratch[2][4];
   const int64_t row = static_cast<int64_t>(blockIdx.x) * (256 / L) + threadIdx.x / L;
   if (row >= rows) return;  // (whole row groups leave; with L = 256 every workgroup has its row)
@@ -173,7 +179,7 @@ __global__ __launch_bounds__(256) void softmax_row_kernel(const typename Io<T>::
   for (int t = 0; t < NV; ++t)
 #pragma unroll
     for (int i = 0; i < V; ++i) {
-      v[t][i] = softmax_exp<T>(v[t][i] - m);
+      v[t][i] = softmax_exp<FAST>(v[t][i] - m);
       s += rv.own(t, i) ? v[t][i] : 0.0f;
     }
   s = row_sum<L>(s, scratch[1]);
@@ -183,7 +189,7 @@ __global__ __launch_bounds__(256) void softmax_row_kernel(const typename Io<T>::
     if (!rv.has(t)) continue;
     float o[V];
 #pragma unroll
-    for (int i = 0; i < V; ++i) o[i] = softmax_div<T>(v[t][i], s, r);
+    for (int i = 0; i < V; ++i) o[i] = softmax_div<FAST>(v[t][i], s, r);
     row_store<T, MODE>(yr + rv.at[t], o);
   }
 }
@@ -198,9 +204,10 @@ __global__ __launch_bounds__(256) void softmax_short_kernel(const typename Io<T>
   if (row >= rows) return;
   const float v = (lane < cols) ? Io<T>::load(x[row * cols + lane]) : -__builtin_inff();
   const float m = wave_max((v > -__builtin_inff()) ? v : -__builtin_inff());
-  const float e = (lane < cols) ? softmax_exp<T>(v - m) : 0.0f;
+  constexpr bool FAST = softmax_fast<T, 64>();
+  const float e = (lane < cols) ? softmax_exp<FAST>(v - m) : 0.0f;
   const float s = wave_sum(e);
-  if (lane < cols) y[row * cols + lane] = Io<T>::store(softmax_div<T>(e, s, 1.0f / s));
+  if (lane < cols) y[row * cols + lane] = Io<T>::store(softmax_div<FAST>(e, s, 1.0f / s));
 }
 
 __device__ float block_reduce(float v, bool is_max, float* scratch) {

@@ -672,6 +672,25 @@ def test_row_kernel_widths(hip, op, dtype):
                      else None, what=f"{op} {rows}x{cols}")
 
 
+@pytest.mark.parametrize("cols", [2049, 4096, 16384])
+def test_softmax_long_16bit_rows_are_correctly_rounded(hip, cols):
+    # bf16 rows of more than 2,048 elements take expf and a correctly rounded division: next to float64 rounded once, an
+    # output differs only where it lies within about 2e-7 of a rounding boundary, and those are 2^-7 to 2^-8 apart: 7 in
+    # 100,000 (5 measured). 2^(d log2 e), off by up to 2e-6 at d = -80, differs in 8 to 15.
+    rows = (1 << 20) // cols
+    say(f"softmax bf16 {rows}x{cols} against float64")
+    x = -80.0 * np.abs(synth.to_float(synth.tensor(67, (rows, cols), F32, "uniform"), F32))
+    x[:, 0] = 0
+    x = synth.to_storage(x.astype(np.float32), BF16)
+    e = np.exp(synth.to_float(x, BF16).astype(np.float64))
+    want = synth.to_storage((e / e.sum(1, keepdims=True)).astype(np.float32), BF16)
+    dx, dy = dev(hip, x), hip.DeviceBuffer(x.nbytes)
+    hip.check(hip.lib().fh_softmax_rows(BF16, dx.value, dy.value, rows, cols, None))
+    differ = float(np.mean(dy.download(x.shape, x.dtype) != want))
+    print(f"  {differ:.2e} of the outputs differ")
+    assert differ <= 7e-5, differ
+
+
 # (BF16, 4096, 1024), (BF16, 5, 512), (F16, 9, 2048), (F32, 6, 256/1024/2048) take the 16-byte vector kernel
 @pytest.mark.parametrize("dtype,rows,cols", [(F32, 2, 5), (BF16, 4096, 1024), (F32, 3, 5000), (BF16, 7, 33),
                                              (BF16, 5, 512), (F16, 9, 2048), (F32, 6, 256), (F32, 6, 1024),

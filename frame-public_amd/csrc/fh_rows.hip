@@ -339,7 +339,9 @@ __global__ __launch_bounds__(256) void layer_norm_block_kernel(const typename Io
 
 // Lanes and vectors per row, for rows of at least one vector. The fewest of 8, 16, 32 or 64 lanes that hold the row as
 // one vector each, so that short rows share a wave; then 64 lanes of up to four vectors, then the whole workgroup of
-// 256, up to 64 values in a lane's registers. go<NV, L, MODE>() launches; false when the row does not fit.
+// 256, up to 64 values in a lane's registers. fp32 rows of 1,025 to 2,048 elements in whole vectors stay with one wave at
+// eight vectors, which needs no barrier ([4096, 2048] LayerNorm 9.1 us, 13.4 on 256 lanes; softmax 9.7 / 12.0); ragged ones do
+// not ([4096, 1999] LayerNorm 13.5 / 11.6). go<NV, L, MODE>() launches; false when the row does not fit.
 template <int V, typename Go>
 bool by_row_width(int64_t cols, Go&& go) {
   const int64_t vecs = (cols + V - 1) / V;
@@ -356,6 +358,7 @@ bool by_row_width(int64_t cols, Go&& go) {
   if (vecs <= 64) return pick.template operator()<1, 64>();
   if (vecs <= 128) return pick.template operator()<2, 64>();
   if (vecs <= 256) return pick.template operator()<4, 64>();
+  if (V == 4 && vecs <= 512 && cols % V == 0) return pick.template operator()<8, 64>();
   if (vecs <= 512) return pick.template operator()<2, 256>();
   if (vecs <= 1024) return pick.template operator()<4, 256>();
   if (vecs <= 2048) return pick.template operator()<8, 256>();

@@ -636,10 +636,10 @@ def test_softmax_known_answer(hip):
 
 
 # Widths around every change of lanes per row and vectors per lane (vectors of 8 16-bit or 4 fp32 elements): shorter than
-# one vector, whole and ragged vectors at 8 / 16 / 32 / 64 / 128 / 256 / 512 / 1024 / 2048 vectors, and past them. Row
+# one vector, whole and ragged vectors at 8 / 16 / 32 / 64 / 128 / 256 / 512 / 1024 / 2048 vectors, between and past them. Row
 # counts leave the last workgroup ragged; x and y start one element into their buffers, so no row is 16-byte aligned,
 # and the elements around y must stay as they were.
-ROW_VECS = [0, 1, 8, 16, 32, 64, 128, 256, 512, 1024, 2048]
+ROW_VECS = [0, 1, 8, 16, 32, 64, 128, 256, 257, 400, 511, 512, 1024, 2048]
 
 
 @pytest.mark.parametrize("op", ["softmax", "layer_norm"])

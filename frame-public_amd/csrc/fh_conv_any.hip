@@ -228,8 +228,10 @@ conv_any_kernel(ConvAnyArgs g) {
 
   // consecutive tiles on one XCD; the channel tiles of one pixel tile are neighbours, so its inputs are shared in L2
   const int tiles = g.tiles_m * g.tiles_n;
-  const int xcd = blockIdx.x & 7;
-  const int bid = xcd * (tiles >> 3) + min(xcd, tiles & 7) + static_cast<int>(blockIdx.x >> 3);
+  const int block = static_cast<int>(blockIdx.z * gridDim.x + blockIdx.x);  // (see tile_grid)
+  if (block >= tiles) return;
+  const int xcd = block & 7;
+  const int bid = xcd * (tiles >> 3) + min(xcd, tiles & 7) + (block >> 3);
   const int m0 = (bid % g.tiles_m) * BM, n0 = (bid / g.tiles_m) * BN;
 
   OpA a;
@@ -349,7 +351,7 @@ template <typename T, int BM, int BN, int BK, int WAVES_M, int WAVES_N>
 fh_status launch_conv(ConvAnyArgs g, int runs, hipStream_t stream) {
   g.tiles_m = (g.cout + BM - 1) / BM;
   g.tiles_n = (g.p + BN - 1) / BN;
-  const dim3 grid(static_cast<uint32_t>(g.tiles_m) * static_cast<uint32_t>(g.tiles_n));
+  const dim3 grid = tile_grid(static_cast<int64_t>(g.tiles_m) * g.tiles_n, 1);
   auto go = [&]<int RUNS, int E>() {
     hipLaunchKernelGGL((conv_any_kernel<T, BM, BN, BK, WAVES_M, WAVES_N, RUNS, E>), grid, dim3(WAVES_M * WAVES_N * 64), 0,
                        stream, g);
@@ -387,7 +389,7 @@ bool conv_any_try_launch(int32_t dtype, const void* x, const void* w, const void
       c.sw > 32767 || (c.oh * c.sh + c.ph + c.kh) * (c.w + c.pw + c.kw) > kMax)
     return false;
   const int64_t tiles = ((c.cout + 63) / 64) * ((pixels + 63) / 64);
-  if (tiles > 0x7fffffff) return false;
+  if (tiles > (int64_t{1} << 30)) return false;
   auto magic = [](int64_t d) { return d == 1 ? 0u : static_cast<uint32_t>(((int64_t{1} << 32) + d - 1) / d); };
   auto i32 = [](int64_t v) { return static_cast<int32_t>(v); };
   ConvAnyArgs g{x,        w,        bias,     y,        i32(c.cin), i32(c.h),  i32(c.w),  i32(c.cout), i32(c.kh),

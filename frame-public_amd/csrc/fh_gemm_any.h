@@ -32,6 +32,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -374,8 +375,10 @@ gemm_any_kernel(GemmArgs args) {
 
   // tile id: consecutive tiles on one XCD (any tile count), in groups of 8 tile rows
   const int tiles = args.tiles_m * args.tiles_n;
-  const int xcd = blockIdx.x & 7;
-  int bid = xcd * (tiles >> 3) + min(xcd, tiles & 7) + static_cast<int>(blockIdx.x >> 3);
+  const int block = static_cast<int>(blockIdx.z * gridDim.x + blockIdx.x);  // (see tile_grid)
+  if (block >= tiles) return;
+  const int xcd = block & 7;
+  const int bid = xcd * (tiles >> 3) + min(xcd, tiles & 7) + (block >> 3);
   constexpr int GROUP_M = 8;
   const int group = bid / (GROUP_M * args.tiles_n);
   const int gsize = min(args.tiles_m - group * GROUP_M, GROUP_M);
@@ -507,12 +510,18 @@ gemm_any_kernel(GemmArgs args) {
   }
 }
 
+// The grid of `tiles` workgroups: a launch holds fewer than 2^32 work items along x, so more than 2^22 workgroups (of up to
+// 512) go along z as well.
+inline dim3 tile_grid(int64_t tiles, int64_t batch) {
+  const int64_t x = std::min<int64_t>(tiles, int64_t{1} << 22);
+  return dim3(static_cast<uint32_t>(x), static_cast<uint32_t>(batch), static_cast<uint32_t>((tiles + x - 1) / x));
+}
+
 template <typename T, int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool TA, bool TB>
 fh_status launch(GemmArgs args, int64_t batch, hipStream_t stream) {
   args.tiles_m = static_cast<int32_t>((args.M + BM - 1) / BM);
   args.tiles_n = static_cast<int32_t>((args.N + BN - 1) / BN);
-  const dim3 grid(static_cast<uint32_t>(args.tiles_m) * static_cast<uint32_t>(args.tiles_n),
-                  static_cast<uint32_t>(batch));
+  const dim3 grid = tile_grid(static_cast<int64_t>(args.tiles_m) * args.tiles_n, batch);
   auto go = [&]<int E>() {
     hipLaunchKernelGGL((gemm_any_kernel<T, BM, BN, BK, WAVES_M, WAVES_N, TA, TB, E>), grid,
                        dim3(WAVES_M * WAVES_N * 64), 0, stream, args);
@@ -540,8 +549,8 @@ inline bool accepts(const GemmArgs& args, int64_t batch) {
   if (args.K < 0 || args.groups > 0 || args.row_softmax || batch > 65535) return false;  // (K = 0: zeros)
   if (args.trans_a ? args.M < 8 : false) return false;
   if (args.trans_b ? false : args.N < 8) return false;
-  const int64_t tiles = ((args.M + 63) / 64) * ((args.N + 63) / 64);
-  return args.K <= (int64_t{1} << 30) && tiles <= 0x7fffffff;
+  const int64_t tiles = ((args.M + 31) / 32) * ((args.N + 63) / 64);
+  return args.K <= (int64_t{1} << 30) && tiles <= (int64_t{1} << 30);
 }
 
 }  // namespace gemm_any

@@ -926,6 +926,51 @@ def test_conv2d_outputs_do_not_depend_on_their_neighbours(hip, dtype, pad):
     assert_bitwise(run()[:2][:, keep], plain[:2][:, keep], "outputs of unchanged channels and images")
 
 
+def fill(hip, buf, pattern):
+    """buf filled with copies of a pattern whose bytes divide its size, on the device."""
+    hip.check(hip.lib().fh_memcpy(buf.ptr, pattern.ctypes.data, pattern.nbytes, hip.H2D, None))
+    done = pattern.nbytes
+    while done < buf.nbytes:
+        n = min(done, buf.nbytes - done)
+        hip.check(hip.lib().fh_memcpy(ctypes.c_void_p(buf.value + done), buf.ptr, n, hip.D2D, None))
+        done += n
+
+
+def part(hip, buf, first, count):
+    out = np.empty(count, np.uint16)
+    hip.check(hip.lib().fh_memcpy(out.ctypes.data, ctypes.c_void_p(buf.value + 2 * first), out.nbytes, hip.D2H, None))
+    return out
+
+
+def test_conv2d_of_2e30_pixels(hip):
+    # 2^24 workgroups of 256: more work items than one dimension of a launch holds. One input channel, 1x1 filters c + 1
+    say("conv bf16 of 2^30 pixels to 16 channels")
+    plane, cout = 1 << 20, 16
+    pattern = synth.tensor(114, (plane,), BF16, "normal")
+    dx, dy = hip.DeviceBuffer(2 << 30), hip.DeviceBuffer((2 << 30) * cout)
+    fill(hip, dx, pattern)
+    dw = dev(hip, synth.to_storage(np.arange(1, cout + 1, dtype=np.float32), BF16))
+    geom = hip.i64_array((1024, 1, 1024, 1024, cout, 1, 1, 1, 1, 0, 0, 1))
+    hip.check(hip.lib().fh_conv2d_fwd(BF16, dx.value, dw.value, None, dy.value, geom, None, None))
+    x = synth.to_float(pattern, BF16)
+    for img, c in ((0, 0), (255, 15), (256, 1), (511, 7), (512, 3), (1023, 15)):
+        got = part(hip, dy, (img * cout + c) * plane, plane)
+        assert_bitwise(got, synth.to_storage(x * np.float32(c + 1), BF16), f"image {img} channel {c}")
+
+
+def test_gemm_of_2e30_rows(hip):
+    # 2^23 workgroups of 512, as above; 8 columns, 8 k
+    say("gemm bf16 of 2^30 rows")
+    rows, period = 1 << 30, 1 << 17
+    a, b = synth.tensor(115, (period, 8), BF16, "normal"), synth.tensor(116, (8, 8), BF16, "normal")
+    da, db, dc = hip.DeviceBuffer(16 * rows), dev(hip, b), hip.DeviceBuffer(16 * rows)
+    fill(hip, da, a)
+    hip.check(hip.lib().fh_gemm(BF16, da.value, db.value, dc.value, rows, 8, 8, None, None))
+    want = run_gemm(hip, BF16, a, b)
+    for first in (0, rows // 2 - period, rows // 2, rows - period):
+        assert_bitwise(part(hip, dc, first * 8, period * 8).reshape(period, 8), want, f"rows from {first}")
+
+
 # paths: whole planes through LDS (rows * cols <= 8192: filters), 16-byte tiles (16-bit, rows and cols multiples
 # of 8; full and partial tiles), element tiles (everything else, e.g. thin late-stage activations)
 @pytest.mark.parametrize("itemsize,shape", [(2, (3, 64, 3136)), (2, (2, 72, 200)), (2, (5, 70, 9)), (4, (2, 33, 130)),

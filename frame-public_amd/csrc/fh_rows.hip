@@ -341,9 +341,10 @@ __global__ __launch_bounds__(256) void layer_norm_block_kernel(const typename Io
 // one vector each, so that short rows share a wave; then 64 lanes of up to four vectors, then the whole workgroup of
 // 256, up to 64 values in a lane's registers. fp32 rows of 1,025 to 2,048 elements in whole vectors stay with one wave at
 // eight vectors, which needs no barrier ([4096, 2048] LayerNorm 9.1 us, 13.4 on 256 lanes; softmax 9.7 / 12.0); ragged ones do
-// not ([4096, 1999] LayerNorm 13.5 / 11.6). go<NV, L, MODE>() launches; false when the row does not fit.
+// not ([4096, 1999] LayerNorm 13.5 / 11.6) until there are 2^24 of them, a workgroup each and more than a launch holds.
+// go<NV, L, MODE>() launches; false when the row does not fit.
 template <int V, typename Go>
-bool by_row_width(int64_t cols, Go&& go) {
+bool by_row_width(int64_t rows, int64_t cols, Go&& go) {
   const int64_t vecs = (cols + V - 1) / V;
   const auto pick = [&]<int NV, int L>() {
     if (cols == int64_t{V} * NV * L) go.template operator()<NV, L, kRowFull>();
@@ -358,7 +359,7 @@ bool by_row_width(int64_t cols, Go&& go) {
   if (vecs <= 64) return pick.template operator()<1, 64>();
   if (vecs <= 128) return pick.template operator()<2, 64>();
   if (vecs <= 256) return pick.template operator()<4, 64>();
-  if (V == 4 && vecs <= 512 && cols % V == 0) return pick.template operator()<8, 64>();
+  if (V == 4 && vecs <= 512 && (cols % V == 0 || rows >= (int64_t{1} << 24))) return pick.template operator()<8, 64>();
   if (vecs <= 512) return pick.template operator()<2, 256>();
   if (vecs <= 1024) return pick.template operator()<4, 256>();
   if (vecs <= 2048) return pick.template operator()<8, 256>();
@@ -379,7 +380,7 @@ fh_status softmax_typed(const void* x, void* y, int64_t rows, int64_t cols, hipS
     hipLaunchKernelGGL((softmax_row_kernel<T, NV, L, MODE>), dim3(row_blocks(rows, L)), dim3(256), 0, s, xs, ys, rows,
                        cols);
   };
-  if (by_row_width<V>(cols, row_kernel)) return launch_status("softmax_row_kernel launch");
+  if (by_row_width<V>(rows, cols, row_kernel)) return launch_status("softmax_row_kernel launch");
   if (cols < V) {
     hipLaunchKernelGGL(softmax_short_kernel<T>, dim3(row_blocks(rows, 64)), dim3(256), 0, s, xs, ys, rows, cols);
     return launch_status("softmax_short_kernel launch");
@@ -400,7 +401,7 @@ fh_status layer_norm_typed(const void* x, const void* g, const void* b, void* y,
     hipLaunchKernelGGL((layer_norm_row_kernel<T, NV, L, MODE>), dim3(row_blocks(rows, L)), dim3(256), 0, s, xs, gs, bs,
                        ys, rows, cols, eps);
   };
-  if (by_row_width<V>(cols, row_kernel)) return launch_status("layer_norm_row_kernel launch");
+  if (by_row_width<V>(rows, cols, row_kernel)) return launch_status("layer_norm_row_kernel launch");
   if (cols < V) {
     hipLaunchKernelGGL(layer_norm_short_kernel<T>, dim3(row_blocks(rows, 64)), dim3(256), 0, s, xs, gs, bs, ys, rows,
                        cols, eps);

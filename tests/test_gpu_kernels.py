@@ -672,6 +672,38 @@ def test_row_kernel_widths(hip, op, dtype):
                      else None, what=f"{op} {rows}x{cols}")
 
 
+def fill(hip, buf, pattern):
+    """buf filled with copies of a pattern whose bytes divide its size, on the device."""
+    hip.check(hip.lib().fh_memcpy(buf.ptr, pattern.ctypes.data, pattern.nbytes, hip.H2D, None))
+    done = pattern.nbytes
+    while done < buf.nbytes:
+        n = min(done, buf.nbytes - done)
+        hip.check(hip.lib().fh_memcpy(ctypes.c_void_p(buf.value + done), buf.ptr, n, hip.D2D, None))
+        done += n
+
+
+def part(hip, buf, dtype, first, count):
+    out = np.empty(count, hip.storage_dtype(dtype))
+    hip.check(hip.lib().fh_memcpy(out.ctypes.data, ctypes.c_void_p(buf.value + out.itemsize * first), out.nbytes, hip.D2H,
+                                  None))
+    return out
+
+
+def test_layer_norm_of_2e24_ragged_rows(hip):
+    # a workgroup per row would be 2^32 work items, more than one dimension of a launch holds
+    rows, cols, period = 1 << 24, 1025, 1 << 10
+    say(f"layer_norm f32 {rows}x{cols}")
+    x = synth.tensor(68, (period, cols), F32, "normal")
+    g, b = synth.tensor(69, (cols,), F32, "normal"), synth.tensor(70, (cols,), F32, "normal")
+    dx, dy = hip.DeviceBuffer(rows * cols * 4), hip.DeviceBuffer(rows * cols * 4)
+    fill(hip, dx, x)
+    dg, db = dev(hip, g), dev(hip, b)
+    hip.check(hip.lib().fh_layer_norm_rows(F32, dx.value, dg.value, db.value, dy.value, rows, cols, 1e-5, None))
+    want = orc.layer_norm(F32, x, g, b, 1e-5)
+    for first in (0, rows // 4 - period, rows // 2, rows - period):
+        assert_close(part(hip, dy, F32, first * cols, period * cols).reshape(x.shape), want, F32, what=f"rows from {first}")
+
+
 @pytest.mark.parametrize("cols", [2049, 4096, 16384])
 def test_softmax_long_16bit_rows_are_correctly_rounded(hip, cols):
     # bf16 rows of more than 2,048 elements take expf and a correctly rounded division: next to float64 rounded once, an
@@ -926,22 +958,6 @@ def test_conv2d_outputs_do_not_depend_on_their_neighbours(hip, dtype, pad):
     assert_bitwise(run()[:2][:, keep], plain[:2][:, keep], "outputs of unchanged channels and images")
 
 
-def fill(hip, buf, pattern):
-    """buf filled with copies of a pattern whose bytes divide its size, on the device."""
-    hip.check(hip.lib().fh_memcpy(buf.ptr, pattern.ctypes.data, pattern.nbytes, hip.H2D, None))
-    done = pattern.nbytes
-    while done < buf.nbytes:
-        n = min(done, buf.nbytes - done)
-        hip.check(hip.lib().fh_memcpy(ctypes.c_void_p(buf.value + done), buf.ptr, n, hip.D2D, None))
-        done += n
-
-
-def part(hip, buf, first, count):
-    out = np.empty(count, np.uint16)
-    hip.check(hip.lib().fh_memcpy(out.ctypes.data, ctypes.c_void_p(buf.value + 2 * first), out.nbytes, hip.D2H, None))
-    return out
-
-
 def test_conv2d_of_2e30_pixels(hip):
     # 2^24 workgroups of 256: more work items than one dimension of a launch holds. One input channel, 1x1 filters c + 1
     say("conv bf16 of 2^30 pixels to 16 channels")
@@ -954,7 +970,7 @@ def test_conv2d_of_2e30_pixels(hip):
     hip.check(hip.lib().fh_conv2d_fwd(BF16, dx.value, dw.value, None, dy.value, geom, None, None))
     x = synth.to_float(pattern, BF16)
     for img, c in ((0, 0), (255, 15), (256, 1), (511, 7), (512, 3), (1023, 15)):
-        got = part(hip, dy, (img * cout + c) * plane, plane)
+        got = part(hip, dy, BF16, (img * cout + c) * plane, plane)
         assert_bitwise(got, synth.to_storage(x * np.float32(c + 1), BF16), f"image {img} channel {c}")
 
 
@@ -968,7 +984,7 @@ def test_gemm_of_2e30_rows(hip):
     hip.check(hip.lib().fh_gemm(BF16, da.value, db.value, dc.value, rows, 8, 8, None, None))
     want = run_gemm(hip, BF16, a, b)
     for first in (0, rows // 2 - period, rows // 2, rows - period):
-        assert_bitwise(part(hip, dc, first * 8, period * 8).reshape(period, 8), want, f"rows from {first}")
+        assert_bitwise(part(hip, dc, BF16, first * 8, period * 8).reshape(period, 8), want, f"rows from {first}")
 
 
 # paths: whole planes through LDS (rows * cols <= 8192: filters), 16-byte tiles (16-bit, rows and cols multiples

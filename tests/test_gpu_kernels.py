@@ -132,6 +132,19 @@ def test_gemm_any_alignment(hip, dtype, shape):
             assert_bitwise(got, run_ew(hip, dtype, [1, 3], [2, 1], [plain, bias]), "epilogue vs separate program")
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16, F16])
+@pytest.mark.parametrize("n", [1, 4, 7])
+def test_gemm_few_columns_of_many_rows(hip, dtype, n):
+    # more row tiles than a grid's y holds (1,048,560 rows), in the reference's order
+    m, k = 1048577 + 40, 20
+    say(f"gemm few columns dtype={dtype} m={m} k={k} n={n}")
+    a, b = synth.tensor(37, (m, k), dtype, "uniform"), synth.tensor(38, (k, n), dtype, "uniform")
+    want = orc.matmul(dtype, a, b)
+    assert_bitwise(run_gemm(hip, dtype, a, b), want, f"gemm {m}x{k}x{n}")
+    bias = synth.tensor(39, (m, n), dtype, "normal")
+    assert_bitwise(run_gemm(hip, dtype, a, b, [(hip.EW_ADD, bias)]), run_ew(hip, dtype, [1], [2], [want, bias]), "epilogue")
+
+
 @pytest.mark.parametrize("dtype", [BF16, F16])
 @pytest.mark.parametrize("shape", [(2001, 20, 101), (4001, 33, 47), (600, 33, 333), (20001, 9, 11), (1000, 1, 401)])
 def test_gemm_little_work_bit_exact(hip, dtype, shape):

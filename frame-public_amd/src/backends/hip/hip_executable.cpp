@@ -1738,7 +1738,9 @@ enum class MatmulGrad {
 // The tiled kernels take a gradient from the same size on as fh_gemm's dispatch on a 256-CU device does (fp32 from 64
 // tiles of 64 x 64, 16-bit from 16); at opt_level >= 1, where the k order is free, smaller ones with k >= 128 as well (the
 // sequential kernel spends 35 ns per k). Of these, large 16-bit ones of whole vectors are transposed: the aligned pipeline
-// makes up for the copy above about 2^30 multiplications (1024^3: 11.5 us in place, 7 + 4.5 us with the copy).
+// makes up for the copy above about 2^30 multiplications (1024^3: 11.5 us in place, 7 + 4.5 us with the copy). So are 16-bit
+// weight gradients of fewer than 8 input or output features, which nothing but the sequential kernel reads in place: 4 to
+// 1024 features over 65,536 rows 394 us with the copy, 2,770 in place, 256 to 4 2,450 / 2,920 (fp32 2,050 / 1,040).
 MatmulGrad plan_matmul_grad(const ir::Node* n, int32_t opt_level) {
   const bool lhs = n->op() == "matmul_grad_lhs_internal";
   if (!lhs && n->op() != "matmul_grad_rhs_internal") return MatmulGrad::kNone;
@@ -1749,6 +1751,8 @@ MatmulGrad plan_matmul_grad(const ir::Node* n, int32_t opt_level) {
   const bool f32 = n->inputs()[0]->type().dtype.code() == DTypeCode::kFloat32;
   const bool tiled = (f32 ? tiles64 >= 64 : tiles64 >= 16) || K > 16384;
   if (!tiled && !(opt_level >= 1 && K >= 128 && M >= 8 && N >= 8)) return MatmulGrad::kKeep;
+  // the in-place kernel takes a transposed A of 8 rows or more, and 8 columns
+  if (!f32 && !lhs && (M < 8 || N < 8)) return MatmulGrad::kTranspose;
   const bool vectors = K % 32 == 0 && N % 8 == 0 && N >= 64;
   const double work = static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(K);
   if (!f32 && vectors && tiled && work > static_cast<double>(int64_t{1} << 30)) return MatmulGrad::kTranspose;

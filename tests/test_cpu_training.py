@@ -438,3 +438,20 @@ def test_attention_gradients_lower_to_one_node(shape):
     g, shapes = graphs.transformer_block(batch=1, seq=40, d_model=128, heads=2, ffn=128, dtype=BF16, train=True)
     low = host.hip_lowered(host.backward(g.text(), 0, list(range(1, len(shapes) + 1))), 1)
     assert "hip_attention_grad_internal(" not in low and " softmax(" in low
+
+
+@pytest.mark.parametrize("features,out", [(4, 1024), (7, 1000), (256, 4), (1, 64)])
+@pytest.mark.parametrize("dtype", [BF16, graphs.F16, F32])
+def test_weight_gradients_of_few_features(features, out, dtype):
+    # nothing but the sequential kernel reads a transposed operand of fewer than 8 rows, or 8 columns, in place: in 16 bits
+    # such a gradient over many rows is a transposed copy and a plain matmul; with 8 of both, and in fp32, it is in place
+    def lowered(f, o):
+        g = graphs.Graph("hip")
+        a, gy = g.input(dtype, (65536, f)), g.input(dtype, (65536, o))
+        g.output(g.op("matmul_grad_rhs_internal", [a, gy], (f, o)))
+        return host.hip_lowered(g.text(), 1)
+
+    low = lowered(features, out)
+    assert (" transpose(" in low and " matmul(" in low) == (dtype != F32), low
+    assert ("transposed=1" in low) == (dtype == F32), low
+    assert "transposed=1" in lowered(8, 8)

@@ -873,6 +873,8 @@ CONV_ANY_CASES = [
     (1, 1, 1, 1, 1, 1, 1, 1, 1, 0, 0, 1),
     (1, 32, 5, 8, 16, 1, 1, 1, 1, 0, 0, 1),
     (4, 11, 8, 9, 100, 3, 3, 1, 1, 1, 1, 1),
+    (1, 1, 2, 2, 8, 5, 5, 1, 1, 2, 2, 1),
+    (1, 13, 1, 1, 9, 1, 1, 1, 1, 0, 0, 1),
 ]
 
 
@@ -904,6 +906,21 @@ def test_conv2d_any_geometry(hip, dtype, geom):
         else:
             ops, arities, ins = check
             assert_bitwise(got, run_ew(hip, dtype, ops, arities, [plain] + ins), "epilogue vs separate program")
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16, F16])
+@pytest.mark.parametrize("geom", [(4, 1, 200, 200, 1, 3, 3, 1, 1, 1, 1, 1), (2, 3, 301, 299, 2, 3, 3, 1, 1, 1, 1, 1),
+                                  (8, 1, 260, 250, 4, 3, 3, 2, 2, 1, 1, 1), (16, 2, 128, 128, 3, 1, 1, 1, 1, 0, 0, 1)])
+def test_conv2d_few_output_channels_bit_exact(hip, dtype, geom):
+    # few output channels of many pixels: one thread per output, in the reference's order
+    say(f"conv of few output channels dtype={dtype} {geom}")
+    x = synth.tensor(117, geom[:4], dtype, "normal")
+    wt = synth.tensor(118, (geom[4], geom[1], geom[5], geom[6]), dtype, "normal")
+    bias = synth.tensor(119, (geom[4],), dtype, "normal")
+    want = orc.conv2d(dtype, x, wt, bias, geom)
+    dx, dw, db, dy = dev(hip, x), dev(hip, wt), dev(hip, bias), hip.DeviceBuffer(want.nbytes)
+    hip.check(hip.lib().fh_conv2d_fwd(dtype, dx.value, dw.value, db.value, dy.value, hip.i64_array(geom), None, None))
+    assert_bitwise(dy.download(want.shape, want.dtype), want, f"conv {geom}")
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16, F16])

@@ -25,7 +25,8 @@ for p in (os.path.join(REPO, "frame-public_amd"), os.path.join(REPO, "tests")):
 import numpy as np  # noqa: E402
 
 PEAK_BF16_TFLOPS = 2516.6  # dense bf16 MFMA, 256 CU x 2.4 GHz x 4096 FLOP/clk/CU
-PEAK_F32_TFLOPS = PEAK_BF16_TFLOPS / 8  # fp32 products as eight bf16 ones (fp32 MFMA itself: 157.3)
+PEAK_F32_TFLOPS = PEAK_BF16_TFLOPS / 8  # fp32 products as eight bf16 ones
+PEAK_F32_MFMA_TFLOPS = 157.3  # the fp32 matrix instructions, for comparison
 PEAK_HBM_GBS = 8000.0
 GRAPH_SETTLE_MS = 200.0  # untimed wall time each secondary measurement runs before its timed region
 
@@ -247,19 +248,23 @@ def extras(steps, only=None):
                 "GB/s": round(by / (ms * 1e-3) / 1e9, 1), "frac_hbm": round(by / (ms * 1e-3) / 1e9 / PEAK_HBM_GBS, 4),
                 "copy_us": round(copy_ms * 1e3, 2)}
 
+    def mfma_fractions(tf, dtype):
+        # fp32 against both: the rate of the bf16 products it is made of, and the fp32 instructions that it does not use
+        if dtype == BF16:
+            return {"frac_mfma": round(tf / PEAK_BF16_TFLOPS, 4)}
+        return {"frac_mfma": round(tf / PEAK_F32_TFLOPS, 4), "frac_fp32_mfma": round(tf / PEAK_F32_MFMA_TFLOPS, 4)}
+
     def conv(dtype):
         flops = 2 * 32 * 64 * 56 * 56 * 64 * 9
         ms = _time_graph(graphs.conv(dtype).text(), [graphs.conv_inputs(dtype)], max(3, steps // 5), 2)
         tf = flops / (ms * 1e-3) / 1e12
-        peak = PEAK_BF16_TFLOPS if dtype == BF16 else PEAK_F32_TFLOPS
         return {"workload": f"C3 conv2d+bias+relu {'bf16' if dtype == BF16 else 'f32'} [32,64,56,56]*[64,64,3,3], whole compiled graph",
-                "us": round(ms * 1e3, 1), "TFLOP/s": round(tf, 1), "frac_mfma": round(tf / peak, 4)}
+                "us": round(ms * 1e3, 1), "TFLOP/s": round(tf, 1), **mfma_fractions(tf, dtype)}
 
     def gemm(n, dtype):
         ms = _time_graph(graphs.gemm(n, dtype).text(), [graphs.gemm_inputs(n, dtype)], max(10, steps // 2), 3)
         tf = gemm_flops(n, n, n) / (ms * 1e-3) / 1e12
-        peak = PEAK_BF16_TFLOPS if dtype == BF16 else PEAK_F32_TFLOPS
-        return {"TFLOP/s": round(tf, 1), "frac_mfma": round(tf / peak, 4), "us": round(ms * 1e3, 1)}
+        return {"TFLOP/s": round(tf, 1), **mfma_fractions(tf, dtype), "us": round(ms * 1e3, 1)}
 
     def mlp():
         ms = _time_graph(graphs.mlp(64, F32).text(), [graphs.mlp_inputs(64, F32)], max(50, steps), 10)

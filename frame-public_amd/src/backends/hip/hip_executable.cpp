@@ -1264,6 +1264,8 @@ Status lower_attention_grads(ir::Graph& g) {
   std::unordered_map<const ir::Value*, std::vector<const ir::Node*>> users;
   for (const ir::Node* n : order)
     for (const ir::Value* v : n->inputs()) users[v].push_back(n);
+  std::unordered_map<const ir::Node*, size_t> place;  // in the stored order
+  for (size_t i = 0; i < order.size(); ++i) place[order[i]] = i;
   std::vector<AttentionGradMatch> matches;
   std::unordered_map<const ir::Node*, size_t> roots;  // producers of the assembled gradients
   for (const ir::Node* n : order) {
@@ -1271,9 +1273,14 @@ Status lower_attention_grads(ir::Graph& g) {
     if (!m) continue;
     std::optional<AttentionGradMatch> grad = match_attention_grad(g, std::move(*m), users);
     if (!grad) continue;
-    bool fresh = true;
-    for (const ir::Value* v : grad->grads) fresh = fresh && !roots.count(v->producer());
-    if (!fresh) continue;
+    // the node stands at the first of the three values, where its operands have to be there already (dV does not need V)
+    bool fits = true;
+    for (const ir::Value* v : grad->grads) {
+      fits = fits && !roots.count(v->producer());
+      for (const ir::Value* x : {grad->fwd.q, grad->fwd.k, grad->fwd.v, grad->dout})
+        fits = fits && place.at(x->producer()) < place.at(v->producer());
+    }
+    if (!fits) continue;
     for (const ir::Value* v : grad->grads) roots[v->producer()] = matches.size();
     matches.push_back(std::move(*grad));
   }

@@ -455,3 +455,41 @@ def test_weight_gradients_of_few_features(features, out, dtype):
     assert (" transpose(" in low and " matmul(" in low) == (dtype != F32), low
     assert ("transposed=1" in low) == (dtype == F32), low
     assert "transposed=1" in lowered(8, 8)
+
+
+def test_attention_gradients_of_any_stored_order():
+    # dV needs P and the output gradient alone, so a graph may hold it before V: such a graph keeps its decomposition
+    batch, seq, heads = 1, 64, 2
+    d = 64 * heads
+
+    def block(v_late):
+        g = graphs.Graph("hip")
+        x, wv, dout = g.input(BF16, (seq, d)), g.input(BF16, (d, d)), g.input(BF16, (seq, d))
+        scale, minus = g.constant_splat(BF16, (seq, seq), 0.125), g.constant_splat(BF16, (seq, seq), -1.0)
+        ones, zeros = g.constant_splat(BF16, (1, seq), 1.0), g.constant_splat(BF16, (seq, 64), 0.0)
+        row = [None if v is None else g.slice(v, 0, 0, seq) for v in (x, dout)]
+        heads_of = lambda t: [g.slice(t, 1, 64 * h, 64 * h + 64) for h in range(heads)]
+        q, do = heads_of(row[0]), heads_of(row[1])
+        place = lambda v, h: g.concat([v, zeros] if h == 0 else [zeros, v], 1)
+        total = lambda parts: g.add(place(parts[0], 0), place(parts[1], 1))
+        kt = [g.transpose(k, (1, 0)) for k in q]
+        p = [g.softmax(g.mul(g.matmul(q[h], kt[h]), scale)) for h in range(heads)]
+        if not v_late:
+            v = heads_of(g.slice(g.matmul(x, wv), 0, 0, seq))
+        dv = total([g.op("matmul_grad_rhs_internal", [p[h], do[h]], (seq, 64)) for h in range(heads)])
+        if v_late:
+            v = heads_of(g.slice(g.matmul(x, wv), 0, 0, seq))
+        out = g.concat([g.concat([g.matmul(p[h], v[h]) for h in range(heads)], 1)], 0)
+        dq, dk = [], []
+        for h in range(heads):
+            dp = g.op("matmul_grad_lhs_internal", [do[h], v[h]], (seq, seq))
+            s = g.matmul(g.reshape(g.sum(g.mul(p[h], dp), [1]), (seq, 1)), ones)
+            ds = g.mul(g.mul(p[h], g.add(dp, g.mul(s, minus))), scale)
+            dq.append(g.op("matmul_grad_lhs_internal", [ds, kt[h]], (seq, 64)))
+            dk.append(g.transpose(g.op("matmul_grad_rhs_internal", [q[h], ds], (64, seq)), (1, 0)))
+        for o in (out, total(dq), total(dk), dv):
+            g.output(o)
+        return host.hip_lowered(g.text(), 1)
+
+    assert block(False).count("hip_attention_grad_internal(") == 1
+    assert "hip_attention_grad_internal(" not in block(True)

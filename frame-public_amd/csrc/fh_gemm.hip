@@ -228,7 +228,7 @@ fh_status dispatch_gemm(GemmArgs args, int64_t batch, hipStream_t stream) {
   const bool little = !std::is_same_v<T, float> && !args.trans_a && !args.trans_b && args.K <= 64 &&
                       outputs / 65536 * (0.3 + 0.005 * static_cast<double>(args.K)) <= 1.7;
   // everything else on the matrix cores: 16-bit operands of whole 16-byte vectors on the aligned pipeline, the rest on
-  // the kernel of any size and alignment
+  // the kernel of any alignment (8 columns or more, 8 rows of a transposed A)
   fh_status st = FH_OK;
   if ((!small || long_k) && !args.row_softmax) {
     if constexpr (std::is_same_v<T, float>) {

@@ -1,7 +1,8 @@
-// GEMM of any size and alignment, either operand transposed, for 16-bit and fp32 operands: C = op(A) · op(B) with fp32
-// accumulation on v_mfma_f32_16x16x32, one rounding per output, then the optional elementwise epilogue (semantics of
-// Frame's matmul and its gradients: reference src/backends/cpu/kernels/matmul.cpp:92-327). The kernel template; its
-// instances and their dispatch are in fh_gemm_any.hip (16-bit) and fh_gemm_f32.hip (fp32).
+// GEMM of any alignment, either operand transposed, for 16-bit and fp32 operands, of any size but the narrowest (an operand
+// contiguous along m or n needs 8 of them, see accepts): C = op(A) · op(B) with fp32 accumulation on v_mfma_f32_16x16x32,
+// one rounding per output, then the optional elementwise epilogue (semantics of Frame's matmul and its gradients: reference
+// src/backends/cpu/kernels/matmul.cpp:92-327). The kernel template; its instances and their dispatch are in
+// fh_gemm_any.hip (16-bit) and fh_gemm_f32.hip (fp32).
 //
 // Operands go global -> registers -> LDS in units of 8 elements along their contiguous index, so a unit needs element
 // alignment only (global memory takes 16-byte accesses at any alignment) and edges are handled per unit: rows past the

@@ -23,12 +23,14 @@ namespace {
 // no contraction, one rounding), so the result is bit-identical to it. K is staged through LDS in chunks of kKC as
 // fp32, A row-major and B transposed, both k-contiguous so each step reads 4 k-values per operand with one
 // 16-byte LDS read; the next chunk's global loads are in flight while the current one is consumed.
+// WAYS > 1 (FH_GEMM_ANY_ORDER): WAYS such groups of 256 threads sum a WAYS-th of every chunk each, added in their order at
+// the end. The chain of one sum, and the LDS latency before each 16 of its k, bound the kernel: 17 ns per k, 8 in four ways.
 constexpr int kSeqT = 16;   // output tile edge
 constexpr int kKC = 128;    // k per LDS chunk
 constexpr int kKP = kKC + 4;  // padded row: 16 consecutive B rows hit distinct 16-byte bank groups
 
-template <typename T>
-__global__ __launch_bounds__(256) void gemm_seq_kernel(GemmArgs args) {
+template <typename T, int WAYS>
+__global__ __launch_bounds__(256 * WAYS) void gemm_seq_kernel(GemmArgs args) {
   using S = typename Io<T>::storage;
   __shared__ __attribute__((aligned(16))) float As[2][kSeqT * kKP];
   __shared__ __attribute__((aligned(16))) float Bt[2][kSeqT * kKP];
@@ -37,28 +39,32 @@ __global__ __launch_bounds__(256) void gemm_seq_kernel(GemmArgs args) {
   S* __restrict__ C = static_cast<S*>(args.C) + blockIdx.z * args.stride_c;
   const int64_t m0 = static_cast<int64_t>(blockIdx.y) * kSeqT, n0 = static_cast<int64_t>(blockIdx.x) * kSeqT;
   const int64_t M = args.M, N = args.N, K = args.K;
-  const int t = threadIdx.x;
+  const int t = WAYS > 1 ? threadIdx.x & 255 : threadIdx.x;
+  const int way = WAYS > 1 ? threadIdx.x >> 8 : 0;
   const int r = t >> 4, c = t & 15;
 
   // chunk loads: A[16][kKC] and B[kKC][16], each with consecutive lanes on the operand's contiguous index: k for
   // row-major A and transposed B (thread -> row / column t/16, k t%16 + 16 i), the row or column otherwise
   // (thread -> k t/16 + 16 i, row / column t%16)
-  float la[8], lb[8];
+  constexpr int U = 8 / WAYS;
+  const int first = 16 * U * way;
+  float la[U], lb[U];
   const bool ta = args.trans_a != 0, tb = args.trans_b != 0;
   auto load_chunk = [&](int64_t k0) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int64_t gm = m0 + (ta ? c : r), gk = k0 + (ta ? r : c) + 16 * i;
+    for (int i = 0; i < U; ++i) {
+      const int64_t gm = m0 + (ta ? c : r), gk = k0 + first + (ta ? r : c) + 16 * i;
       la[i] = (gm < M && gk < K) ? Io<T>::load(A[ta ? gk * args.lda + gm : gm * args.lda + gk]) : 0.0f;
-      const int64_t bk = k0 + (tb ? c : r) + 16 * i, bn = n0 + (tb ? r : c);
+      const int64_t bk = k0 + first + (tb ? c : r) + 16 * i, bn = n0 + (tb ? r : c);
       lb[i] = (bk < K && bn < N) ? Io<T>::load(B[tb ? bn * args.ldb + bk : bk * args.ldb + bn]) : 0.0f;
     }
   };
   auto store_chunk = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      As[buf][ta ? c * kKP + r + 16 * i : r * kKP + c + 16 * i] = la[i];
-      Bt[buf][tb ? r * kKP + c + 16 * i : c * kKP + r + 16 * i] = lb[i];
+    for (int i = 0; i < U; ++i) {
+      const int k = first + 16 * i;
+      As[buf][ta ? c * kKP + r + k : r * kKP + c + k] = la[i];
+      Bt[buf][tb ? r * kKP + c + k : c * kKP + r + k] = lb[i];
     }
   };
 
@@ -72,10 +78,11 @@ __global__ __launch_bounds__(256) void gemm_seq_kernel(GemmArgs args) {
   for (int ch = 0; ch < chunks; ++ch) {
     const int buf = ch & 1;
     if (ch + 1 < chunks) load_chunk(static_cast<int64_t>(ch + 1) * kKC);
-    const int kn = static_cast<int>(min<int64_t>(kKC, K - static_cast<int64_t>(ch) * kKC));
+    int kn = static_cast<int>(min<int64_t>(kKC, K - static_cast<int64_t>(ch) * kKC));
+    if constexpr (WAYS > 1) kn = min(kn, (way + 1) * (kKC / WAYS));
     const float* ar = &As[buf][r * kKP];
     const float* br = &Bt[buf][c * kKP];
-    int kk = 0;
+    int kk = way * (kKC / WAYS);
     // 16 k per step: the four LDS reads of each operand are issued before the sum uses them, so one LDS latency
     // covers 16 k instead of 4 (the sum itself is the same chain, in the same order)
     for (; kk + 16 <= kn; kk += 16) {
@@ -104,6 +111,15 @@ __global__ __launch_bounds__(256) void gemm_seq_kernel(GemmArgs args) {
     for (; kk < kn; ++kk) acc = acc + ar[kk] * br[kk];
     if (ch + 1 < chunks) store_chunk(buf ^ 1);
     __syncthreads();
+  }
+  if constexpr (WAYS > 1) {  // (past the last chunk's barrier, or without a chunk, nothing else uses As)
+    float* part = &As[0][0];
+    static_assert((WAYS - 1) * 256 <= 2 * kSeqT * kKP, "the partial sums fit");
+    if (way > 0) part[(way - 1) * 256 + t] = acc;
+    __syncthreads();
+    if (way > 0) return;
+#pragma unroll
+    for (int w = 0; w < WAYS - 1; ++w) acc = acc + part[w * 256 + t];
   }
   const int64_t row = m0 + r, col = n0 + c;
   if (row < M && col < N) {
@@ -217,9 +233,15 @@ fh_status dispatch_gemm(GemmArgs args, int64_t batch, hipStream_t stream) {
   // to there: the C4 classifier, 16 tiles, 7.8 us there against 22 us sequential).
   const int64_t tiles64 = ((args.M + 63) / 64) * ((args.N + 63) / 64) * batch;
   const bool small = (std::is_same_v<T, float> ? tiles64 * 4 < cus : tiles64 < 16) && args.K <= 16384;
-  // A transposed operand in any order: the sequential kernel takes 3 us + 35 ns per k, the MFMA kernels 3.5 us + 10 ns per
-  // k on few tiles (64x512x1000 bf16, B transposed: 40 us against 14)
+  // A transposed operand in any order: the sequential kernel takes 3 us + 35 ns per k in 16 bits, the MFMA kernels 3.5 us +
+  // 10 ns per k on few tiles (64x512x1000 bf16, B transposed: 40 us against 14). In fp32 it takes 17 ns per k, 8 in four
+  // ways, while the planes' tiles take 23 with A transposed and 14 with B (256x1000x10 18.3 / 10.7 / 27.1 us, 17x3000x1000
+  // 53 / 28 / 70). With more than two workgroups per CU the tiles are ahead (500x1000x400 32 us in four ways, 27 on tiles),
+  // but for A transposed and k below 256, where two ways are (500x200x400 8.4 in order, 8.8, 9.5). The sums in ways are closer
+  // to the exact ones than those in order: 500x128x400 1.5e-7 (2.1e-7), 256x3000x10 5.0e-7 (9.5e-7).
   const bool long_k = args.any_order && (args.trans_a || args.trans_b) && args.K >= 128;
+  const double outputs16 = static_cast<double>((args.M + 15) / 16) * static_cast<double>((args.N + 15) / 16) * batch;
+  const bool planes = long_k && (!std::is_same_v<T, float> || (outputs16 > 2 * cus && (args.trans_b || args.K >= 256)));
   // 16-bit operands that are not whole vectors and little work: the sequential kernel takes 3 us + 20 ns per k + (0.3 us + 5
   // ns per k) for every 65,536 outputs, an MFMA tile of any alignment 4.3-5 us at the least (bf16 2001x20x101 3.7 us against
   // 5.1, 4001x33x47 4.3 / 5.4, 600x33x333 4.2 / 4.7; past the line 1501x64x131 4.9 / 4.4, 511x63x513 7.2 / 5.0, 300x264x200
@@ -230,7 +252,7 @@ fh_status dispatch_gemm(GemmArgs args, int64_t batch, hipStream_t stream) {
   // everything else on the matrix cores: 16-bit operands of whole 16-byte vectors on the aligned pipeline, the rest on
   // the kernel of any alignment (8 columns or more, 8 rows of a transposed A)
   fh_status st = FH_OK;
-  if ((!small || long_k) && !args.row_softmax) {
+  if ((!small || planes) && !args.row_softmax) {
     if constexpr (std::is_same_v<T, float>) {
       if (gemm_f32_try_launch(args, batch, stream, &st)) return st;
     } else {
@@ -262,7 +284,13 @@ fh_status dispatch_gemm(GemmArgs args, int64_t batch, hipStream_t stream) {
       if (ew_is_binary(args.ep.ops[s])) part.ep.ins[s] = static_cast<const S*>(args.ep.ins[s]) + m0 * args.ldc;
     const dim3 grid(static_cast<uint32_t>((part.N + kSeqT - 1) / kSeqT),
                     static_cast<uint32_t>((part.M + kSeqT - 1) / kSeqT), static_cast<uint32_t>(batch));
-    hipLaunchKernelGGL((gemm_seq_kernel<T>), grid, dim3(256), 0, stream, part);
+    if constexpr (std::is_same_v<T, float>) {
+      if (long_k && outputs16 <= 2 * cus) hipLaunchKernelGGL((gemm_seq_kernel<T, 4>), grid, dim3(1024), 0, stream, part);
+      else if (long_k) hipLaunchKernelGGL((gemm_seq_kernel<T, 2>), grid, dim3(512), 0, stream, part);
+      else hipLaunchKernelGGL((gemm_seq_kernel<T, 1>), grid, dim3(256), 0, stream, part);
+    } else {
+      hipLaunchKernelGGL((gemm_seq_kernel<T, 1>), grid, dim3(256), 0, stream, part);
+    }
     st = launch_status("gemm_seq_kernel launch");
     if (st != FH_OK) break;
   }
@@ -461,13 +489,13 @@ extern "C" fh_status fh_matmul_grad(int32_t dtype, int32_t rhs, const void* p, c
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (dtype) {
     case FH_F32:
-      hipLaunchKernelGGL((gemm_seq_kernel<float>), grid, dim3(256), 0, s, args);
+      hipLaunchKernelGGL((gemm_seq_kernel<float, 1>), grid, dim3(256), 0, s, args);
       break;
     case FH_BF16:
-      hipLaunchKernelGGL((gemm_seq_kernel<bf16_t>), grid, dim3(256), 0, s, args);
+      hipLaunchKernelGGL((gemm_seq_kernel<bf16_t, 1>), grid, dim3(256), 0, s, args);
       break;
     default:
-      hipLaunchKernelGGL((gemm_seq_kernel<f16_t>), grid, dim3(256), 0, s, args);
+      hipLaunchKernelGGL((gemm_seq_kernel<f16_t, 1>), grid, dim3(256), 0, s, args);
       break;
   }
   return launch_status("fh_matmul_grad");

@@ -1744,7 +1744,7 @@ enum class MatmulGrad {
 
 // The tiled kernels take a gradient from the same size on as fh_gemm's dispatch on a 256-CU device does (fp32 from 64
 // tiles of 64 x 64, 16-bit from 16); at opt_level >= 1, where the k order is free, smaller ones with k >= 128 as well (the
-// sequential kernel spends 35 ns per k). Of these, large 16-bit ones of whole vectors are transposed: the aligned pipeline
+// sequential kernel spends 35 ns per k in 16 bits; few fp32 outputs are summed in four ways). Of these, large 16-bit ones of whole vectors are transposed: the aligned pipeline
 // makes up for the copy above about 2^30 multiplications (1024^3: 11.5 us in place, 7 + 4.5 us with the copy). So are 16-bit
 // weight gradients of fewer than 8 input or output features, which nothing but the sequential kernel reads in place: 4 to
 // 1024 features over 65,536 rows 394 us with the copy, 2,770 in place, 256 to 4 2,450 / 2,920 (fp32 2,050 / 1,040).

@@ -211,6 +211,31 @@ def test_gemm_transposed_operand(hip, dtype, transposed):
         assert hip.lib().fh_gemm_transposed(dtype, bad, da.value, db.value, dc.value, m, n, k, None, 1, None) == 1
 
 
+@pytest.mark.parametrize("transposed,shape", [(t, s) for s in [(8, 128, 8), (17, 129, 31), (10, 200, 300), (257, 161, 33),
+                                                               (3, 300, 20), (40, 1000, 5)] for t in (1, 2)]
+                         + [(1, (500, 131, 400))])
+def test_gemm_f32_transposed_small_sum_order(hip, transposed, shape):
+    # few outputs, any order: four sums in order (two past 512 tiles of 16 x 16), each over its share of every 128 k, added in
+    # their order, bit for bit
+    m, k, n = shape
+    ways = 2 if m == 500 else 4
+    say(f"gemm f32 transposed={transposed} in {ways} ways m={m} k={k} n={n}")
+    a, b = synth.tensor(120, (m, k), F32, "uniform"), synth.tensor(121, (k, n), F32, "uniform")
+    bias = synth.tensor(122, (m, n), F32, "normal")
+    sums = np.zeros((ways, m, n), np.float32)
+    for i in range(k):
+        sums[i % 128 // (128 // ways)] += a[:, i:i + 1] * b[i:i + 1]
+    want = sums[0]
+    for part in sums[1:]:
+        want = want + part
+    da, db = dev(hip, a.T if transposed == 1 else a), dev(hip, b.T if transposed == 2 else b)
+    dbias, dc = dev(hip, bias), hip.DeviceBuffer(m * n * 4)
+    ep = hip.make_epilogue([(hip.EW_ADD, dbias.value)])
+    for program, expected in ((None, want), (ctypes.byref(ep), want + bias)):
+        hip.check(hip.lib().fh_gemm_transposed(F32, transposed, da.value, db.value, dc.value, m, n, k, program, 1, None))
+        assert_bitwise(dc.download((m, n), np.float32), expected, f"transposed {shape}")
+
+
 def test_gemm_f32_outside_the_split_range(hip):
     # operands that three bf16 planes do not hold: infinities, NaN, values that round to a bf16 infinity, and values
     # below 2^-110 (whole rows, so that the result is theirs). Rows without them keep their values next to them

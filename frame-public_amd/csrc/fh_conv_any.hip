@@ -376,6 +376,13 @@ fh_status launch_conv(ConvAnyArgs g, int runs, hipStream_t stream) {
 // 35 / 54, 21 / 113 / 28, 27 / 303 / 47).
 template <typename T>
 fh_status dispatch_conv(const ConvAnyArgs& g, int runs, hipStream_t stream) {
+  // fp32 with a tile per CU or less waits for its loads, splits and barriers in turn: half of the channels and twice the k
+  // between barriers take 0.6-0.75 us per k32 against 0.75-0.9 (one image of 512 channels, 14 x 14, 3x3 to 64: 130 us,
+  // 108 so; 106 channels-last on fp32 MFMA)
+  const int64_t tiles32 = ((g.cout + 31) / 32) * ((static_cast<int64_t>(g.p) + 63) / 64);
+  if constexpr (std::is_same_v<T, float>) {
+    if (tiles32 <= device_cu_count()) return launch_conv<T, 32, 64, 64, 2, 2>(g, runs, stream);
+  }
   return launch_conv<T, 64, 64, std::is_same_v<T, float> ? 32 : 64, 2, 2>(g, runs, stream);
 }
 

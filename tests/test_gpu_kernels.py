@@ -900,6 +900,10 @@ CONV_ANY_CASES = [
     (4, 11, 8, 9, 100, 3, 3, 1, 1, 1, 1, 1),
     (1, 1, 2, 2, 8, 5, 5, 1, 1, 2, 2, 1),
     (1, 13, 1, 1, 9, 1, 1, 1, 1, 0, 0, 1),
+    # more than a tile of 32 channels per CU (fp32: tiles of 64), each way its pixels lie
+    (9, 5, 47, 43, 70, 3, 3, 1, 1, 1, 1, 1),
+    (8, 5, 48, 48, 70, 3, 3, 1, 1, 1, 1, 1),
+    (16, 6, 65, 65, 40, 3, 3, 2, 2, 1, 1, 1),
 ]
 
 

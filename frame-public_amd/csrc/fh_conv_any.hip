@@ -387,15 +387,21 @@ fh_status dispatch_conv(const ConvAnyArgs& g, int runs, hipStream_t stream) {
 }
 
 // Whether one thread per output (conv2d_direct_kernel, in the reference's order) is done first: with few output channels most
-// of a tile's 64 are idle. us, measured on MI355X over 1 to 16 channels and K from 9 to 576: a tile costs 2.8 ns and 1.8 per
-// step; 64 outputs of the direct kernel 0.3 ns and 0.05 (16-bit 0.042) per k, and its sum in order 0.12 us per k once.
+// of a tile's 64 are idle, and in planes lower than the filter the tiles multiply the rows of padding that it skips. us,
+// measured on MI355X over 1 to 512 channels, 1 to 2^22 pixels and K from 1 to 2000: a tile costs 2.8 ns and 1.8 per step, and
+// 0.9 us per step where it waits for each; 64 outputs of the direct kernel 0.3 ns and 0.05 (16-bit 0.042) per k, its sum in
+// order 0.12 us per k and 0.03 per skipped row, whichever is longer and a part of the other.
 // 3x3 of one channel to one, [16,1,512,512] f32 54 us against 306, to four 185 / 309, to eight 374 / 309; three to one,
-// [16,3,224,224] bf16 20 / 59; 16 to one, [16,16,128,128] f32 35 / 51; 64 to one 1x1, [16,64,64,64] f32 18 / 9; one 8x8 plane 3.7 / 5.1.
-bool direct_first(int64_t k, int64_t pixels, int64_t cout, bool f32) {
-  const double rows = static_cast<double>((pixels + 63) / 64), dk = static_cast<double>(k);
-  const double steps = std::ceil(dk / (f32 ? 32 : 64));
-  const double direct = 3.1 + 0.12 * dk + 1e-3 * rows * static_cast<double>(cout) * (0.3 + (f32 ? 0.05 : 0.042) * dk);
-  const double tiles = 4.4 + 1e-3 * rows * static_cast<double>((cout + 63) / 64) * (2.8 + 1.8 * steps);
+// [16,3,224,224] bf16 20 / 59; 16 to one, [16,16,128,128] f32 35 / 51; 64 to one 1x1, [16,64,64,64] f32 18 / 9; one 8x8 plane
+// 3.7 / 5.1; 7x7 stride 2, [9,3,1,14] to 512 f32 7.6 / 11.8, [4,24,1,100] to 64 31 / 43.
+bool direct_first(const ConvGeom& c, int64_t pixels, bool f32) {
+  const double rows = static_cast<double>((pixels + 63) / 64), cin = static_cast<double>(c.cin);
+  const double inside = static_cast<double>(std::min(c.kh, c.h)), k = cin * inside * static_cast<double>(c.kw);
+  const double steps = std::ceil(cin * static_cast<double>(c.kh * c.kw) / (f32 ? 32 : 64));
+  const double sum = 0.12 * k + 0.03 * cin * (static_cast<double>(c.kh) - inside);
+  const double all = 1e-3 * rows * static_cast<double>(c.cout) * (0.3 + (f32 ? 0.05 : 0.042) * k);
+  const double direct = 3.1 + std::max(sum, all) + 0.3 * std::min(sum, all);
+  const double tiles = 4.4 + std::max(0.9 * steps, 1e-3 * rows * static_cast<double>((c.cout + 63) / 64) * (2.8 + 1.8 * steps));
   return direct < tiles;
 }
 
@@ -410,7 +416,7 @@ bool conv_any_try_launch(int32_t dtype, const void* x, const void* w, const void
       c.sw > 32767 || (c.oh * c.sh + c.ph + c.kh) * (c.w + c.pw + c.kw) > kMax)
     return false;
   const int64_t tiles = ((c.cout + 63) / 64) * ((pixels + 63) / 64);
-  if (tiles > (int64_t{1} << 30) || direct_first(k, pixels, c.cout, dtype == FH_F32)) return false;
+  if (tiles > (int64_t{1} << 30) || direct_first(c, pixels, dtype == FH_F32)) return false;
   auto magic = [](int64_t d) { return d == 1 ? 0u : static_cast<uint32_t>(((int64_t{1} << 32) + d - 1) / d); };
   auto i32 = [](int64_t v) { return static_cast<int32_t>(v); };
   ConvAnyArgs g{x,        w,        bias,     y,        i32(c.cin), i32(c.h),  i32(c.w),  i32(c.cout), i32(c.kh),

@@ -939,9 +939,11 @@ def test_conv2d_any_geometry(hip, dtype, geom):
 
 @pytest.mark.parametrize("dtype", [F32, BF16, F16])
 @pytest.mark.parametrize("geom", [(4, 1, 200, 200, 1, 3, 3, 1, 1, 1, 1, 1), (2, 3, 301, 299, 2, 3, 3, 1, 1, 1, 1, 1),
-                                  (8, 1, 260, 250, 4, 3, 3, 2, 2, 1, 1, 1), (16, 2, 128, 128, 3, 1, 1, 1, 1, 0, 0, 1)])
+                                  (8, 1, 260, 250, 4, 3, 3, 2, 2, 1, 1, 1), (16, 2, 128, 128, 3, 1, 1, 1, 1, 0, 0, 1),
+                                  (51, 16, 93, 52, 1, 3, 3, 1, 1, 0, 0, 1), (9, 3, 1, 14, 512, 7, 7, 2, 2, 3, 3, 1),
+                                  (2, 1, 1, 14, 512, 3, 3, 1, 1, 1, 1, 1)])
 def test_conv2d_few_output_channels_bit_exact(hip, dtype, geom):
-    # few output channels of many pixels: one thread per output, in the reference's order
+    # few output channels of many pixels, planes lower than the filter: one thread per output, in the reference's order
     say(f"conv of few output channels dtype={dtype} {geom}")
     x = synth.tensor(117, geom[:4], dtype, "normal")
     wt = synth.tensor(118, (geom[4], geom[1], geom[5], geom[6]), dtype, "normal")

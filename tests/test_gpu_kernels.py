@@ -904,6 +904,9 @@ CONV_ANY_CASES = [
     (9, 5, 47, 43, 70, 3, 3, 1, 1, 1, 1, 1),
     (8, 5, 48, 48, 70, 3, 3, 1, 1, 1, 1, 1),
     (16, 6, 65, 65, 40, 3, 3, 2, 2, 1, 1, 1),
+    # vectors over one image's end, and over several
+    (30, 24, 2, 13, 70, 1, 1, 1, 1, 0, 0, 1),
+    (9, 40, 1, 3, 70, 1, 1, 1, 1, 0, 0, 1),
 ]
 
 

@@ -236,12 +236,14 @@ fh_status dispatch_gemm(GemmArgs args, int64_t batch, hipStream_t stream) {
   // A transposed operand in any order: the sequential kernel takes 3 us + 35 ns per k in 16 bits, the MFMA kernels 3.5 us +
   // 10 ns per k on few tiles (64x512x1000 bf16, B transposed: 40 us against 14). In fp32 it takes 17 ns per k, 8 in four
   // ways, while the planes' tiles take 23 with A transposed and 14 with B (256x1000x10 18.3 / 10.7 / 27.1 us, 17x3000x1000
-  // 53 / 28 / 70). With more than two workgroups per CU the tiles are ahead (500x1000x400 32 us in four ways, 27 on tiles),
-  // but for A transposed and k below 256, where two ways are (500x200x400 8.4 in order, 8.8, 9.5). The sums in ways are closer
-  // to the exact ones than those in order: 500x128x400 1.5e-7 (2.1e-7), 256x3000x10 5.0e-7 (9.5e-7).
+  // 53 / 28 / 70). With more than two workgroups per CU the tiles are ahead for B transposed, with more than three for A and k
+  // from 256 on (500x1000x400 32 us in four ways, 27 on tiles); till then two ways are (500x200x400 8.4 in order, 8.8, 9.5;
+  // 40x384x3974 12.0, 11.5, 13.2). The sums in ways are closer to the exact ones than those in order: 500x128x400 1.5e-7
+  // (2.1e-7), 256x3000x10 5.0e-7 (9.5e-7).
   const bool long_k = args.any_order && (args.trans_a || args.trans_b) && args.K >= 128;
   const double outputs16 = static_cast<double>((args.M + 15) / 16) * static_cast<double>((args.N + 15) / 16) * batch;
-  const bool planes = long_k && (!std::is_same_v<T, float> || (outputs16 > 2 * cus && (args.trans_b || args.K >= 256)));
+  const bool full = args.trans_b ? outputs16 > 2 * cus : outputs16 > 3 * cus && args.K >= 256;
+  const bool planes = long_k && (!std::is_same_v<T, float> || full);
   // 16-bit operands that are not whole vectors and little work: the sequential kernel takes 3 us + 20 ns per k + (0.3 us + 5
   // ns per k) for every 65,536 outputs, an MFMA tile of any alignment 4.3-5 us at the least (bf16 2001x20x101 3.7 us against
   // 5.1, 4001x33x47 4.3 / 5.4, 600x33x333 4.2 / 4.7; past the line 1501x64x131 4.9 / 4.4, 511x63x513 7.2 / 5.0, 300x264x200

@@ -1,9 +1,10 @@
 // Conv2d forward, NCHW (reference semantics: src/backends/cpu/kernels/conv.cpp:223-314).
 //
 // conv2d_direct_kernel: one thread per output element, products summed over (ci, kh, kw) in the reference's
-// order, bias added last inside the fp32 accumulator, one rounding. It serves grouped convolutions, few output
-// channels of many pixels and sizes past the MFMA kernel's 32-bit offsets; every other geometry runs on the implicit GEMM over NCHW operands (fh_conv_any.hip). The
-// kernels over channels-last operands are fh_conv2d_nhwc_fwd's (fh_conv_igemm.hip), selected at graph compile time.
+// order, bias added last inside the fp32 accumulator, one rounding. It serves grouped convolutions, few output channels of
+// many pixels, planes lower than the filter and sizes past the MFMA kernel's 32-bit offsets; every other geometry runs on
+// the implicit GEMM over NCHW operands (fh_conv_any.hip, whose direct_first draws the line). The kernels over channels-last
+// operands are fh_conv2d_nhwc_fwd's (fh_conv_igemm.hip), selected at graph compile time.
 #include <hip/hip_runtime.h>
 
 #include <string>

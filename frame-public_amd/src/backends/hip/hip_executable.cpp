@@ -684,7 +684,7 @@ Result<ir::Graph> lower_convs(const ir::Graph& src) {
   // Whether a lowered conv reads its NCHW activation (FH_CONV_IN_NCHW) and, writing NCHW, takes its filter in the
   // graph's own [Cout][Cin][KH][KW] layout too (FH_CONV_W_OIHW, the band kernel): then neither operand is copied.
   // fp32 convs of forward graphs read both operands as they are too and write NCHW, on fh_conv2d_fwd's implicit GEMM over
-  // split operands ([32,64,56,56] x [64,64,3,3]: 67 us, against 102 channels-last with its two transposes).
+  // split operands ([32,64,56,56] x [64,64,3,3]: 71 us, against 102 channels-last with its two transposes).
   const bool forward = is_forward(src);
   auto f32_nchw = [&](const ir::Node* n, const ConvLowering& p) {
     return p.ok && forward && conv_dtype_code(n->inputs()[0]->type()) == FH_F32 && f32_conv_nchw(p.geom) &&

@@ -1123,6 +1123,7 @@ std::optional<AttentionGradMatch> match_attention_grad(
     int which;
     int64_t row, col;  // offset from the block's own place
   };
+  if (m.batch * m.heads > 65535) return std::nullopt;  // (the heads of fh_attention_grad's GEMMs are one grid dimension)
   const DType dtype = m.q->type().dtype;
   std::unordered_map<const ir::Node*, std::optional<float>> splats;
   auto splat = [&](const ir::Value* v) {

@@ -1,8 +1,8 @@
 """Benchmark of the `hip` backend's compiled-graph hot path on one MI355X.
 
-Workload (the dense GEMM sweep, at its largest size): C = A·B, row-major
+Workload (the dense GEMM sweep at its largest size): C = A·B, row-major
 A[4096,4096]·B[4096,4096], bfloat16 inputs, fp32 accumulation, bfloat16 output; entries U(-1,1) from the
-build's seeded generator. One step = one forward pass of that graph on inputs already resident in HBM.
+package's seeded generator. One step = one forward pass of that graph on inputs already resident in HBM.
 
 Prints ONE JSON line with the metric (TFLOP/s), the dominant kernel's roofline fraction (its average duration
 measured with HIP events on the stream it runs on) and a CPU baseline: the reference's own CPU backend
@@ -124,7 +124,7 @@ def copy_calibration(mib: int, reps: int):
     print(json.dumps({"copy_calibration_bytes": nbytes, "launches": reps}), flush=True)
 
 
-# ---- secondary measurements of the same metric (BASELINE.json: GEMM/Conv2d TFLOP/s, fused-op GB/s, graph latency) --
+# ---- secondary measurements of the same metric (GEMM/Conv2d TFLOP/s, fused-op GB/s, graph latency) --
 
 def _time_graph(graph_text, input_sets, steps, warmup, settle_ms=GRAPH_SETTLE_MS):
     """ms per Executable::run of the compiled graph, rotating over input_sets (lists of numpy arrays), HIP events
@@ -498,7 +498,7 @@ def main():
         "vs_baseline": None,
         "dtype": "bf16",
         "data": "synthetic" if args.gemm_data == "uniform" else f"synthetic, diagnostic all-{args.gemm_data} operands",
-        "config": {"workload": "dense GEMM C=A·B, M=N=K=4096, bf16 in/out, fp32 accumulate (configs[1])",
+        "config": {"workload": "dense GEMM C=A·B, M=N=K=4096, bf16 in/out, fp32 accumulate",
                    "M": N, "N": N, "K": N},
         "roofline": {"bound": "mfma", "achieved": round(tflops, 2), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(tflops / PEAK_BF16_TFLOPS, 4), "traffic": measured_traffic()},

@@ -4,7 +4,7 @@ Graph shapes follow the reference's own factories so that the compiled graphs ar
 Linear = matmul(x, W) then add(., bias[batch, out]) (reference: src/nn/layers.cpp:238-270); multi-head
 attention is unrolled per (batch, head) into slice/transpose/matmul/mul(constant 1/sqrt(dh))/softmax/matmul
 and concatenated per batch then across batches (reference: src/nn/layers.cpp:1014-1080). The transformer block
-is pre-LN with GELU as BASELINE.json specifies (the reference's own block is post-LN + ReLU,
+is pre-LN with GELU (the reference's own block is post-LN + ReLU,
 src/nn/layers.cpp:1099-1172); residual adds are written add(sublayer_out, residual) so the fusion pass chains
 them. ResNet-18 uses conv2d with bias for folded batch norm.
 """

@@ -1,4 +1,4 @@
-"""Compiled-graph parity on the MI355X: every configuration of BASELINE.json goes through
+"""Compiled-graph parity on the MI355X: every benchmark configuration goes through
 runtime::compile(graph, "hip") -> HipBackend::compile -> HipExecutable::run (the product path, C ABI kernels
 underneath) and is compared with the same graph compiled for the oracle's `cpu` backend on identical seeded
 inputs. Tolerances (stated per test) follow the north star: rtol 1e-5 for float32, 1e-2 for bfloat16, with
